@@ -352,6 +352,11 @@ struct Plan {
     size_t off_work = 0;     // PWork[n_work] in the upload region
     int n_work = 0;
     size_t lds_persist = 0;  // dynamic LDS of the persistent kernel (largest volume)
+    // resident path
+    size_t off_team = 0;     // team words of every volume and the ticket (zeroed with the states)
+    size_t off_slots = 0;    // int32 per workgroup slot
+    int n_slots = 0;
+    size_t lds_resident = 0;
     unsigned char* base = nullptr;  // device arena the plan lives in
 };
 
@@ -382,6 +387,8 @@ static const int kStepTileVox = 8192;
 // first kTraceCap of a call are not recorded).
 static const int kTraceCap = 4096;
 static const int kReconTileVox = 8192;
+// Resident path: 16-row units of foreground per workgroup of a full team.
+static const int kResUnitsPerChunk = 4;
 // Default iteration steps per captured graph, and the largest chunk.
 static const int kGraphSteps = 8;
 static const int kMaxGraphSteps = 64;
@@ -394,6 +401,7 @@ struct Schedule {
     bool mfma_eval;   // MFMA field-increment kernel (MFMA precisions)
     int path;         // N4_PATH_*
     int team_per_cu;  // persistent path: workgroups per compute unit (0 = occupancy limit)
+    bool resident;    // path AUTO with no setting of the step path: the resident kernel where it covers the call
 };
 
 static int env_int(const char* name, int dflt) {
@@ -432,9 +440,14 @@ static Schedule resolve_schedule(const n4_handle* h, int nvol) {
                                             : (uint32_t)env_int("N4_EVAL_KERNEL", (int)N4_EVAL_FP32);
     s.mfma_eval = ek == N4_EVAL_MFMA;
     s.path = h->tune.path ? (int)h->tune.path : env_int("N4_PATH", (int)N4_PATH_AUTO);
-    // the step kernels measured faster than the team kernel on every
-    // workload tried (per-tile memory latency is exposed when a workgroup
-    // walks its tiles one after another), so AUTO runs the steps
+    // AUTO: the resident kernel (plan_resident), unless the caller chose a
+    // schedule of the step path (groups, tiles, graphs, evaluation kernel);
+    // team_wgs_per_cu, a field of the persistent paths, overrides that.
+    // The team kernel measured slower than the steps on every workload.
+    const bool steps_asked = h->tune.groups || h->tune.step_tile_voxels || h->tune.graph_steps || h->tune.eval_kernel ||
+                             getenv("N4_GROUPS") || getenv("N4_STEP_TILE_VOX") || getenv("N4_GRAPH_STEPS") ||
+                             getenv("N4_EVAL_KERNEL");
+    s.resident = s.path == (int)N4_PATH_AUTO && (!steps_asked || h->tune.team_wgs_per_cu != 0);
     if (s.path == (int)N4_PATH_AUTO) s.path = (int)N4_PATH_STEPS;
     s.team_per_cu = h->tune.team_wgs_per_cu ? (int)h->tune.team_wgs_per_cu : env_int("N4_TEAM_WGS_PER_CU", 0);
     return s;
@@ -512,6 +525,13 @@ static n4_status stage_upload(n4_handle* h, void* dst, size_t off, size_t n, voi
     return N4_OK;
 }
 
+// Resident path: chunks (workgroups of a full team) and LDS batch size per
+// volume.
+struct ResPlan {
+    std::vector<int> nchunk, nbatch;
+    int cus = 0;
+};
+
 // Builds the plan and fills h->stage with the upload region.  Pointers in
 // the descriptors are arena-relative until `rebase` adds the arena base.
 // tiled: cut working slabs into row tiles for the step kernels (the
@@ -524,9 +544,12 @@ static n4_status stage_upload(n4_handle* h, void* dst, size_t off, size_t n, voi
 // noalloc: the plan lives in the device's file-scope scratch array (no
 // allocation; N4_ERR_NO_MEMORY beyond its size) and carries no progress
 // words (pinned host memory).
+// res (nullable, resident path): the plan holds the packed foreground in
+// place of logU, the unit lists and the slot list; no step tiles.
 static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4_params* p, Plan* P,
                             bool need_tables_full = true, bool tiled = false, int tile_vox = kStepTileVox,
-                            const std::vector<int>* teams = nullptr, bool noalloc = false) {
+                            const std::vector<int>* teams = nullptr, bool noalloc = false,
+                            const ResPlan* res = nullptr) {
     const int nv = (int)in.size();
     const int L = (int)p->number_of_fitting_levels;
     h->last.valid = false;  // the plan reuses the memory of the last run's records
@@ -563,6 +586,7 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
         nps += I.W[0] * I.prep_tiles_x;
         nfs += in[v].F[0] * I.recon_tiles_x;
     }
+    if (res) nws = 0;  // no step tiles
     P->n_wslab = nws;
     P->n_pslab = nps;
     P->recon_tiles.assign(nv, 0);
@@ -575,6 +599,11 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
     P->off_fslab = lay.take(sizeof(Slab) * (P->n_fslab > 0 ? P->n_fslab : 1));
     P->off_pslab = lay.take(sizeof(Slab) * (nps > 0 ? nps : 1));
     P->off_state = lay.take(sizeof(VolState) * nv);
+    P->off_team = lay.take(res ? 64 * (size_t)(nv + 1) : 0);
+    P->n_slots = 0;
+    if (res)
+        for (int v = 0; v < nv; ++v) P->n_slots += res->nchunk[v];
+    P->off_slots = lay.take(sizeof(int32_t) * P->n_slots);
     P->off_tw = lay.take(sizeof(D2) * P->rp.P);
     P->n_work = 0;
     if (teams)
@@ -622,12 +651,16 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
     // per-volume working buffers
     struct Offs {
         size_t imlog, logU, wmask, wconf, lat0, lat1, den, latf, lresf, part, numfx, hist, spart, etab, ppart, team,
-            trace, lvlat;
+            trace, lvlat, xq, mq, cq, slab, uent, ulist, cpart;
     };
     // histogram copies: per tile (step kernels) or per team member (teams)
     auto hcopies = [&](int v) {
+        if (res) return std::min(kHistCopies, res->nchunk[v]);
         if (teams) return std::max(1, std::min(kHistCopies, ((*teams)[v] + 7) / 8));
         return hist_copies(vi[v].W[0] * vi[v].wtiles_x, tiled);
+    };
+    auto ncopies = [&](int v) {
+        return res ? std::min(kResNumCopies, res->nchunk[v]) : num_copies(vi[v].W[0] * vi[v].wtiles_x, tiled);
     };
     int trace_cap = 0;
     for (int l = 0; l < L; ++l) trace_cap += (int)std::min<uint32_t>(p->max_iterations[l], (uint32_t)kTraceCap);
@@ -641,7 +674,7 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
         const size_t nw = (size_t)I.W[0] * I.W[1] * I.W[2];
         Offs& o = off[v];
         o.imlog = lay.take(sizeof(float) * nw);
-        o.logU = lay.take(sizeof(float) * (nw + kQuadPad));
+        o.logU = res ? 0 : lay.take(sizeof(float) * (nw + kQuadPad));
         o.wmask = lay.take(nw + kQuadPad);
         o.wconf = weighted(v) ? lay.take(sizeof(float) * nw) : 0;
         o.lat0 = lay.take(sizeof(double) * I.Lmax);
@@ -649,13 +682,25 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
         o.den = lay.take(sizeof(double) * I.Lmax);
         o.latf = lay.take(sizeof(float) * I.Lmax);
         o.lresf = lay.take(sizeof(float) * I.Lmax);
-        o.part = lay.take(sizeof(float) * I.W[0] * I.part_stride);
-        o.numfx = lay.take(sizeof(uint64_t) * I.Lmax * num_copies(I.W[0] * I.wtiles_x, tiled));
+        o.part = res ? 0 : lay.take(sizeof(float) * I.W[0] * I.part_stride);
+        o.numfx = lay.take(sizeof(uint64_t) * I.Lmax * ncopies(v));
         o.hist = lay.take(sizeof(uint64_t) * nb * hcopies(v));
-        o.spart = lay.take(sizeof(double) * 4 * I.W[0] * I.wtiles_x);
+        o.spart = res ? 0 : lay.take(sizeof(double) * 4 * I.W[0] * I.wtiles_x);
         o.ppart = lay.take(sizeof(double) * 4 * I.W[0] * I.prep_tiles_x);
         o.etab = lay.take(sizeof(double) * nb);
-        o.team = teams ? lay.take(64 + sizeof(uint64_t) * kPhases) : 0;
+        o.team = teams || res ? lay.take(64 + sizeof(uint64_t) * kPhases) : 0;
+        if (res) {
+            // a slab has at most umax units, each of at most ceil(Z / 16) tiles
+            const size_t umax = (size_t)(I.W[1] + 15) / 16, units = I.W[0] * umax;
+            const size_t tiles = units * ((size_t)(I.W[2] + 15) / 16);
+            o.xq = lay.take(sizeof(float) * 256 * tiles);
+            o.mq = lay.take(64 * tiles);
+            o.cq = weighted(v) ? lay.take(sizeof(float) * 256 * tiles) : 0;
+            o.slab = lay.take(sizeof(uint64_t) * I.W[0]);
+            o.uent = lay.take(sizeof(uint64_t) * units);
+            o.ulist = lay.take(sizeof(ResUnit) * units);
+            o.cpart = lay.take(sizeof(double) * 4 * res->nchunk[v]);
+        }
         // run records of a correction (tiled plans): CV trace, level lattices
         o.trace = tiled ? lay.take(sizeof(double) * trace_cap) : 0;
         size_t lsum = 0;
@@ -700,6 +745,7 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
     // the volume states start at zero (the rest of the image is written
     // below wherever a kernel reads it)
     memset(hb + P->off_state, 0, sizeof(VolState) * nv);
+    if (res) memset(hb + P->off_team, 0, 64 * (size_t)(nv + 1));
     // the distinct axis tables, on up to 8 host threads when there are many
     // (each thread takes the next table; the calling thread works too, so
     // every table is computed even if no other thread could be started)
@@ -751,7 +797,7 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
         D.nvox_w = (int64_t)I.W[0] * I.W[1] * I.W[2];
         const Offs& o = off[v];
         D.imlog = (float*)(base + o.imlog);
-        D.logU = (float*)(base + o.logU);
+        D.logU = res ? nullptr : (float*)(base + o.logU);
         D.wmask = (uint8_t*)(base + o.wmask);
         D.wconf = weighted(v) ? (float*)(base + o.wconf) : nullptr;
         D.lat[0] = (double*)(base + o.lat0);
@@ -759,12 +805,25 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
         D.den = (double*)(base + o.den);
         D.latf = (float*)(base + o.latf);
         D.lresf = (float*)(base + o.lresf);
-        D.part = (float*)(base + o.part);
+        D.part = res ? nullptr : (float*)(base + o.part);
         D.numfx = (uint64_t*)(base + o.numfx);
-        D.num_copies = num_copies(I.W[0] * I.wtiles_x, tiled);
+        D.num_copies = ncopies(v);
         D.lmax = (int32_t)I.Lmax;
         D.hist = (uint64_t*)(base + o.hist);
-        D.spart = (double*)(base + o.spart);
+        D.spart = res ? nullptr : (double*)(base + o.spart);
+        if (res) {
+            D.res.nchunk = res->nchunk[v];
+            D.res.umax = (I.W[1] + 15) / 16;
+            D.res.nbatch = res->nbatch[v];
+            D.res.xq = (float*)(base + o.xq);
+            D.res.mq = (uint8_t*)(base + o.mq);
+            D.res.cq = weighted(v) ? (float*)(base + o.cq) : nullptr;
+            D.res.slab = (uint64_t*)(base + o.slab);
+            D.res.uent = (uint64_t*)(base + o.uent);
+            D.res.ulist = (ResUnit*)(base + o.ulist);
+            D.res.cpart = (double*)(base + o.cpart);
+            D.res.team = (uint32_t*)(base + P->off_team + 64 * (size_t)v);
+        }
         D.ppart = (double*)(base + o.ppart);
         D.prep_rows = I.prep_rows;
         D.prep_tiles_x = I.prep_tiles_x;
@@ -773,7 +832,7 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
         D.wtiles_x = I.wtiles_x;
         D.hist_copies = hcopies(v);
         D.team_ctr = teams ? (uint32_t*)(base + o.team) : nullptr;
-        D.tphase = (teams && (h->prof_mask >> N4_K_TEAMS & 1u)) ? (uint64_t*)(base + o.team + 64) : nullptr;
+        D.tphase = ((teams || res) && (h->prof_mask >> N4_K_TEAMS & 1u)) ? (uint64_t*)(base + o.team + 64) : nullptr;
         D.mW2 = magic_div((uint32_t)I.W[2]);
         D.mF2 = magic_div((uint32_t)in[v].F[2]);
         D.etab = (double*)(base + o.etab);
@@ -807,7 +866,7 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
             P->lds_persist = std::max(P->lds_persist, lds_persist(D, nb, P->rp.P, P->rp.prec));
         }
         for (int x = 0; x < I.W[0]; ++x) {
-            for (int y0 = 0; y0 < I.W[1]; y0 += I.wtile_rows)
+            for (int y0 = 0; y0 < I.W[1] && !res; y0 += I.wtile_rows)
                 ws[iws++] = Slab{v, x, y0, std::min(I.wtile_rows, I.W[1] - y0)};
             for (int y0 = 0; y0 < I.W[1]; y0 += I.prep_rows)
                 ps[ips++] = Slab{v, x, y0, std::min(I.prep_rows, I.W[1] - y0)};
@@ -817,6 +876,7 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
                 for (int y0 = 0; y0 < in[v].F[1]; y0 += I.recon_rows)
                     fs[ifs++] = Slab{v, x, y0, std::min(I.recon_rows, in[v].F[1] - y0)};
         const int prec = P->rp.prec;
+        if (res) P->lds_resident = std::max(P->lds_resident, lds_resident(D, nb, P->rp.P, prec));
         for (int l = 0; l < L; ++l) {
             P->lds_fit_max[l] = std::max(P->lds_fit_max[l], lds_fit(nb, D, l, prec));
             P->lds_eval_max[l] = std::max(P->lds_eval_max[l], lds_eval(D, l, prec));
@@ -826,6 +886,15 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
             P->nt[l] = mfma_tiles(D.lev[l].C[2]);
         }
         if (need_tables_full) P->lds_recon = std::max(P->lds_recon, lds_recon(D));
+    }
+    if (res) {
+        // the largest volumes first, each with all its slots in a row
+        std::vector<std::pair<double, int>> by(nv);
+        for (int v = 0; v < nv; ++v) by[v] = {-(double)P->desc[v].nvox_w, v};
+        std::sort(by.begin(), by.end());
+        int32_t* sl = (int32_t*)(hb + P->off_slots);
+        for (const auto& b : by)
+            for (int k = 0; k < res->nchunk[b.second]; ++k) *sl++ = b.second;
     }
     P->lds_hist = lds_hist(nb);
     P->lds_wiener = lds_wiener(P->rp.P);
@@ -1169,6 +1238,64 @@ static bool plan_teams(const std::vector<VolIn>& in, const n4_params* p, const S
     return true;
 }
 
+// Resident path: chunks per volume, or false where a volume is not covered:
+// the matrix operands hold 16 control points along y and z, a volume's
+// factor tables, lattice increment and one batch of units share a compute
+// unit's LDS, and the unit entries hold 16-bit positions.
+// Chunks: a workgroup per kResUnitsPerChunk units (below that a workgroup's
+// share of the per-iteration chain outweighs its work), scaled down in
+// proportion to the volumes' sizes when the batch asks for more workgroups
+// than the device has compute units.
+// The resident kernel runs wherever it covers the call.  Measured against the
+// step kernels (five launches a step), whole calls: 64^3 FP32 2.30 -> 1.62
+// ms, 256x256x176 at shrink 4 FP32 2.63 -> 2.03, 512x512x320 at shrink 2 BF16
+// 4.91 -> 3.65, 12 mixed volumes split BF16 5.40 -> 3.52, 64 volumes at
+// shrink 4 BF16 7.70 -> 7.62.
+#ifndef N4_EMULATE
+static bool plan_resident(const std::vector<VolIn>& in, const n4_params* p, const Schedule& sch, ResPlan* R) {
+    const int nv = (int)in.size(), L = (int)p->number_of_fitting_levels;
+    const RunParams rp = make_run_params(p);
+    size_t lds_cap = 0;
+    if (resident_limits(&R->cus, &lds_cap) != 0 || R->cus < 1) return false;
+    R->nchunk.assign(nv, 1);
+    R->nbatch.assign(nv, 64);
+    const int per = std::max(1, env_int("N4_RES_UNITS", kResUnitsPerChunk));
+    std::vector<double> want(nv);
+    std::vector<int> strips(nv);
+    double sum = 0.0;
+    for (int v = 0; v < nv; ++v) {
+        VolDesc D;
+        memset(&D, 0, sizeof D);
+        for (int d = 0; d < 3; ++d) D.W[d] = (in[v].F[d] + in[v].s - 1) / in[v].s;
+        if (D.W[0] > kResMaxSlabs || D.W[1] > kResMaxDim || D.W[2] > kResMaxDim) return false;
+        D.nlevels = L;
+        LevelDesc& F = D.lev[L - 1];
+        for (int d = 0; d < 3; ++d) F.C[d] = level_ncpt((int)p->ncpt[d], L - 1);
+        F.L = F.C[0] * F.C[1] * F.C[2];
+        if (F.C[1] > 16 || F.C[2] > 16) return false;
+        D.res.nchunk = R->cus;
+        D.res.nbatch = 64;
+        int rows, strips_x;
+        step_tiles(D.W, true, sch.tile_vox, &rows, &strips_x);
+        const int least = (rows + 15) / 16;  // a batch holds whole strips
+        if (least > 64) return false;
+        while (D.res.nbatch / 2 >= least && lds_resident(D, rp.nbins, rp.P, rp.prec) > lds_cap) D.res.nbatch /= 2;
+        if (lds_resident(D, rp.nbins, rp.P, rp.prec) > lds_cap) return false;
+        R->nbatch[v] = D.res.nbatch;
+        strips[v] = D.W[0] * strips_x;
+        // about three quarters of a head volume's 16-row units hold foreground
+        want[v] = 0.75 * D.W[0] * ((D.W[1] + 15) / 16) / per;
+        sum += std::max(want[v], 1.0);
+    }
+    for (int v = 0; v < nv; ++v) {
+        const double n = sum > R->cus ? want[v] * R->cus / sum : want[v];
+        // (at most 1024 chunks: their partials are reduced by one workgroup)
+        R->nchunk[v] = std::max(1, std::min(std::min(std::min(R->cus, 1024), strips[v]), (int)floor(n + 0.5)));
+    }
+    return true;
+}
+#endif
+
 #define GLAUNCH(id, expr)                  \
     do {                                   \
         ProfScope ps_(h, (id), gs);        \
@@ -1180,7 +1307,7 @@ static bool plan_teams(const std::vector<VolIn>& in, const n4_params* p, const S
 // layout or the descriptors.
 static std::vector<unsigned char> correction_plan_key(const n4_handle* h, const std::vector<VolIn>& in,
                                                       const n4_params* p, int tile_vox,
-                                                      const std::vector<int>* teams) {
+                                                      const std::vector<int>* teams, const ResPlan* res) {
     std::vector<unsigned char> k;
     auto add = [&](const auto& x) {
         const unsigned char* b = reinterpret_cast<const unsigned char*>(&x);
@@ -1208,6 +1335,12 @@ static std::vector<unsigned char> correction_plan_key(const n4_handle* h, const 
     add(teams ? teams->size() : (size_t)0);
     if (teams)
         for (int t : *teams) add(t);
+    add(res != nullptr);
+    if (res)
+        for (size_t v = 0; v < res->nchunk.size(); ++v) {
+            add(res->nchunk[v]);
+            add(res->nbatch[v]);
+        }
     add(h->dev_flags);
     add(h->flag_cap);
     add(h->prof_mask);
@@ -1240,7 +1373,15 @@ static n4_status run_batch(n4_handle* h, const std::vector<VolIn>& in_user, cons
         if (!teams_path && sch.path == (int)N4_PATH_TEAMS)
             return fail(N4_ERR_UNSUPPORTED, "persistent team path not available for this batch: %s", why.c_str());
     }
-    const int G = (teams_path || noalloc) ? 1 : sch.groups;
+    ResPlan res_user;
+    bool resident = false;
+#ifndef N4_EMULATE
+    if (sch.resident) {
+        N4_CHECK_HIP(hipSetDevice(h->device));
+        resident = plan_resident(in_user, p, sch, &res_user);
+    }
+#endif
+    const int G = (teams_path || noalloc || resident) ? 1 : sch.groups;
     // kernel timing creates events: off for the allocation-free path
     struct ProfMaskGuard {
         n4_handle* h;
@@ -1275,9 +1416,15 @@ static n4_status run_batch(n4_handle* h, const std::vector<VolIn>& in_user, cons
     }
     std::vector<VolIn> in(nv);
     std::vector<int> teams(teams_path ? nv : 0);
+    ResPlan res;
+    res.cus = res_user.cus;
     for (int k = 0; k < nv; ++k) {
         in[k] = in_user[order[k]];
         if (teams_path) teams[k] = teams_user[order[k]];
+        if (resident) {
+            res.nchunk.push_back(res_user.nchunk[order[k]]);
+            res.nbatch.push_back(res_user.nbatch[order[k]]);
+        }
     }
 #ifndef N4_EMULATE
     N4_CHECK_HIP(hipSetDevice(h->device));
@@ -1305,7 +1452,8 @@ static n4_status run_batch(n4_handle* h, const std::vector<VolIn>& in_user, cons
 #endif
     Plan P;
     std::vector<unsigned char> pkey;
-    if (!noalloc) pkey = correction_plan_key(h, in, p, sch.tile_vox, teams_path ? &teams : nullptr);
+    if (!noalloc)
+        pkey = correction_plan_key(h, in, p, sch.tile_vox, teams_path ? &teams : nullptr, resident ? &res : nullptr);
     const bool plan_reused = !noalloc && h->plan_cached && pkey == h->plan_key;
     if (plan_reused) {
         // the plan of the last call, whose upload image is still in the stage:
@@ -1324,21 +1472,33 @@ static n4_status run_batch(n4_handle* h, const std::vector<VolIn>& in_user, cons
         stage_wait(h);
         memcpy(h->stage + P.off_desc, P.desc.data(), sizeof(VolDesc) * nv);
     } else {
-        s = build_plan(h, in, p, &P, true, true, sch.tile_vox, teams_path ? &teams : nullptr, noalloc);
+        s = build_plan(h, in, p, &P, true, true, sch.tile_vox, teams_path ? &teams : nullptr, noalloc,
+                       resident ? &res : nullptr);
+        if (s == N4_ERR_NO_MEMORY && noalloc && resident) {
+            // (the step path needs a little less of the scratch array)
+            resident = false;
+            g_err.clear();
+            P = Plan();
+            s = build_plan(h, in, p, &P, true, true, sch.tile_vox, nullptr, true);
+        }
         if (s != N4_OK) return s;
         if (!noalloc) {
             h->plan_cached.reset(new Plan(P));
             h->plan_key = pkey;
         }
     }
-    s = check_lds(P, !teams_path, true);
+    // the volume states and, on the resident path, the team words behind them
+    const size_t state_bytes =
+        resident ? P.off_team + 64 * (size_t)(nv + 1) - P.off_state : sizeof(VolState) * (size_t)nv;
+    s = check_lds(P, !teams_path && !resident, true);
     if (s != N4_OK) return s;
     if (plan_reused) {
         // the arena still holds the rest of the upload region (slab lists,
         // twiddles, axis tables; no kernel writes them): descriptors, and the
         // volume states back to their initial (zero) image
         s = stage_upload(h, P.base + P.off_desc, P.off_desc, sizeof(VolDesc) * nv, stream);
-        if (s == N4_OK) s = stage_upload(h, P.base + P.off_state, P.off_state, sizeof(VolState) * nv, stream);
+        if (s == N4_OK)  // (and, on the resident path, the team words behind them)
+            s = stage_upload(h, P.base + P.off_state, P.off_state, state_bytes, stream);
     } else {
         s = stage_upload(h, P.base, 0, P.upload_bytes, stream);
     }
@@ -1362,7 +1522,7 @@ static n4_status run_batch(n4_handle* h, const std::vector<VolIn>& in_user, cons
             R.pc[0] = ps;
             while (v < nv && gid[order[v]] == g) {
                 while (ci < 4 && prep_class(P.desc[v].s) != kPrepClasses[ci]) R.pc[++ci] = ps;
-                ws += P.desc[v].W[0] * P.desc[v].wtiles_x;
+                ws += resident ? 0 : P.desc[v].W[0] * P.desc[v].wtiles_x;
                 fs += P.recon_tiles[v];
                 ps += P.desc[v].W[0] * P.desc[v].prep_tiles_x;
                 ++v;
@@ -1423,7 +1583,16 @@ static n4_status run_batch(n4_handle* h, const std::vector<VolIn>& in_user, cons
             if (R.pc[c + 1] > R.pc[c])
                 GLAUNCH(N4_K_PREP,
                         launch_prep(dd, dev_pslab(h, P) + R.pc[c], R.pc[c + 1] - R.pc[c], kPrepClasses[c], rp, gs));
-        GLAUNCH(N4_K_LEVEL, launch_level(dd + R.v0, R.v1 - R.v0, 0, rp, gs));
+        if (!resident) GLAUNCH(N4_K_LEVEL, launch_level(dd + R.v0, R.v1 - R.v0, 0, rp, gs));
+    }
+    if (resident) {
+        // one launch runs every volume's level/iteration loop
+        void* gs = stream;
+        GLAUNCH(N4_K_TEAMS, launch_resident(dd, (const int32_t*)(P.base + P.off_slots), P.n_slots,
+                                            std::min(P.n_slots, res.cus),
+                                            (uint32_t*)(P.base + P.off_team + 64 * (size_t)nv), rp, P.lds_resident, gs));
+        GLAUNCH(N4_K_RECON, launch_recon(dd, fsl, P.n_fslab, P.nlevels - 1, rp, P.lds_recon, gs));
+        for (GroupRun& R : gr) R.finished = true;
     }
     if (teams_path) {
         // one launch runs every volume's level/iteration loop
@@ -1508,7 +1677,7 @@ static n4_status run_batch(n4_handle* h, const std::vector<VolIn>& in_user, cons
     };
     // one host thread drives every group, round robin (a thread per group
     // measured no faster: the host's launch cost is not the bound)
-    int remaining = teams_path ? 0 : G;
+    int remaining = (teams_path || resident) ? 0 : G;
     uint64_t idle_rounds = 0;
     while (remaining > 0) {
         bool advanced = false;
@@ -1530,13 +1699,14 @@ static n4_status run_batch(n4_handle* h, const std::vector<VolIn>& in_user, cons
 #endif
         }
     }
-    std::vector<VolState> st(nv);
-    D2H(st.data(), dev_state(h, P), sizeof(VolState) * nv, stream);
+    std::vector<unsigned char> st_bytes(state_bytes);
+    const VolState* st = reinterpret_cast<const VolState*>(st_bytes.data());
+    D2H(st_bytes.data(), dev_state(h, P), state_bytes, stream);
     std::vector<uint32_t> tctr(teams_path ? 2 * nv : 0);
-    std::vector<uint64_t> tph(teams_path && P.desc[0].tphase ? (size_t)kPhases * nv : 0);
-    if (teams_path)
+    std::vector<uint64_t> tph((teams_path || resident) && P.desc[0].tphase ? (size_t)kPhases * nv : 0);
+    if (teams_path || resident)
         for (int v = 0; v < nv; ++v) {
-            D2H(&tctr[2 * v], P.desc[v].team_ctr, 2 * sizeof(uint32_t), stream);
+            if (teams_path) D2H(&tctr[2 * v], P.desc[v].team_ctr, 2 * sizeof(uint32_t), stream);
             if (!tph.empty()) D2H(&tph[(size_t)kPhases * v], P.desc[v].tphase, sizeof(uint64_t) * kPhases, stream);
         }
     float ms = 0.0f;
@@ -1564,6 +1734,9 @@ static n4_status run_batch(n4_handle* h, const std::vector<VolIn>& in_user, cons
                 h->prof_n[kPhaseId[k]] += tph[(size_t)kPhases * v + kPhSteps];
             }
     }
+    if (resident)
+        for (int v = 0; v < nv; ++v)
+            if (!st[v].done) return fail(N4_ERR_INTERNAL, "resident path: volume %d did not finish", order[v]);
     for (int v = 0; v < (int)tctr.size() / 2; ++v)
         if (tctr[2 * v + 1])
             return fail(N4_ERR_INTERNAL, "persistent path: a team barrier of volume %d timed out", order[v]);
@@ -1891,6 +2064,8 @@ n4_status n4_autotune_batch(n4_handle* h, const n4_volume* vols, uint32_t nvol, 
                 if (p->precision != N4_PREC_FP32) cand.push_back(n4_tuning{g, t, k, N4_EVAL_MFMA, N4_PATH_STEPS, 0, 0.0f});
             }
     }
+    // the resident kernel (team_wgs_per_cu asks for it), where it covers the batch
+    cand.push_back(n4_tuning{1u, 8192u, N4_GRAPH_OFF, N4_EVAL_FP32, N4_PATH_AUTO, 1u, 0.0f});
     // best wall time of `reps` timed runs after one untimed run; N4_AUTOTUNE_LOG=1
     // prints every measurement to stderr
     const bool log = env_int("N4_AUTOTUNE_LOG", 0) != 0;

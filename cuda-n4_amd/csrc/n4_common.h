@@ -75,6 +75,36 @@ struct VolState {
     double lastcv[kMaxLevels];
 };
 
+// One unit of a volume's foreground (resident path, n4_resident.h): rows
+// [y0, y0 + 16) of slab x, z from zlo in nt tiles of 16 rows x 16 z, the
+// first of them tile `tile` of the volume's packed copy.
+struct alignas(16) ResUnit {
+    int32_t x;
+    uint16_t y0, zlo;
+    int32_t tile;
+    int32_t nt;
+};
+
+constexpr int kResNumCopies = 8;   // most numerator copies of a resident plan
+constexpr int kResMaxDim = 1024;   // most working rows / z positions it covers
+constexpr int kResMaxSlabs = 2048; // most working slabs
+
+// A volume's buffers on the resident path (nchunk 0: not a resident plan).
+struct ResDesc {
+    int32_t nchunk;   // runs of strips = workgroups of a full team
+    int32_t umax;     // unit entries per slab
+    int32_t nbatch;   // units whose list and T2 slots fit the LDS at once (at most 64)
+    int32_t pad;
+    float* xq;        // packed logU: 256 floats per tile, lane-major quads
+    uint8_t* mq;      // mask bits of every quad (bits 0..3)
+    float* cq;        // packed confidence weights (weighted masks; else null)
+    uint64_t* slab;   // [W0] units | tiles << 32
+    uint64_t* uent;   // [W0][umax] y0 | zlo << 16 | tiles << 32 | first tile in the slab << 48
+    ResUnit* ulist;   // all units in slab order
+    double* cpart;    // [nchunk][4] convergence sums and range of each chunk
+    uint32_t* team;   // 16 words, zero before the launch (ResWord)
+};
+
 struct VolDesc {
     // full resolution
     const float* im;
@@ -127,6 +157,7 @@ struct VolDesc {
     uint64_t mF2;              // magic divisor for the full-resolution z extent
     uint32_t* team_ctr;        // persistent path: [0] the team's barrier counter, [1] abort flag
     uint64_t* tphase;          // persistent path (nullable): leader's device-clock ticks per phase (kPhases)
+    ResDesc res;               // resident path
 };
 
 // Phases of the persistent path timed by a team's leader (tphase slots).

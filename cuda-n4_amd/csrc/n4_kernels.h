@@ -78,6 +78,15 @@ int persist_capacity(size_t lds, int prec, int* per_cu, int* cus);
 int launch_persist(const VolDesc* vols, const Slab* slabs, const PWork* work, int nwg, RunParams rp, size_t lds,
                    void* stream);
 
+// Resident path (n4_resident.h): every volume's level/iteration loop in one
+// launch of nwg workgroups (one per compute unit); slots[k] names the volume
+// whose team the k-th workgroup to ask joins (a volume's nchunk slots are
+// consecutive), *ticket (zero) counts the slots taken.
+size_t lds_resident(const VolDesc& v, int nbins, int P, int prec);
+int resident_limits(int* cus, size_t* lds);
+int launch_resident(const VolDesc* vols, const int32_t* slots, int nslots, int nwg, uint32_t* ticket, RunParams rp,
+                    size_t lds, void* stream);
+
 // Flat (1-D) stage helpers used by the stage entry points.  A flat array of
 // n voxels is cut into slabs of kChunkVox voxels; each slab writes
 // spart[x] = 4 doubles (reduced on the host by the stage call).

@@ -34,6 +34,7 @@
 #endif
 
 #include <math.h>
+#include <string.h>
 
 #include <type_traits>
 
@@ -154,7 +155,7 @@ HD void store_quad(float* p, const F4& x) {
 template <class T>
 HD T ld_agent(const T* p) {
 #ifdef N4_DEVICE_PASS
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return __hip_atomic_load(gp(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #else
     T v;
     __atomic_load(p, &v, __ATOMIC_SEQ_CST);
@@ -164,7 +165,7 @@ HD T ld_agent(const T* p) {
 template <class T>
 HD void st_agent(T* p, T v) {
 #ifdef N4_DEVICE_PASS
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(gp(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #else
     __atomic_store(p, &v, __ATOMIC_SEQ_CST);
 #endif
@@ -465,7 +466,7 @@ HD void prep_commit(const VolDesc& V, int x, int J, int K, int nm, int nb, float
     const bool fg = nm > 0 && 2 * nm >= nb;
     const float lg = nm > 0 ? acc / (float)nm : 0.0f;
     gp(V.imlog)[w] = lg;
-    gp(V.logU)[w] = lg;
+    if (V.logU) gp(V.logU)[w] = lg;  // (a resident plan packs its own copy)
     gp(V.wmask)[w] = fg ? 1 : 0;
     if constexpr (MK == 3) gp(V.wconf)[w] = fg ? wsum / (float)nm : 0.0f;
     nfull += nm;
@@ -617,6 +618,44 @@ HD float* level_lattice_record(const VolDesc& V, int lvl) {
 // TEAM (persistent path, run by the team's leader): the lattices are read
 // and written with agent-scope accesses (the team's owners update them).
 template <bool TEAM>
+HD double refine_cp(const VolDesc& V, int level, int l) {
+    const LevelDesc& LD = V.lev[level];
+    const LevelDesc& PD = V.lev[level - 1];
+    const double* src = V.lat[(level - 1) & 1];
+    int c[3];
+    c[0] = l / (LD.C[1] * LD.C[2]);
+    c[1] = (l / LD.C[2]) % LD.C[1];
+    c[2] = l % LD.C[2];
+    int par[3], odd[3];
+    for (int d = 0; d < 3; ++d) {
+        const int ic = c[d] - 1;  // child index in [-1, 2n+1]
+        const int i = (ic >= 0) ? ic / 2 : -((-ic + 1) / 2);
+        par[d] = i;
+        odd[d] = ic - 2 * i;
+    }
+    double acc = 0.0;
+    for (int a = 0; a < 3; ++a) {
+        int X = par[0] - 1 + a;
+        const int nx = PD.C[0] - 3;
+        X = X < -1 ? -1 : (X > nx + 1 ? nx + 1 : X);
+        for (int b = 0; b < 3; ++b) {
+            int Y = par[1] - 1 + b;
+            const int ny = PD.C[1] - 3;
+            Y = Y < -1 ? -1 : (Y > ny + 1 ? ny + 1 : Y);
+            for (int e = 0; e < 3; ++e) {
+                int Z = par[2] - 1 + e;
+                const int nz = PD.C[2] - 3;
+                Z = Z < -1 ? -1 : (Z > nz + 1 ? nz + 1 : Z);
+                const double wgt = refine_w(odd[0], a) * refine_w(odd[1], b) * refine_w(odd[2], e);
+                const double* sp = src + ((size_t)(X + 1) * PD.C[1] + (Y + 1)) * PD.C[2] + (Z + 1);
+                acc += wgt * (TEAM ? ld_agent(sp) : *sp);
+            }
+        }
+    }
+    return acc;
+}
+
+template <bool TEAM>
 HD void refine_lattice(const VolDesc& V, int level, int t) {
     const LevelDesc& LD = V.lev[level];
     const LevelDesc& PD = V.lev[level - 1];
@@ -625,36 +664,7 @@ HD void refine_lattice(const VolDesc& V, int level, int t) {
     if (float* rec = level_lattice_record(V, level - 1))
         for (int l = t; l < PD.L; l += kBlock) rec[l] = (float)(TEAM ? ld_agent(src + l) : src[l]);
     for (int l = t; l < LD.L; l += kBlock) {
-        int c[3];
-        c[0] = l / (LD.C[1] * LD.C[2]);
-        c[1] = (l / LD.C[2]) % LD.C[1];
-        c[2] = l % LD.C[2];
-        int par[3], odd[3];
-        for (int d = 0; d < 3; ++d) {
-            const int ic = c[d] - 1;  // child index in [-1, 2n+1]
-            const int i = (ic >= 0) ? ic / 2 : -((-ic + 1) / 2);
-            par[d] = i;
-            odd[d] = ic - 2 * i;
-        }
-        double acc = 0.0;
-        for (int a = 0; a < 3; ++a) {
-            int X = par[0] - 1 + a;
-            const int nx = PD.C[0] - 3;
-            X = X < -1 ? -1 : (X > nx + 1 ? nx + 1 : X);
-            for (int b = 0; b < 3; ++b) {
-                int Y = par[1] - 1 + b;
-                const int ny = PD.C[1] - 3;
-                Y = Y < -1 ? -1 : (Y > ny + 1 ? ny + 1 : Y);
-                for (int e = 0; e < 3; ++e) {
-                    int Z = par[2] - 1 + e;
-                    const int nz = PD.C[2] - 3;
-                    Z = Z < -1 ? -1 : (Z > nz + 1 ? nz + 1 : Z);
-                    const double wgt = refine_w(odd[0], a) * refine_w(odd[1], b) * refine_w(odd[2], e);
-                    const double* sp = src + ((size_t)(X + 1) * PD.C[1] + (Y + 1)) * PD.C[2] + (Z + 1);
-                    acc += wgt * (TEAM ? ld_agent(sp) : *sp);
-                }
-            }
-        }
+        const double acc = refine_cp<TEAM>(V, level, l);
         if (TEAM) {
             st_agent(dst + l, acc);
         } else {
@@ -744,6 +754,64 @@ HD void hist_zero(N4_LDS unsigned long long* h, int hs) {
     BLOCK_END
 }
 
+// Slots of one LDS copy of nb bins: one past the last bin, and an odd
+// stride (the copies of one bin fall in different banks).
+HD int hist_stride(int nb) { return (nb + 1) | 1; }
+
+// The histogram's bins: origin, width and the width's reciprocal (0: the
+// quotient below falls back to the division).
+struct Bins {
+    double mn, slope, rinv;
+    int nb;
+};
+
+HD Bins make_bins(double mn, double slope, int nb) {
+    return Bins{mn, slope, slope > 1e-100 && slope < 1e100 ? 1.0 / slope : 0.0, nb};
+}
+
+// x / slope, correctly rounded: the product with the reciprocal, and two
+// corrections by the exact remainder (Markstein 1990: from a quotient within
+// one ulp and the correctly rounded reciprocal, one such step rounds
+// correctly; the first step brings the product within one ulp).  Six FP64
+// operations in place of the division's scaling, seed and fix-up.
+HD double bins_quotient(const Bins& B, double d) {
+    if (B.rinv == 0.0) return d / B.slope;
+    const double q0 = d * B.rinv;
+    const double q1 = fma(fma(-q0, B.slope, d), B.rinv, q0);
+    return fma(fma(-q1, B.slope, d), B.rinv, q1);
+}
+
+// Bin index and share of one voxel, in one rounding: c + 2^20 keeps c to a
+// multiple of 2^-32, so its low word is the share q of the next bin and the
+// 20 bits above it the bin (a share that rounds to 2^32 is a whole count of
+// the next bin, which is what rint(off 2^32) gives as well).  in: c is
+// within the bins; past the last bin's left edge nothing is counted
+// (N4.py:25-27).
+struct BinShare {
+    uint32_t idx, q;
+    bool in;
+};
+HD BinShare bin_share(const Bins& B, float x) {
+    const double c = bins_quotient(B, (double)x - B.mn);
+    const double v = c + 1048576.0;
+    uint64_t u;
+    memcpy(&u, &v, sizeof u);
+    return BinShare{(uint32_t)(u >> 32) & 0xfffffu, (uint32_t)u, c >= 0.0 && c <= (double)(B.nb - 1)};
+}
+
+// One foreground voxel into a copy hl of the bins (nb + 1 slots: a share of
+// zero may go to the slot past the last bin); returns its bin index (-1:
+// outside the bins), floor(c) as N4.py has it.
+HD int hist_voxel(float x, const Bins& B, N4_LDS unsigned long long* hl) {
+    const BinShare s = bin_share(B, x);
+    if (s.in) {
+        lds_add_u64(&hl[s.idx], (1ull << 32) - s.q);
+        lds_add_u64(&hl[s.idx + 1], s.q);
+    }
+    const double fl = floor(bins_quotient(B, (double)x - B.mn));
+    return (fl >= 0.0 && fl < (double)B.nb) ? (int)fl : -1;
+}
+
 HD void hist_tile(const VolDesc& V, const Slab sl, double mn, double slope, int nb, N4_LDS unsigned long long* h,
                   int hs, int32_t* dbg_idx) {
     const int YZ = sl.ny * V.W[2];
@@ -751,6 +819,7 @@ HD void hist_tile(const VolDesc& V, const Slab sl, double mn, double slope, int 
     const size_t vend = std::min(base + (size_t)YZ, (size_t)V.nvox_w);
     const size_t q0 = base & ~(size_t)3;
     const int nq = (int)((vend - q0 + 3) >> 2);
+    const Bins B = make_bins(mn, slope, nb);
     BLOCK_FOR(t)
     N4_LDS unsigned long long* hl = h + (size_t)(t & (kHistLanes - 1)) * hs;
     for (int i0 = 0; i0 < nq; i0 += 4 * kBlock) {
@@ -772,19 +841,8 @@ HD void hist_tile(const VolDesc& V, const Slab sl, double mn, double slope, int 
                     if (dbg_idx) dbg_idx[w] = -1;
                     continue;
                 }
-                const double c = ((double)xs[u].v[j] - mn) / slope;
-                const double fl = floor(c);
-                const int idx = (fl >= 0.0 && fl < (double)nb) ? (int)fl : -1;
+                const int idx = hist_voxel(xs[u].v[j], B, hl);
                 if (dbg_idx) dbg_idx[w] = idx;
-                if (idx < 0) continue;
-                const double off = c - fl;
-                if (off == 0.0) {
-                    lds_add_u64(&hl[idx], 1ull << 32);
-                } else if (idx < nb - 1) {
-                    const unsigned long long q = (unsigned long long)rint(off * 4294967296.0);
-                    lds_add_u64(&hl[idx], (1ull << 32) - q);
-                    lds_add_u64(&hl[idx + 1], q);
-                }
             }
         }
     }
@@ -832,7 +890,7 @@ HD void body_hist(const VolDesc* vols, const Slab* slabs, int step, RunParams rp
     N4_LDS double* red = Carve{smem, 0}.take<double>(4 * kBlock);
     // kHistLanes lane-strided copies of the bins (odd stride: the copies of
     // one bin fall in different LDS banks), merged before the global flush
-    const int hs = nb | 1;
+    const int hs = hist_stride(nb);
     N4_LDS unsigned long long* h = Carve{smem, 0}.take<unsigned long long>((size_t)kHistLanes * hs);
     const int mode = step < 0 ? kModeIter : st->mode;
     const int lvl = step < 0 ? 0 : st->lvl, it = step < 0 ? 0 : st->it;
@@ -952,13 +1010,13 @@ HD void dft_small(D2 (&v)[R], double sg) {
 // constants: with every pass unrolled and its index arithmetic folded, a
 // 512-point transform takes 1.3 us on MI355X against 2.3 us for the same
 // code with a run-time size and direction.
-template <int R, int P, bool INV>
+template <int R, int P, bool INV, int NT>
 HD void block_fft_pass(const N4_LDS D2* a, N4_LDS D2* b, const N4_LDS D2* tw, int Ns) {
     constexpr int nbf = P / R;
     const int tstep = P / (Ns * R);
     constexpr double sg = INV ? 1.0 : -1.0;
     BLOCK_FOR(t)
-    for (int j = t; j < nbf; j += kBlock) {
+    for (int j = t; j < nbf; j += NT) {
         const int k = j & (Ns - 1);
         D2 v[R];
         UNROLL for (int r = 0; r < R; ++r) v[r] = a[j + r * nbf];
@@ -982,17 +1040,17 @@ HD void block_fft_pass(const N4_LDS D2* a, N4_LDS D2* b, const N4_LDS D2* tw, in
 // free).  (Radix 2 and 4 over all 256 threads, and radix 8 in one
 // wavefront with wave-level ordering, measured equal or slower on MI355X.)
 constexpr int kFftRadix = 8;
-template <int P, bool INV>
+template <int P, bool INV, int NT>
 HD N4_LDS D2* block_fft(N4_LDS D2* a, N4_LDS D2* b, const N4_LDS D2* tw) {
     UNROLL for (int Ns = 1; Ns < P;) {
         const int rem = P / Ns;
         const int R = rem >= kFftRadix ? kFftRadix : rem;
         if (R == 8)
-            block_fft_pass<8, P, INV>(a, b, tw, Ns);
+            block_fft_pass<8, P, INV, NT>(a, b, tw, Ns);
         else if (R == 4)
-            block_fft_pass<4, P, INV>(a, b, tw, Ns);
+            block_fft_pass<4, P, INV, NT>(a, b, tw, Ns);
         else
-            block_fft_pass<2, P, INV>(a, b, tw, Ns);
+            block_fft_pass<2, P, INV, NT>(a, b, tw, Ns);
         BLOCK_SYNC();
         N4_LDS D2* tmp = a;
         a = b;
@@ -1006,8 +1064,8 @@ HD N4_LDS D2* block_fft(N4_LDS D2* a, N4_LDS D2* b, const N4_LDS D2* tw) {
 // N4.py:31-101 (cudaN4.cu:733-820 did this on the host with FFTW).  Two real
 // transforms share one complex FFT (V in the real part, F in the
 // imaginary).  Reads and clears the volume's histogram.
-template <int WM, int P>
-HD void wiener_table_p(const VolDesc& V, double bmin, double slope, RunParams rp, N4_LDS unsigned char* smem,
+template <int WM, int P, int NT>
+HD void wiener_table_p(const VolDesc& V, double bmin, double slope, const RunParams& rp, N4_LDS unsigned char* smem,
                        N4_LDS float* Ef) {
     constexpr bool TEAM = WM == kWienerTeam;
     constexpr bool AGENT = WM != kWienerLocal;
@@ -1022,7 +1080,7 @@ HD void wiener_table_p(const VolDesc& V, double bmin, double slope, RunParams rp
     const double expF = 4.0 * log(2.0) / (scaledFWHM * scaledFWHM);
     const double scale = 2.0 * sqrt(log(2.0) / M_PI) / scaledFWHM;
     BLOCK_FOR(t)
-    for (int j = t; j < P; j += kBlock) {
+    for (int j = t; j < P; j += NT) {
         const int jj = (j <= half) ? j : P - j;
         const double Fj = (j == 0) ? scale : scale * exp((double)(-(int64_t)jj * jj) * expF);
         double Vj = 0.0;
@@ -1051,11 +1109,11 @@ HD void wiener_table_p(const VolDesc& V, double bmin, double slope, RunParams rp
     BLOCK_END
     BLOCK_SYNC();
     // the chain of transforms and pointwise steps, block-wide
-    N4_LDS D2* Z = block_fft<P, false>(z, y, tw);
+    N4_LDS D2* Z = block_fft<P, false, NT>(z, y, tw);
     N4_LDS D2* U = (Z == z) ? y : z;
     // Split Vf and Ff, Gf = conj(Ff)/(conj(Ff)Ff + noise), Uf = Vf*Re(Gf)
     BLOCK_FOR(t)
-    for (int k = t; k < P; k += kBlock) {
+    for (int k = t; k < P; k += NT) {
         const D2 a = Z[k];
         const D2 m = Z[(P - k) & (P - 1)];
         const D2 Vf{0.5 * (a.x + m.x), 0.5 * (a.y - m.y)};
@@ -1066,26 +1124,26 @@ HD void wiener_table_p(const VolDesc& V, double bmin, double slope, RunParams rp
     }
     BLOCK_END
     BLOCK_SYNC();
-    N4_LDS D2* Ur = block_fft<P, true>(U, Z, tw);
+    N4_LDS D2* Ur = block_fft<P, true, NT>(U, Z, tw);
     N4_LDS D2* Wb = (Ur == U) ? Z : U;
     const double invP = 1.0 / (double)P;
     BLOCK_FOR(t)
-    for (int j = t; j < P; j += kBlock) {
+    for (int j = t; j < P; j += NT) {
         double u = Ur[j].x * invP;
         if (u < 0.0) u = 0.0;
         Wb[j] = D2{(bmin + (double)(j - off) * slope) * u, u};
     }
     BLOCK_END
     BLOCK_SYNC();
-    N4_LDS D2* Wf = block_fft<P, false>(Wb, Ur, tw);
+    N4_LDS D2* Wf = block_fft<P, false, NT>(Wb, Ur, tw);
     N4_LDS D2* Wo = (Wf == Wb) ? Ur : Wb;
     BLOCK_FOR(t)
-    for (int k = t; k < P; k += kBlock) Wf[k] = cmul(Wf[k], ff[k]);
+    for (int k = t; k < P; k += NT) Wf[k] = cmul(Wf[k], ff[k]);
     BLOCK_END
     BLOCK_SYNC();
-    N4_LDS D2* R = block_fft<P, true>(Wf, Wo, tw);
+    N4_LDS D2* R = block_fft<P, true, NT>(Wf, Wo, tw);
     BLOCK_FOR(t)
-    for (int i = t; i < nb; i += kBlock) {
+    for (int i = t; i < nb; i += NT) {
         const double nu = R[off + i].x * invP;
         const double de = R[off + i].y * invP;
         const double e = (de != 0.0) ? nu / de : 0.0;
@@ -1098,20 +1156,20 @@ HD void wiener_table_p(const VolDesc& V, double bmin, double slope, RunParams rp
 }
 
 // wiener_table_p for the run's padded size P = 2^(ceil(log2 nbins) + 1),
-// 4 <= P <= 1024 (nbins in [2, 512]).
-template <int WM>
-HD void wiener_table(const VolDesc& V, double bmin, double slope, RunParams rp, N4_LDS unsigned char* smem,
+// 4 <= P <= 1024 (nbins in [2, 512]), by a block of NT threads.
+template <int WM, int NT = kBlock>
+HD void wiener_table(const VolDesc& V, double bmin, double slope, const RunParams& rp, N4_LDS unsigned char* smem,
                      N4_LDS float* Ef = nullptr) {
     switch (rp.P) {
-        case 4: wiener_table_p<WM, 4>(V, bmin, slope, rp, smem, Ef); break;
-        case 8: wiener_table_p<WM, 8>(V, bmin, slope, rp, smem, Ef); break;
-        case 16: wiener_table_p<WM, 16>(V, bmin, slope, rp, smem, Ef); break;
-        case 32: wiener_table_p<WM, 32>(V, bmin, slope, rp, smem, Ef); break;
-        case 64: wiener_table_p<WM, 64>(V, bmin, slope, rp, smem, Ef); break;
-        case 128: wiener_table_p<WM, 128>(V, bmin, slope, rp, smem, Ef); break;
-        case 256: wiener_table_p<WM, 256>(V, bmin, slope, rp, smem, Ef); break;
-        case 512: wiener_table_p<WM, 512>(V, bmin, slope, rp, smem, Ef); break;
-        default: wiener_table_p<WM, 1024>(V, bmin, slope, rp, smem, Ef); break;
+        case 4: wiener_table_p<WM, 4, NT>(V, bmin, slope, rp, smem, Ef); break;
+        case 8: wiener_table_p<WM, 8, NT>(V, bmin, slope, rp, smem, Ef); break;
+        case 16: wiener_table_p<WM, 16, NT>(V, bmin, slope, rp, smem, Ef); break;
+        case 32: wiener_table_p<WM, 32, NT>(V, bmin, slope, rp, smem, Ef); break;
+        case 64: wiener_table_p<WM, 64, NT>(V, bmin, slope, rp, smem, Ef); break;
+        case 128: wiener_table_p<WM, 128, NT>(V, bmin, slope, rp, smem, Ef); break;
+        case 256: wiener_table_p<WM, 256, NT>(V, bmin, slope, rp, smem, Ef); break;
+        case 512: wiener_table_p<WM, 512, NT>(V, bmin, slope, rp, smem, Ef); break;
+        default: wiener_table_p<WM, 1024, NT>(V, bmin, slope, rp, smem, Ef); break;
     }
 }
 
@@ -2185,7 +2243,7 @@ HD size_t carve_persist(N4_LDS unsigned char* base, const VolDesc& V, int nbins,
     size_t um = 0;
     {  // histogram
         Carve h{L.u, 0};
-        L.h = h.take<unsigned long long>((size_t)kHistLanes * (nbins | 1));
+        L.h = h.take<unsigned long long>((size_t)kHistLanes * hist_stride(nbins));
         um = h.off > um ? h.off : um;
     }
     {  // Wiener (carved again by wiener_table from the union base)
@@ -2410,7 +2468,7 @@ HD void body_persist(const VolDesc* vols, const Slab* slabs, const PWork* work, 
         // ---- ITER(lvl, it)
         const LevelDesc& LD = V.lev[lvl];
         const int CyCz = LD.C[1] * LD.C[2];
-        const int hs = nb | 1;
+        const int hs = hist_stride(nb);
         if (!degenerate) {
             hist_zero(S.h, hs);
             BLOCK_SYNC();
@@ -2490,6 +2548,14 @@ HD void body_persist(const VolDesc* vols, const Slab* slabs, const PWork* work, 
 }
 
 
+}  // namespace n4
+
+#ifndef N4_EMULATE
+#include "n4_resident.h"
+#endif
+
+namespace n4 {
+
 // ---------------------------------------------------------------- sizing --
 
 // MFMA tiles of 16 control points along one axis (0: not an MFMA launch).
@@ -2498,7 +2564,7 @@ static int cp_tiles(int c) { return (c + 15) / 16; }
 size_t lds_prep() { return align16(4 * kBlock * sizeof(double)); }
 size_t lds_level() { return align16(4 * kBlock * sizeof(double)); }
 size_t lds_hist(int nbins) {
-    return std::max(align16(4 * kBlock * sizeof(double)), align16((size_t)kHistLanes * (nbins | 1) * sizeof(uint64_t)));
+    return std::max(align16(4 * kBlock * sizeof(double)), align16((size_t)kHistLanes * hist_stride(nbins) * sizeof(uint64_t)));
 }
 size_t lds_wiener(int P) { return align16(4 * (size_t)P * sizeof(D2)); }
 size_t lds_lattice() { return align16(kBlock * sizeof(double)); }
@@ -2686,6 +2752,56 @@ int launch_persist(const VolDesc* vols, const Slab* slabs, const PWork* work, in
         hipLaunchKernelGGL(k_persist<2>, g, b, lds, s, vols, slabs, work, rp);
     else
         hipLaunchKernelGGL(k_persist<0>, g, b, lds, s, vols, slabs, work, rp);
+    return last_launch_status();
+}
+
+// Resident path: workgroups take the slots in order, each with the volume
+// whose team it joins, until none is left.
+template <int PREC>
+__global__ __launch_bounds__(kResThreads) void k_resident(const VolDesc* __restrict__ vols,
+                                                          const int32_t* __restrict__ slots, int nslots,
+                                                          uint32_t* ticket, RunParams rp) {
+    HIP_DYNAMIC_SHARED(double, smem_);
+    const LdsP smem = SMEM();
+    N4_LDS int* bc = reinterpret_cast<N4_LDS int*>(smem);
+    for (;;) {
+        __syncthreads();
+        if (threadIdx.x == 0)
+            bc[3] = (int)__hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        const int k = uni(bc[3]);
+        if (k >= nslots) return;
+        const VolDesc& V = vols[slots[k]];
+        const int rank = uni(res_join(V.res.team, V.res.nchunk, smem));
+        if (rank == -1) continue;  // its team runs without this workgroup
+        if (rank < 0 || !res_volume<PREC>(V, rp, rank, uni(bc[2]), smem)) return;
+    }
+}
+
+size_t lds_resident(const VolDesc& v, int nbins, int P, int prec) {
+    return carve_res(v, nbins, P, prec, nullptr);
+}
+
+int resident_limits(int* cus, size_t* lds) {
+    int dev = 0, bytes = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&bytes, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
+    *lds = (size_t)bytes;
+    return (int)e;
+}
+
+int launch_resident(const VolDesc* vols, const int32_t* slots, int nslots, int nwg, uint32_t* ticket, RunParams rp,
+                    size_t lds, void* stream) {
+    if (nwg <= 0) return 0;
+    const dim3 g(nwg), b(kResThreads);
+    const hipStream_t s = (hipStream_t)stream;
+    if (rp.prec == 1)
+        hipLaunchKernelGGL(k_resident<1>, g, b, lds, s, vols, slots, nslots, ticket, rp);
+    else if (rp.prec == 2)
+        hipLaunchKernelGGL(k_resident<2>, g, b, lds, s, vols, slots, nslots, ticket, rp);
+    else
+        hipLaunchKernelGGL(k_resident<0>, g, b, lds, s, vols, slots, nslots, ticket, rp);
     return last_launch_status();
 }
 

@@ -233,15 +233,18 @@ n4_status n4_reduce_max(n4_handle *h, uint64_t n, const float *d_in, float *out)
 n4_status n4_reduce_min(n4_handle *h, uint64_t n, const float *d_in, float *out);
 
 /* ---- launch schedule and autotuner (no counterpart in the reference) --- */
-/* How n4_correct / n4_correct_batch lay out their launches.  Two paths run
+/* How n4_correct / n4_correct_batch lay out their launches.  Three paths run
  * the level/iteration loop (cudaN4.cu:1517-1657):
  *   steps: the host enqueues identical steps of five launches (histogram,
  *     Wiener, fit, lattice update, evaluation) per volume group, each
  *     volume advancing its own state machine on the device;
  *   teams: one persistent launch in which a team of workgroups per volume
  *     runs the volume's whole loop, synchronising at team barriers (every
- *     workgroup of the launch is resident at once).
- * Both run the same per-tile arithmetic, so they give the same bits.
+ *     workgroup of the launch is resident at once);
+ *   resident: one launch in which teams, formed by the workgroups that
+ *     arrive, keep a volume's foreground packed and its tables in LDS for
+ *     the whole loop; up to 16 control points along y and z.
+ * All run the same per-tile arithmetic, so they give the same bits.
  * Results do not depend on the schedule except through the summation order
  * of the FP64 convergence partials (one partial per tile).  A field left 0 takes the
  * environment override (N4_GROUPS, N4_STEP_TILE_VOX, N4_GRAPH_STEPS) if set,
@@ -257,13 +260,18 @@ typedef struct n4_tuning {
     uint32_t eval_kernel;      /* field-increment kernel of the MFMA
                                   precisions: N4_EVAL_FP32 (default) or
                                   N4_EVAL_MFMA; FP32 runs use FP32 */
-    uint32_t path;             /* N4_PATH_AUTO (default: the step kernels,
-                                  the faster path on every workload measured);
+    uint32_t path;             /* N4_PATH_AUTO (default): the resident kernel
+                                  where it covers the call, else the step
+                                  kernels; with one of the fields above set,
+                                  the step kernels they describe;
                                   N4_PATH_STEPS; N4_PATH_TEAMS: the persistent
                                   team kernel (N4_ERR_UNSUPPORTED where the
                                   batch is not eligible) */
-    uint32_t team_wgs_per_cu;  /* persistent path: workgroups per compute
-                                  unit (0 = as many as fit, at most 4) */
+    uint32_t team_wgs_per_cu;  /* team path: workgroups per compute unit
+                                  (0 = as many as fit, at most 4); with
+                                  N4_PATH_AUTO, nonzero asks for the resident
+                                  kernel (one per compute unit) whatever the
+                                  fields above */
     float ms;                  /* n4_autotune_batch: wall time of one batch */
 } n4_tuning;
 #define N4_EVAL_FP32 1u
@@ -278,7 +286,7 @@ n4_status n4_set_tuning(n4_handle *h, const n4_tuning *t);
 /* Times n4_correct_batch on these volumes (outputs are written) under each
  * candidate schedule -- groups {1,2,4,8} up to nvol, tiles {4096, 8192,
  * 16384} voxels, graphs {off, 8, 16} steps and, for the MFMA precisions,
- * both field-increment kernels -- keeps the fastest on the handle and
+ * both field-increment kernels, and the resident kernel -- keeps the fastest on the handle and
  * returns it in *best (ms = its best wall time). */
 n4_status n4_autotune_batch(n4_handle *h, const n4_volume *vols, uint32_t nvol,
                             const n4_params *p, n4_tuning *best, void *stream);
@@ -297,7 +305,7 @@ typedef enum n4_kernel_id {
     N4_K_LATTICE = 8, /* mode-x contraction + lattice update (stage calls) */
     N4_K_UPDATE = 9,  /* lattice update of a correction step */
     N4_K_TEAMS = 10,  /* persistent path: every volume's level/iteration loop */
-    /* Phases of the persistent path, timed inside the launch by each team's
+    /* Phases of the persistent paths, timed inside the launch by each team's
      * leader workgroup (device clock; total over the volumes' leaders,
      * launches = iteration steps).  Enabled with the N4_K_TEAMS bit. */
     N4_K_T_WAIT = 11,   /* team barrier waits */

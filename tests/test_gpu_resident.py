@@ -1,0 +1,105 @@
+"""The resident kernel (one launch runs every volume's level/iteration loop,
+a team of workgroups per volume) against the step path on the same inputs.
+
+Both form the fit's and the field's sums in the same order with the same
+roundings, so fields, lattices and normalised images are equal bit for bit;
+only the FP64 convergence sums have another order (compared to 1e-9), which
+moves no stop decision here."""
+import numpy as np
+import pytest
+
+import parity_cases as PC
+
+pytestmark = pytest.mark.gpu
+
+
+def _both(gpu, vols, tile=0, **kw):
+    try:
+        gpu.set_tuning(path="steps", step_tile_voxels=tile, groups=1)
+        ref = gpu.correct_batch(vols, **kw)
+        # a workgroup count asks for the persistent kernel whatever the tile
+        gpu.set_tuning(step_tile_voxels=tile, team_wgs_per_cu=1)
+        out = gpu.correct_batch(vols, **kw)
+        again = gpu.correct_batch(vols, **kw)
+    finally:
+        gpu.set_tuning(reset=True)
+    for a, b, c in zip(ref, out, again):
+        assert a["iterations"] == b["iterations"]
+        assert (a["n_mask_full"], a["n_mask_work"]) == (b["n_mask_full"], b["n_mask_work"])
+        assert np.allclose(a["last_cv"], b["last_cv"], rtol=1e-9, atol=1e-12)
+        for k in ("log_bias", "normalized", "lattice"):
+            assert np.array_equal(a[k], b[k]), k
+            assert np.array_equal(b[k], c[k]), k  # reproducible
+    return ref, out
+
+
+def _vol(dims, seed, mask="f32"):
+    im, m, _ = PC.small_phantom(dims, seed=seed)
+    if mask == "none":
+        return im, None
+    return im, m.astype(np.uint8) if mask == "u8" else m
+
+
+@pytest.mark.parametrize("precision", ["fp32", "bf16", "split_bf16"])
+@pytest.mark.parametrize("dims,tile", [((17, 16, 16), 0), ((9, 33, 31), 0), ((20, 70, 45), 512), ((12, 130, 67), 1024),
+                                       ((64, 15, 129), 0), ((3, 5, 200), 0), ((40, 48, 96), 2048)])
+def test_shapes(gpu, precision, dims, tile):
+    _both(gpu, [_vol(dims, 5)], tile, levels=3, max_iter=[5, 4, 3], fixed_iterations=True, precision=precision)
+
+
+@pytest.mark.parametrize("mask", ["f32", "u8", "none"])
+@pytest.mark.parametrize("precision", ["fp32", "bf16"])
+def test_uneven_batch_masks_and_shrinks(gpu, precision, mask):
+    vols = [_vol(d, 30 + k, mask) for k, d in enumerate([(60, 52, 44), (34, 66, 50), (82, 38, 56), (97, 101, 89)])]
+    _both(gpu, vols, levels=4, max_iter=[8, 6, 4, 2], threshold=0.001, precision=precision, shrink=[1, 1, 2, 3])
+
+
+@pytest.mark.parametrize("kw", [dict(nbins=500), dict(nbins=16), dict(ncpt=(4, 5, 6), levels=2), dict(ncpt=(9, 16, 16), levels=1),
+                                dict(max_iter=[3, 0, 2]), dict(fwhm=0.4, noise=0.1)])
+def test_parameters(gpu, kw):
+    p = dict(dict(levels=3, max_iter=[4, 3, 2], threshold=0.0005), **kw)
+    _both(gpu, [_vol((44, 40, 36), 8)], **p)
+
+
+def test_weighted_mask(gpu):
+    im, m, _ = PC.small_phantom((48, 44, 40), seed=9)
+    w = (m * np.linspace(0.2, 1.0, 40, dtype=np.float32)).astype(np.float32)
+    _both(gpu, [(im, w)], levels=3, max_iter=[6, 5, 4], threshold=0.001, weighted_mask=True)
+
+
+def test_degenerate_masks(gpu):
+    im, m, _ = PC.small_phantom((30, 28, 26), seed=6)
+    one = np.zeros_like(m)
+    one[11, 13, 17] = 1
+    split = m.copy()
+    split[8:20] = 0  # slabs without foreground between two with
+    ref, out = _both(gpu, [(im, np.zeros_like(m)), (np.full(im.shape, 100.0, np.float32), m), (im, one), (im, split)],
+                     levels=2, max_iter=[4, 4], threshold=0.001)
+    assert out[0]["n_mask_work"] == 0 and np.all(out[0]["log_bias"] == 0)
+
+
+def test_more_volumes_than_compute_units(gpu):
+    vols = [_vol((12 + k % 7, 14, 13), 100 + k) for k in range(40)] * 8
+    _both(gpu, vols, levels=2, max_iter=[3, 3], threshold=0.001)
+
+
+def test_large_single_volume_of_many_batches(gpu):
+    """One workgroup holds more units than one LDS batch: few chunks, many
+    slabs (a long x axis with small slabs in a batch of larger volumes)."""
+    vols = [_vol((700, 16, 16), 3)] + [_vol((60, 70, 64), 40 + k) for k in range(24)]
+    _both(gpu, vols, levels=2, max_iter=[3, 2], fixed_iterations=True, precision="bf16")
+    _both(gpu, vols, levels=2, max_iter=[3, 2], fixed_iterations=True)
+
+
+def test_covered_up_to_16_control_points_then_steps(gpu):
+    """19 control points along y and z run on the step kernels: the default
+    call equals them bit for bit."""
+    v = [_vol((40, 36, 32), 4)]
+    kw = dict(levels=4, max_iter=[2] * 4, ncpt=(5, 5, 5), fixed_iterations=True)
+    a = gpu.correct_batch(v, **kw)
+    try:
+        gpu.set_tuning(path="steps")
+        b = gpu.correct_batch(v, **kw)
+    finally:
+        gpu.set_tuning(reset=True)
+    assert np.array_equal(a[0]["log_bias"], b[0]["log_bias"])
