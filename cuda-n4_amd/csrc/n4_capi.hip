@@ -234,8 +234,19 @@ static void cubic_bspline(double t, double w[4]) {  // N4.py:174-181
     w[3] = t3 / 6.0;
 }
 
-// Span index / weights per position (N4.py:192, 210-217) and, per control
-// point, the contiguous range of positions whose 4-support contains it.
+// Span index and weights of position i (N4.py:192, 210-217).
+static int axis_position(int i, double span, int ncpt, double w[4]) {
+    const double pos = (double)i + 0.5;
+    int b = (int)floor(pos / span);
+    const double t = (pos - (double)b * span) / span;
+    if (b < 0) b = 0;
+    if (b > ncpt - 4) b = ncpt - 4;
+    cubic_bspline(t, w);
+    return b;
+}
+
+// Entries of a working-grid axis and, per control point, the contiguous
+// range of positions whose 4-support contains it.
 static void axis_table(int npos, double domain, int ncpt, AxisEntry* out, int32_t* sup) {
     const double span = domain / (double)(ncpt - 3);
     for (int c = 0; c < ncpt; ++c) {
@@ -243,13 +254,8 @@ static void axis_table(int npos, double domain, int ncpt, AxisEntry* out, int32_
         sup[2 * c + 1] = 0;
     }
     for (int i = 0; i < npos; ++i) {
-        const double pos = (double)i + 0.5;
-        int b = (int)floor(pos / span);
-        const double t = (pos - (double)b * span) / span;
-        if (b < 0) b = 0;
-        if (b > ncpt - 4) b = ncpt - 4;
         double w[4];
-        cubic_bspline(t, w);
+        const int b = axis_position(i, span, ncpt, w);
         const double S = w[0] * w[0] + w[1] * w[1] + w[2] * w[2] + w[3] * w[3];
         AxisEntry& e = out[i];
         memset(&e, 0, sizeof e);
@@ -265,6 +271,17 @@ static void axis_table(int npos, double domain, int ncpt, AxisEntry* out, int32_
     }
     for (int c = 0; c < ncpt; ++c)
         if (sup[2 * c] >= sup[2 * c + 1]) sup[2 * c] = sup[2 * c + 1] = 0;
+}
+
+// Weights and span indices of a full-resolution axis, the last position
+// repeated three times.
+static void full_table(int npos, double domain, int ncpt, F4* w, int32_t* b) {
+    const double span = domain / (double)(ncpt - 3);
+    for (int i = 0; i < npos + 3; ++i) {
+        double d[4];
+        b[i] = axis_position(i < npos ? i : npos - 1, span, ncpt, d);
+        for (int a = 0; a < 4; ++a) w[i].v[a] = (float)d[a];
+    }
 }
 
 static int padded_size(int nbins, int* log2P) {  // N4.py:31-37
@@ -347,7 +364,7 @@ struct Plan {
     size_t lds_fit_max[kMaxLevels] = {0}, lds_eval_max[kMaxLevels] = {0}, lds_eval32_max[kMaxLevels] = {0};
     int cx_max[kMaxLevels] = {0};
     int mt[kMaxLevels] = {0}, nt[kMaxLevels] = {0};  // MFMA tiles along y, z per level
-    size_t lds_hist = 0, lds_wiener = 0, lds_recon = 0;
+    size_t lds_hist = 0, lds_wiener = 0, lds_recon = 0, lds_recon_limit = 0;
     // persistent path
     size_t off_work = 0;     // PWork[n_work] in the upload region
     int n_work = 0;
@@ -386,7 +403,10 @@ static const int kStepTileVox = 8192;
 // Convergence values recorded per volume and call (iterations after the
 // first kTraceCap of a call are not recorded).
 static const int kTraceCap = 4096;
-static const int kReconTileVox = 8192;
+// Full-resolution voxels per reconstruction tile: about kReconTiles tiles (as
+// many workgroups as the device holds at four per compute unit), so that a
+// tile's set-up is paid once per resident workgroup, within these bounds.
+static const int kReconTiles = 1024, kReconTileMin = 8192, kReconTileMax = 32768;
 // Resident path: 16-row units of foreground per workgroup of a full team.
 static const int kResUnitsPerChunk = 4;
 // Default iteration steps per captured graph, and the largest chunk.
@@ -568,6 +588,9 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
         int prep_rows, prep_tiles_x, recon_rows, recon_tiles_x, wtile_rows, wtiles_x;
     };
     std::vector<VInfo> vi(nv);
+    double full_vox = 0.0;
+    for (int v = 0; v < nv; ++v) full_vox += (double)in[v].F[0] * in[v].F[1] * in[v].F[2];
+    const int recon_tile = (int)std::min<double>(kReconTileMax, std::max<double>(kReconTileMin, full_vox / kReconTiles));
     int nws = 0, nfs = 0, nps = 0;
     for (int v = 0; v < nv; ++v) {
         VInfo& I = vi[v];
@@ -579,7 +602,7 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
         I.part_stride = (size_t)Cf[1] * Cf[2];
         I.prep_rows = rows_for(I.W[1], I.W[2], kPrepTileVox);
         I.prep_tiles_x = (I.W[1] + I.prep_rows - 1) / I.prep_rows;
-        I.recon_rows = rows_for(in[v].F[1], in[v].F[2], kReconTileVox);
+        I.recon_rows = rows_for(in[v].F[1], in[v].F[2], recon_tile);
         I.recon_tiles_x = (in[v].F[1] + I.recon_rows - 1) / I.recon_rows;
         step_tiles(I.W, tiled, tile_vox, &I.wtile_rows, &I.wtiles_x);
         nws += I.W[0] * I.wtiles_x;
@@ -617,7 +640,7 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
         int npos;
         double domain;
         int ncpt;
-        size_t oa, os;  // entries; support ranges (working-grid tables)
+        size_t oa, os;  // entries and support ranges; full-resolution tables: weights and span indices
         bool full;
     };
     std::vector<AxisJob> ax_jobs;
@@ -626,14 +649,15 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
         const auto key = std::make_tuple(full, npos, domain, ncpt);
         auto it = ax_index.find(key);
         if (it == ax_index.end()) {
-            AxisJob j{npos, domain, ncpt, lay.take(sizeof(AxisEntry) * npos, 64),
-                      full ? 0 : lay.take(sizeof(int32_t) * 2 * ncpt, 16), full};
+            // (full-resolution tables: weights, span indices, three positions of padding)
+            AxisJob j{npos, domain, ncpt, full ? lay.take(sizeof(F4) * (npos + 3), 64) : lay.take(sizeof(AxisEntry) * npos, 64),
+                      full ? lay.take(sizeof(int32_t) * (npos + 3), 16) : lay.take(sizeof(int32_t) * 2 * ncpt, 16), full};
             it = ax_index.emplace(key, ax_jobs.size()).first;
             ax_jobs.push_back(j);
         }
         return ax_jobs[it->second];
     };
-    std::vector<size_t> off_ax(nv * kMaxLevels * 3), off_sup(nv * kMaxLevels * 3), off_fax(nv * 3);
+    std::vector<size_t> off_ax(nv * kMaxLevels * 3), off_sup(nv * kMaxLevels * 3), off_fw(nv * 3), off_fb(nv * 3);
     for (int v = 0; v < nv; ++v)
         for (int l = 0; l < L; ++l)
             for (int d = 0; d < 3; ++d) {
@@ -643,9 +667,11 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
             }
     if (need_tables_full)
         for (int v = 0; v < nv; ++v)
-            for (int d = 0; d < 3; ++d)
-                off_fax[v * 3 + d] =
-                    axis_slot(true, in[v].F[d], (double)vi[v].W[d] * (double)in[v].s, vi[v].C[L - 1][d]).oa;
+            for (int d = 0; d < 3; ++d) {
+                const AxisJob& j = axis_slot(true, in[v].F[d], (double)vi[v].W[d] * (double)in[v].s, vi[v].C[L - 1][d]);
+                off_fw[v * 3 + d] = j.oa;
+                off_fb[v * 3 + d] = j.os;
+            }
     P->upload_bytes = lay.take(0);
 
     // per-volume working buffers
@@ -753,15 +779,12 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
         const int nj = (int)ax_jobs.size();
         std::atomic<int> next{0};
         auto run_jobs = [&]() {
-            std::vector<int32_t> sup_tmp;
             for (int k = next.fetch_add(1); k < nj; k = next.fetch_add(1)) {
                 const AxisJob& j = ax_jobs[k];
-                int32_t* sup = (int32_t*)(hb + j.os);
-                if (j.full) {
-                    sup_tmp.assign(2 * (size_t)j.ncpt, 0);
-                    sup = sup_tmp.data();
-                }
-                axis_table(j.npos, j.domain, j.ncpt, (AxisEntry*)(hb + j.oa), sup);
+                if (j.full)
+                    full_table(j.npos, j.domain, j.ncpt, (F4*)(hb + j.oa), (int32_t*)(hb + j.os));
+                else
+                    axis_table(j.npos, j.domain, j.ncpt, (AxisEntry*)(hb + j.oa), (int32_t*)(hb + j.os));
             }
         };
         size_t entries = 0;
@@ -855,7 +878,10 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
             LD.mCz = magic_div((uint32_t)LD.C[2]);
         }
         if (need_tables_full)
-            for (int d = 0; d < 3; ++d) D.fax[d] = (const AxisEntry*)(base + off_fax[v * 3 + d]);
+            for (int d = 0; d < 3; ++d) {
+                D.fw[d] = (const F4*)(base + off_fw[v * 3 + d]);
+                D.fb[d] = (const int32_t*)(base + off_fb[v * 3 + d]);
+            }
         P->desc[v] = D;
         if (teams) {
             PWork* wk = (PWork*)(hb + P->off_work);
@@ -885,7 +911,10 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
             P->mt[l] = mfma_tiles(D.lev[l].C[1]);
             P->nt[l] = mfma_tiles(D.lev[l].C[2]);
         }
-        if (need_tables_full) P->lds_recon = std::max(P->lds_recon, lds_recon(D));
+        if (need_tables_full) {
+            P->lds_recon = std::max(P->lds_recon, lds_recon(D));
+            P->lds_recon_limit = std::max(P->lds_recon_limit, lds_recon_limit(D));
+        }
     }
     if (res) {
         // the largest volumes first, each with all its slots in a row
@@ -909,7 +938,7 @@ static n4_status check_lds(const Plan& P, bool grid_kernels, bool recon) {
     size_t worst = std::max(P.lds_hist, P.lds_wiener);
     if (grid_kernels)
         for (int l = 0; l < P.nlevels; ++l) worst = std::max(worst, std::max(P.lds_fit_max[l], P.lds_eval_max[l]));
-    if (recon) worst = std::max(worst, P.lds_recon);
+    if (recon) worst = std::max(worst, std::max(P.lds_recon, P.lds_recon_limit));
     if (worst > kLdsCap)
         return fail(N4_ERR_UNSUPPORTED, "volume/lattice too large for one workgroup's LDS (%zu bytes)", worst);
     return N4_OK;
@@ -1490,7 +1519,8 @@ static n4_status run_batch(n4_handle* h, const std::vector<VolIn>& in_user, cons
     // the volume states and, on the resident path, the team words behind them
     const size_t state_bytes =
         resident ? P.off_team + 64 * (size_t)(nv + 1) - P.off_state : sizeof(VolState) * (size_t)nv;
-    s = check_lds(P, !teams_path && !resident, true);
+    // (a call that the step kernels' LDS refuses is refused on the resident path too)
+    s = check_lds(P, !teams_path, true);
     if (s != N4_OK) return s;
     if (plan_reused) {
         // the arena still holds the rest of the upload region (slab lists,

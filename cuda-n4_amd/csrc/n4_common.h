@@ -140,7 +140,10 @@ struct VolDesc {
     int32_t trace_cap;         // entries of cvtrace (later iterations are not recorded)
     float* lvlat;              // each level's lattice at the level's end, level-major (null: none)
     LevelDesc lev[kMaxLevels];
-    const AxisEntry* fax[3];   // full-res axis tables for the final lattice
+    // full-resolution axis tables for the final lattice: weights and span
+    // index per position (three positions of padding repeat the last)
+    const F4* fw[3];
+    const int32_t* fb[3];
     int32_t nlevels;
     int32_t max_iter[kMaxLevels];
     int32_t part_stride;       // floats per slab in part (max Cy*Cz)

@@ -1809,11 +1809,19 @@ HD void body_eval(const VolDesc* vols, const Slab* slabs, RunParams rp, int bid,
 // Final field at full resolution from the last lattice (N4.py:329-330,
 // cudaN4.cu:1700-1729): separable evaluation, then normalised image
 // (thresholded input / exp(field)), optional exp(field) and field.
+//
+// Bound by HBM once the vector work is small: a thread keeps one column of
+// four consecutive z for all the rows it takes, so the z factors stay in its
+// registers, one 16-byte access moves four voxels of each array (dword
+// alignment is enough, so rows of any length do) and a quad costs 5 LDS
+// reads and 20 FMAs.  (With voxels dealt to the lanes one by one -- a
+// division by the row length, 4 z factors and 4 row values from LDS each --
+// the kernel was bound by vector instructions: 64 volumes of 652 M voxels
+// 2010 us, 3.9 TB/s, now 1497 us, 5.2 TB/s; 512x512x320 260 -> 196 us;
+// 256x256x176, field only, 23.8 -> 21.4 us.)
 struct ReconLds {
     N4_LDS float* A;
     N4_LDS float* B;
-    N4_LDS float* zw;
-    N4_LDS int* zb;
     N4_LDS float* yw;  // [tile rows][4] y factors of the tile's rows
     N4_LDS int* yb;
 };
@@ -1823,22 +1831,152 @@ struct ReconLds {
 // barrier between its voxels.
 constexpr int kReconChunkFloats = 8192;
 HD int recon_chunk_rows(int tile_rows, int Cz) {
-    int r = kReconChunkFloats / (Cz > 0 ? Cz : 1);
+    int r = kReconChunkFloats / (Cz + 1 > 0 ? Cz + 1 : 1);
     if (r < 1) r = 1;
     return r < tile_rows ? r : tile_rows;
 }
 
-HD size_t carve_recon(N4_LDS unsigned char* base, int Z, int R, int Yt, int Cy, int Cz, ReconLds* o) {
+// (A row of B has one slot past its Cz values: the fifth of a quad whose
+// control points end at the last one, met with a zero factor.)
+HD size_t carve_recon(N4_LDS unsigned char* base, int R, int Yt, int Cy, int Cz, ReconLds* o) {
     Carve c{base, 0};
     ReconLds L;
     L.A = c.take<float>((size_t)Cy * Cz);
-    L.B = c.take<float>((size_t)R * Cz);
-    L.zw = c.take<float>((size_t)4 * Z);
-    L.zb = c.take<int>(Z);
+    L.B = c.take<float>((size_t)R * (Cz + 1));
     L.yw = c.take<float>((size_t)4 * Yt);
     L.yb = c.take<int>(Yt);
     if (o) *o = L;
     return align16(c.off);
+}
+
+// A column of four z positions: factors of the five control points from b
+// on that they touch (near: all four start at b or b + 1); spans shorter
+// than four voxels may need more and go voxel by voxel.
+struct ReconCol {
+    float w[4][5];
+    int b;
+    bool near;
+};
+HD ReconCol recon_col(const VolDesc& V, int z0) {
+    ReconCol c;
+    const F4* w = V.fw[2] + z0;
+    const int32_t* b = V.fb[2] + z0;
+    c.b = gp(b)[0];
+    c.near = true;
+    UNROLL for (int j = 0; j < 4; ++j) {
+        const F4 e = load_quad(w[j].v);
+        const int d = gp(b)[j] - c.b;
+        c.near = c.near && d <= 1;
+        UNROLL for (int k = 0; k < 5; ++k)
+            c.w[j][k] = d == 0 ? (k < 4 ? e.v[k < 4 ? k : 3] : 0.0f) : (k > 0 ? e.v[k > 0 ? k - 1 : 0] : 0.0f);
+    }
+    return c;
+}
+
+HD void store_run4(float* p, const F4& x) {
+#ifdef N4_DEVICE_PASS
+    typedef float v4u __attribute__((ext_vector_type(4), aligned(4)));
+    v4u y = {x.v[0], x.v[1], x.v[2], x.v[3]};
+    *reinterpret_cast<N4_GLOBAL v4u*>(gp(p)) = y;
+#else
+    memcpy(p, x.v, sizeof x.v);
+#endif
+}
+
+// A thread's place in a chunk: column block 0's quad and its first row, with
+// the column's factors and the image quads of its first rows.  On the
+// device they are loaded in the set-up round of the tile, before the
+// barriers.
+constexpr int kReconRows = 4;  // rows in flight
+struct ReconThread {
+    int cols, nr, r0, q0;
+    ReconCol c;
+    F4 x[kReconRows];
+};
+// Image quads of rows r, r + nr, ... (zeros past ny) at z0 of a chunk.
+HD void recon_load(const float* im, size_t v0, int Z, int z0, int r, int nr, int ny, F4 (&x)[kReconRows]) {
+    const int nz = Z - z0 < 4 ? Z - z0 : 4;
+    UNROLL for (int u = 0; u < kReconRows; ++u) {
+        const int rr = r + u * nr;
+        x[u] = F4{{0.0f, 0.0f, 0.0f, 0.0f}};
+        if (im && rr < ny) {
+            const float* p = im + v0 + (size_t)rr * Z + z0;
+            if (nz == 4) {
+                x[u] = load_run4(p);
+            } else {
+                UNROLL for (int j = 0; j < 3; ++j)
+                    if (j < nz) x[u].v[j] = gp(p)[j];
+            }
+        }
+    }
+}
+template <int NT>
+HD void recon_thread(const VolDesc& V, int t, size_t v0, int ny, ReconThread& T) {
+    const int nq = (V.F[2] + 3) >> 2;
+    T.cols = nq < NT ? nq : NT;
+    T.nr = NT / T.cols;
+    T.r0 = t / T.cols;
+    T.q0 = t - T.r0 * T.cols;
+    if (T.r0 >= T.nr) T.r0 = 1 << 30;  // a spare thread
+    T.c = recon_col(V, 4 * T.q0);
+    recon_load(V.out_norm ? V.im : nullptr, v0, V.F[2], 4 * T.q0, T.r0, T.nr, ny, T.x);
+}
+
+// The voxels of rows [0, ny) of a chunk (B: its y-contracted rows; v0: the
+// first voxel's index) of thread T; first: its image quads are those of this
+// chunk.
+HD void recon_rows(const VolDesc& V, const N4_LDS float* B, int Cz, size_t v0, int ny, float low, ReconThread& T,
+                   bool first) {
+    const int Z = V.F[2], nq = (Z + 3) >> 2, nr = T.nr;
+    float* o_lb = V.out_logbias;
+    float* o_b = V.out_bias;
+    float* o_n = V.out_norm;
+    const float* im = o_n ? V.im : nullptr;
+    for (int q = T.q0; q < nq; q += T.cols) {
+        const int z0 = 4 * q, nz = Z - z0 < 4 ? Z - z0 : 4;
+        if (q != T.q0) T.c = recon_col(V, z0);  // (rows of more than NT quads)
+        for (int r = T.r0; r < ny; r += kReconRows * nr) {
+            if (!first || q != T.q0 || r != T.r0) recon_load(im, v0, Z, z0, r, nr, ny, T.x);
+            UNROLL for (int u = 0; u < kReconRows; ++u) {
+                const int rr = r + u * nr;
+                if (rr >= ny) break;
+                const N4_LDS float* br = B + rr * (Cz + 1) + T.c.b;
+                F4 f, n, e;
+                if (T.c.near) {
+                    const float b0 = br[0], b1 = br[1], b2 = br[2], b3 = br[3], b4 = br[4];
+                    UNROLL for (int j = 0; j < 4; ++j)
+                        f.v[j] = T.c.w[j][0] * b0 + T.c.w[j][1] * b1 + T.c.w[j][2] * b2 + T.c.w[j][3] * b3 + T.c.w[j][4] * b4;
+                } else {
+                    for (int j = 0; j < 4; ++j) {
+                        const F4 a = V.fw[2][z0 + j];
+                        const N4_LDS float* bj = B + rr * (Cz + 1) + V.fb[2][z0 + j];
+                        f.v[j] = a.v[0] * bj[0] + a.v[1] * bj[1] + a.v[2] * bj[2] + a.v[3] * bj[3];
+                    }
+                }
+                UNROLL for (int j = 0; j < 4; ++j) {
+                    // thresholded image / exp(f) as a product with exp(-f):
+                    // no IEEE division per voxel (within 2 ulp of the quotient)
+                    const float xo = (T.x[u].v[j] <= low) ? 0.0f : T.x[u].v[j];  // N4.py:285
+                    n.v[j] = o_n ? xo * expf(-f.v[j]) : 0.0f;
+                    e.v[j] = o_b ? expf(f.v[j]) : 0.0f;
+                }
+                const size_t o = v0 + (size_t)rr * Z + z0;
+                if (nz == 4) {
+                    if (o_lb) store_run4(o_lb + o, f);
+                    if (o_b) store_run4(o_b + o, e);
+                    if (o_n) store_run4(o_n + o, n);
+                } else {
+                    UNROLL for (int j = 0; j < 3; ++j) {
+                        if (j >= nz) continue;
+                        if (o_lb) gp(o_lb)[o + j] = f.v[j];
+                        if (o_b) gp(o_b)[o + j] = e.v[j];
+                        if (o_n) gp(o_n)[o + j] = n.v[j];
+                    }
+                }
+            }
+        }
+        if (q != T.q0 && q + T.cols >= nq) T.c = recon_col(V, 4 * T.q0);  // back for the next chunk
+    }
 }
 
 HD void body_recon(const VolDesc* vols, const Slab* slabs, int level, RunParams rp, int bid,
@@ -1851,33 +1989,34 @@ HD void body_recon(const VolDesc* vols, const Slab* slabs, int level, RunParams 
     const int CyCz = Cy * Cz;
     const int R = recon_chunk_rows(V.recon_rows, Cz);
     ReconLds S;
-    carve_recon(smem, Z, R, V.recon_rows, Cy, Cz, &S);
+    carve_recon(smem, R, V.recon_rows, Cy, Cz, &S);
     const int x = sl.x;
-    const AxisEntry ex = V.fax[0][x];
-    // set-up: x-contracted planes, and the z and (tile) y factor tables, all
-    // from one round of global loads
+    const F4 ex = V.fw[0][x];
+    const int xb = V.fb[0][x];
+    // set-up: x-contracted planes, the (tile) y factor table and the threads'
+    // own columns and first image quads, from one round of global loads
+    const size_t vt = ((size_t)x * Y + sl.y0) * Z;
+#ifdef N4_DEVICE_PASS
+    ReconThread T;
+    recon_thread<kBlock>(V, (int)threadIdx.x, vt, sl.ny < R ? sl.ny : R, T);
+#endif
     BLOCK_FOR(t)
     for (int pr = t; pr < CyCz; pr += kBlock) {
         float a = 0.0f;
-        for (int k = 0; k < 4; ++k) a += ex.w[k] * V.latf[(size_t)(ex.b + k) * CyCz + pr];
+        for (int k = 0; k < 4; ++k) a += ex.v[k] * V.latf[(size_t)(xb + k) * CyCz + pr];
         S.A[pr] = a;
     }
-    for (int z = t; z < Z; z += kBlock) {
-        const AxisEntry& e = V.fax[2][z];
-        for (int k = 0; k < 4; ++k) S.zw[4 * z + k] = e.w[k];
-        S.zb[z] = e.b;
-    }
     for (int r = t; r < sl.ny; r += kBlock) {
-        const AxisEntry& e = V.fax[1][sl.y0 + r];
-        for (int k = 0; k < 4; ++k) S.yw[4 * r + k] = e.w[k];
-        S.yb[r] = e.b;
+        const F4 e = V.fw[1][sl.y0 + r];
+        for (int k = 0; k < 4; ++k) S.yw[4 * r + k] = e.v[k];
+        S.yb[r] = V.fb[1][sl.y0 + r];
     }
+    for (int r = t; r < R; r += kBlock) S.B[r * (Cz + 1) + Cz] = 0.0f;
     BLOCK_END
     BLOCK_SYNC();
     const int yend = sl.y0 + sl.ny;
     for (int y0 = sl.y0; y0 < yend; y0 += R) {
         const int ny = (yend - y0 < R) ? yend - y0 : R;
-        const size_t base = ((size_t)x * Y + y0) * Z;
         BLOCK_FOR(t)
         for (int pr = t; pr < ny * Cz; pr += kBlock) {
             const int r = (int)fdiv((uint32_t)pr, LD.mCz), c = pr - r * Cz;
@@ -1886,44 +2025,18 @@ HD void body_recon(const VolDesc* vols, const Slab* slabs, int level, RunParams 
             const int b0 = S.yb[tr];
             float b = 0.0f;
             for (int k = 0; k < 4; ++k) b += yw[k] * S.A[(b0 + k) * Cz + c];
-            S.B[pr] = b;
+            S.B[r * (Cz + 1) + c] = b;
         }
         BLOCK_END
         BLOCK_SYNC();
         BLOCK_FOR(t)
-        const N4_GLOBAL float* im = gp(V.im);
-        N4_GLOBAL float* o_lb = gp(V.out_logbias);
-        N4_GLOBAL float* o_b = gp(V.out_bias);
-        N4_GLOBAL float* o_n = gp(V.out_norm);
-        // consecutive lanes on consecutive voxels, kReconLoads image loads
-        // in flight per thread (8 measured 9% faster than 16 once the
-        // division became a product)
-        constexpr int kReconLoads = 8;
-        for (int v0 = 0; v0 < ny * Z; v0 += kReconLoads * kBlock) {
-            float xin[kReconLoads];
-            UNROLL for (int u = 0; u < kReconLoads; ++u) {
-                const int v = v0 + u * kBlock + t;
-                xin[u] = (o_n && v < ny * Z) ? im[base + v] : 0.0f;
-            }
-            UNROLL for (int u = 0; u < kReconLoads; ++u) {
-                const int v = v0 + u * kBlock + t;
-                if (v >= ny * Z) continue;
-                const int r = (int)fdiv((uint32_t)v, V.mF2), z = v - r * Z;
-                const N4_LDS float* wz = S.zw + 4 * z;
-                const N4_LDS float* br = S.B + r * Cz + S.zb[z];
-                const float f = wz[0] * br[0] + wz[1] * br[1] + wz[2] * br[2] + wz[3] * br[3];
-                if (o_lb) o_lb[base + v] = f;
-                if (o_b) o_b[base + v] = expf(f);
-                if (o_n) {
-                    // thresholded image / exp(f) as a product with exp(-f):
-                    // no IEEE division per voxel (within 2 ulp of the quotient)
-                    const float xo = (xin[u] <= rp.low_f) ? 0.0f : xin[u];  // N4.py:285
-                    o_n[base + v] = xo * expf(-f);
-                }
-            }
-        }
+#ifndef N4_DEVICE_PASS
+        ReconThread T;
+        recon_thread<kBlock>(V, t, vt, sl.ny < R ? sl.ny : R, T);
+#endif
+        recon_rows(V, S.B, Cz, ((size_t)x * Y + y0) * Z, ny, rp.low_f, T, y0 == sl.y0);
         BLOCK_END
-        BLOCK_SYNC();
+        if (y0 + R < yend) BLOCK_SYNC();
     }
 }
 
@@ -2594,8 +2707,14 @@ size_t lds_eval(const VolDesc& v, int level, int prec) {
 
 size_t lds_recon(const VolDesc& v) {
     const LevelDesc& L = v.lev[v.nlevels - 1];
-    return carve_recon(nullptr, v.F[2], recon_chunk_rows(v.recon_rows, L.C[2]), v.recon_rows, L.C[1], L.C[2],
-                       nullptr);
+    return carve_recon(nullptr, recon_chunk_rows(v.recon_rows, L.C[2]), v.recon_rows, L.C[1], L.C[2], nullptr);
+}
+
+size_t lds_recon_limit(const VolDesc& v) {
+    const LevelDesc& L = v.lev[v.nlevels - 1];
+    const size_t Cy = L.C[1], Cz = L.C[2], Z = v.F[2], Yt = v.recon_rows;
+    const size_t R = std::min<size_t>(Yt, std::max<size_t>(1, kReconChunkFloats / Cz));
+    return align16(4 * Cy * Cz) + align16(4 * R * Cz) + align16(16 * Z) + align16(4 * Z) + align16(16 * Yt) + align16(4 * Yt);
 }
 
 int mfma_tiles(int c) { return cp_tiles(c); }
