@@ -406,18 +406,23 @@ __device__ inline int res_batch_len(CtxP C, int ub, int u1) {
 
 // fit_input of one voxel with the paired E table (same operations: the
 // difference of neighbouring entries is formed once per bin, and from the
-// last bin on the entry itself comes back as fma(0, ., E)).
-__device__ inline float res_input(bool den, bool m, float xv, bool degenerate, const Remap& R, const N4_LDS float* Ed) {
-    if (den) return m ? 1.0f : 0.0f;
+// last bin on the entry itself comes back as fma(0, ., E)).  on: all ones
+// where the voxel counts, else 0; as a bit mask it keeps the table reads of
+// all voxels in flight (a select becomes a branch around each read, with a
+// wait of its own; FP32, 256 x 256 x 160: 2.17 against 2.19 ms).
+template <bool DEN>
+__device__ inline float res_input(int on, float xv, const Remap& R, const N4_LDS float* Ed) {
+    if constexpr (DEN) return __int_as_float(on & __float_as_int(1.0f));
     float c = (xv - R.bmin) * R.islope;
     c = fminf(fmaxf(c, 0.0f), (float)R.nb);
     const int idx = (int)c;
     const float fr = c - (float)idx;
     typedef float f2 __attribute__((ext_vector_type(2)));
     const f2 e = *reinterpret_cast<const N4_LDS f2*>(Ed + 2 * idx);
-    const float sh = fmaf(e[1], fr, e[0]);
-    return m && !degenerate ? xv - sh : 0.0f;
+    return __int_as_float(on & __float_as_int(xv - fmaf(e[1], fr, e[0])));
 }
+// Bit j of a quad's mask byte as all ones or 0.
+__device__ inline int res_on(uint32_t m, int j) { return (int)(m << (31 - j)) >> 31; }
 
 // A pair of floats as BF16, round to nearest even, low half first.
 __device__ inline uint32_t res_pk(float a, float b) {
@@ -430,10 +435,10 @@ __device__ inline uint32_t res_pk(float a, float b) {
 // unit's voxels.  Row 4 g4 + i of the result is a row of voxels in the tile
 // order, column lane % 16 a control point along z.  pz: the lane's row of
 // the factor table.
-template <int PREC>
+template <int PREC, bool DEN>
 __device__ inline f32x4 res_fit_unit(const float* xq, const uint8_t* mq, const float* cq, const N4_LDS float* Ed,
                                      const N4_LDS unsigned char* pz, const N4_LDS unsigned char* pzl, int tile, int nt,
-                                     int zlo, bool den, bool degenerate, const Remap& rm) {
+                                     int zlo, uint32_t live, const Remap& rm) {
     const int lane = (int)threadIdx.x & 63, r16 = lane & 15, g4 = lane >> 4;
     f32x4 t1 = f32x4{0, 0, 0, 0};
     if constexpr (PREC == 0) {
@@ -445,19 +450,23 @@ __device__ inline f32x4 res_fit_unit(const float* xq, const uint8_t* mq, const f
             UNROLL for (int k = 0; k < kAhead; ++k) {
                 const bool ok = tb + k < nt;
                 const size_t q = q0 + (size_t)(ok ? tb + k : tb) * 64;
-                ms[k] = ok ? gp(mq)[q] : 0u;
+                ms[k] = gp(mq)[q] & (ok ? live : 0u);
                 xs[k] = load_quad(xq + 4 * q);
                 if (cq) cs[k] = load_quad(cq + 4 * q);
             }
             const N4_LDS float* b = reinterpret_cast<const N4_LDS float*>(pz) + (zlo >> 2) + 4 * tb;
+            float g[kAhead][4], f[kAhead][4];
+            UNROLL for (int k = 0; k < kAhead; ++k) UNROLL for (int j = 0; j < 4; ++j) {
+                g[k][j] = res_input<DEN>(res_on(ms[k], j), xs[k].v[j], rm, Ed);
+                f[k][j] = b[4 * k + j];
+            }
+            if (cq)
+                UNROLL for (int k = 0; k < kAhead; ++k) UNROLL for (int j = 0; j < 4; ++j)
+                    if ((ms[k] >> j) & 1u) g[k][j] *= cs[k].v[j];
+            // (tiles past the unit's end: zeros, which leave the chain as it is)
             UNROLL for (int k = 0; k < kAhead; ++k) {
                 if (tb + k >= nt) break;
-                UNROLL for (int j = 0; j < 4; ++j) {
-                    const bool m = (ms[k] >> j) & 1u;
-                    float g = res_input(den, m, xs[k].v[j], degenerate, rm, Ed);
-                    if (cq && m) g *= cs[k].v[j];
-                    t1 = mma_f32(g, b[4 * k + j], t1);
-                }
+                UNROLL for (int j = 0; j < 4; ++j) t1 = mma_f32(g[k][j], f[k][j], t1);
             }
         }
     } else {
@@ -470,16 +479,21 @@ __device__ inline f32x4 res_fit_unit(const float* xq, const uint8_t* mq, const f
                 const int a = ((32 * (T + (k >> 1)) + 8 * g4 - zlo) >> 2) + (k & 1);
                 const bool ok = a >= 0 && a < 4 * nt;
                 const size_t q = (size_t)tile * 64 + (ok ? 16 * a : 0) + r16;
-                ms[k] = ok ? gp(mq)[q] : 0u;
+                ms[k] = gp(mq)[q] & (ok ? live : 0u);
                 xs[k] = load_quad(xq + 4 * q);
             }
+            // (a branch per voxel here: its waits, one quad at a time, cost
+            // less than all sixteen table reads at once -- 64-volume batch
+            // 6.74 against 6.93 ms)
+            auto in = [&](int k, int j) {
+                return (ms[k] >> j) & 1u ? res_input<DEN>(-1, xs[k].v[j], rm, Ed) : 0.0f;
+            };
             UNROLL for (int k = 0; k < 4; k += 2) {
                 if (T + (k >> 1) >= T1) break;
                 uint32_t h4[4], l4[4];
                 UNROLL for (int p = 0; p < 4; ++p) {
                     const int kk = k + (p >> 1), j = 2 * (p & 1);
-                    const float g0 = res_input(den, (ms[kk] >> j) & 1u, xs[kk].v[j], degenerate, rm, Ed);
-                    const float g1 = res_input(den, (ms[kk] >> (j + 1)) & 1u, xs[kk].v[j + 1], degenerate, rm, Ed);
+                    const float g0 = in(kk, j), g1 = in(kk, j + 1);
                     const uint32_t h = res_pk(g0, g1);
                     h4[p] = h;
                     if constexpr (PREC == 2)
@@ -500,18 +514,12 @@ __device__ inline f32x4 res_fit_unit(const float* xq, const uint8_t* mq, const f
     return t1;
 }
 
-__device__ __attribute__((noinline)) unsigned long long res_fixed_wide(double v) {
-    return (unsigned long long)(long long)rint(v);
-}
-
-// rint(v) as a 64-bit integer: read from the low bits of v + 1.5 2^52 while
-// that is exact.
+// rint(v) as a 64-bit integer, read from the low bits of v + 1.5 2^52; exact
+// for |v| < kResFixedMax.
+constexpr double kResFixedMax = 2251799813685248.0;  // 2^51
 __device__ inline unsigned long long res_fixed(double v) {
-    if (fabs(v) < 2251799813685248.0) {  // 2^51
-        constexpr double kMagic = 6755399441055744.0;
-        return (unsigned long long)(__double_as_longlong(v + kMagic) - __double_as_longlong(kMagic));
-    }
-    return res_fixed_wide(v);
+    constexpr double kMagic = 6755399441055744.0;
+    return (unsigned long long)(__double_as_longlong(v + kMagic) - __double_as_longlong(kMagic));
 }
 
 // Fit of the workgroup's chunks, per batch of whole strips: T1 of every unit
@@ -522,13 +530,14 @@ __device__ inline unsigned long long res_fixed(double v) {
 // atomic per control point into the numerator copy of the chunk.  (Summing
 // the strips per control point instead, each thread walking the batch's
 // strips, took two thirds of the fit on a 64-volume batch.)
-template <int PREC>
-N4_PHASE void res_fit(LdsP smem, int kf, int degenerate_, double bmin, double slope) {
+template <int PREC, bool DEN>
+N4_PHASE void res_fit(LdsP smem, int degenerate_, double bmin, double slope) {
     const LdsP base = res_base(smem);
     const CtxP C = res_ctx(base);
     const int t = (int)threadIdx.x, wv = uni(t >> 6), lane = t & 63, r16 = lane & 15, g4 = lane >> 4;
     const int Cy = uni(C->Cy), Cz = uni(C->Cz), CyCz = Cy * Cz;
-    const bool degenerate = uni(degenerate_) != 0, den = uni(kf) == 2, single = uni(C->single) != 0;
+    const bool single = uni(C->single) != 0;
+    const uint32_t live = uni(degenerate_) != 0 ? 0u : 0xffu;  // (degenerate: no residual anywhere)
     const float* xq = uni(C->xq);
     const uint8_t* mq = uni(C->mq);
     const float* cq = uni(C->cq);
@@ -553,12 +562,12 @@ N4_PHASE void res_fit(LdsP smem, int kf, int degenerate_, double bmin, double sl
             n = single ? u1 - ub : res_batch_len(C, ub, u1);
             if (!single) {
                 __syncthreads();
-                res_load_batch(smem, ub, n, kf);
+                res_load_batch(smem, ub, n, DEN ? 2 : 1);
                 __syncthreads();
             }
             for (int i = wv; i < n; i += kResWaves) {
-                const f32x4 a = res_fit_unit<PREC>(xq, mq, cq, Ed, pz, pzl, uni(lu[i].tile), uni(lu[i].nt),
-                                                   uni(lu[i].zlo), den, degenerate, rm);
+                const f32x4 a = res_fit_unit<PREC, DEN>(xq, mq, cq, Ed, pz, pzl, uni(lu[i].tile), uni(lu[i].nt),
+                                                        uni(lu[i].zlo), live, rm);
                 *reinterpret_cast<N4_LDS f32x4*>(slot + i * 256 + 4 * lane) = a;
             }
             __syncthreads();
@@ -587,14 +596,26 @@ N4_PHASE void res_fit(LdsP smem, int kf, int degenerate_, double bmin, double sl
                 // wave order), into the strip's four planes
                 const N4_LDS ResLUnit& U = lu[s0];
                 N4_LDS unsigned long long* dp = acc + (uni(U.b) - pa) * CyCz + 4 * g4 * Cz + r16;
-                double f[4];
+                double f[4], t2[4], big = 0.0;
                 UNROLL for (int p = 0; p < 4; ++p) f[p] = (double)U.f[p];
                 UNROLL for (int i = 0; i < 4; ++i) {
-                    float t2 = v[0][i];
-                    if constexpr (PREC != 0) t2 = ((t2 + v[1][i]) + v[2][i]) + v[3][i];
-                    if (4 * g4 + i < Cy && r16 < Cz)
+                    float x = v[0][i];
+                    if constexpr (PREC != 0) x = ((x + v[1][i]) + v[2][i]) + v[3][i];
+                    t2[i] = (double)x;
+                    big = fmax(big, fabs(t2[i]));
+                }
+                // (the factors are at most 1; NaN counts as wide)
+                const bool wide = __ballot(!(big * kNumScale < kResFixedMax)) != 0;
+                UNROLL for (int i = 0; i < 4; ++i) {
+                    if (4 * g4 + i >= Cy || r16 >= Cz) continue;
+                    if (!wide) {
                         UNROLL for (int p = 0; p < 4; ++p)
-                            lds_add_u64(dp + p * CyCz + i * Cz, res_fixed(f[p] * (double)t2 * kNumScale));
+                            lds_add_u64(dp + p * CyCz + i * Cz, res_fixed(f[p] * t2[i] * kNumScale));
+                    } else {
+                        for (int p = 0; p < 4; ++p)
+                            lds_add_u64(dp + p * CyCz + i * Cz,
+                                        (unsigned long long)(long long)rint((double)U.f[p] * t2[i] * kNumScale));
+                    }
                 }
             }
             __syncthreads();
@@ -793,7 +814,8 @@ N4_PHASE void res_hist(LdsP smem, double mn, double slope) {
     const Bins B = make_bins(mn, slope, nb);
     for (int Ta = T0; Ta < T1; Ta += kResHistTiles) {
         const int Te = T1 - Ta > kResHistTiles ? Ta + kResHistTiles : T1;
-        for (int i = t; i < nb * hc; i += kResThreads) h[i] = 0ull;
+        typedef unsigned long long u2 __attribute__((ext_vector_type(2)));
+        for (int i = t; i < nb * hc / 2; i += kResThreads) reinterpret_cast<N4_LDS u2*>(h)[i] = u2{0ull, 0ull};
         __syncthreads();
         N4_LDS unsigned long long* hl = h + (t & (hc - 1));
         const int hs = uni(__ffs(hc) - 1);
@@ -822,8 +844,8 @@ N4_PHASE void res_hist(LdsP smem, double mn, double slope) {
             const int i = i0 + (t >> 2), part = t & 3, per = hc >> 2;
             unsigned long long cnt = 0, sq = 0;
             if (i < nb)
-                for (int k = 0; k < per; ++k) {
-                    const unsigned long long v = h[(size_t)i * hc + part * per + k];
+                for (int k = 0; k < per; ++k) {  // (rotated by the bin: bins are a multiple of the banks apart)
+                    const unsigned long long v = h[(size_t)i * hc + part * per + ((k + i) & (per - 1))];
                     cnt += v >> 48;
                     sq += v & ((1ull << 48) - 1);
                 }
@@ -1181,7 +1203,7 @@ N4_PHASE bool res_enter_level(const VolDesc* Vp, LdsP smem, int level_, uint32_t
     res_tables<PREC>(smem, 2);
     if (single) res_load_batch(smem, U0, U1 - U0, 2);
     if (!res_barrier(team, m, gen, smem)) return false;
-    res_fit<PREC>(smem, 2, 0, 0.0, 1.0);
+    res_fit<PREC, true>(smem, 0, 0.0, 1.0);
     if (!res_barrier(team, m, gen + 1, smem)) return false;
     res_clear_numerator(base, true);
     res_tables<PREC>(smem, 1);
@@ -1356,7 +1378,7 @@ __device__ bool res_volume(const VolDesc& V, const RunParams& rp, int rank, int 
         pt.mark(kPhWait);
         if (!degenerate) res_wiener(&V, smem, mn, slope);
         pt.mark(kPhWiener);
-        res_fit<PREC>(smem, 1, degenerate, mn, slope);
+        res_fit<PREC, false>(smem, degenerate, mn, slope);
         pt.mark(kPhFit);
         if (!res_barrier(team, m, gen++, smem)) return false;
         pt.mark(kPhWait);
