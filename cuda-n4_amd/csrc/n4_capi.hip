@@ -851,6 +851,7 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
         D.prep_rows = I.prep_rows;
         D.prep_tiles_x = I.prep_tiles_x;
         D.recon_rows = I.recon_rows;
+        D.recon_tiles_x = I.recon_tiles_x;
         D.wtile_rows = I.wtile_rows;
         D.wtiles_x = I.wtiles_x;
         D.hist_copies = hcopies(v);
@@ -902,7 +903,9 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
                 for (int y0 = 0; y0 < in[v].F[1]; y0 += I.recon_rows)
                     fs[ifs++] = Slab{v, x, y0, std::min(I.recon_rows, in[v].F[1] - y0)};
         const int prec = P->rp.prec;
-        if (res) P->lds_resident = std::max(P->lds_resident, lds_resident(D, nb, P->rp.P, prec));
+        if (res)  // (the kernel also reconstructs tiles, in the same LDS behind the broadcast words)
+            P->lds_resident =
+                std::max(P->lds_resident, std::max(lds_resident(D, nb, P->rp.P, prec), lds_recon(D) + kResBcBytes));
         for (int l = 0; l < L; ++l) {
             P->lds_fit_max[l] = std::max(P->lds_fit_max[l], lds_fit(nb, D, l, prec));
             P->lds_eval_max[l] = std::max(P->lds_eval_max[l], lds_eval(D, l, prec));
@@ -1618,7 +1621,7 @@ static n4_status run_batch(n4_handle* h, const std::vector<VolIn>& in_user, cons
     if (resident) {
         // one launch runs every volume's level/iteration loop
         void* gs = stream;
-        GLAUNCH(N4_K_TEAMS, launch_resident(dd, (const int32_t*)(P.base + P.off_slots), P.n_slots,
+        GLAUNCH(N4_K_TEAMS, launch_resident(dd, nv, (const int32_t*)(P.base + P.off_slots), P.n_slots,
                                             std::min(P.n_slots, res.cus),
                                             (uint32_t*)(P.base + P.off_team + 64 * (size_t)nv), rp, P.lds_resident, gs));
         GLAUNCH(N4_K_RECON, launch_recon(dd, fsl, P.n_fslab, P.nlevels - 1, rp, P.lds_recon, gs));

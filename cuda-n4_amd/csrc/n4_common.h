@@ -85,9 +85,18 @@ struct alignas(16) ResUnit {
     int32_t nt;
 };
 
+constexpr uint32_t kResBcBytes = 64;  // broadcast words at the start of the resident kernel's LDS
 constexpr int kResNumCopies = 8;   // most numerator copies of a resident plan
 constexpr int kResMaxDim = 1024;   // most working rows / z positions it covers
 constexpr int kResMaxSlabs = 2048; // most working slabs
+
+// Words of a volume's team area (64 bytes, zero before the launch): joined
+// members and closed flag, team size, barrier counter, abort flag, the
+// working and full foreground counts (64-bit), lattice ready, reconstruction
+// tiles taken.
+enum ResWord : int {
+    kRwJoin = 0, kRwSize = 1, kRwBarrier = 2, kRwAbort = 3, kRwMaskWork = 4, kRwMaskFull = 6, kRwReady = 8, kRwTiles = 9
+};
 
 // A volume's buffers on the resident path (nchunk 0: not a resident plan).
 struct ResDesc {
@@ -150,6 +159,7 @@ struct VolDesc {
     int32_t prep_rows;         // working rows per prep tile
     int32_t prep_tiles_x;      // prep tiles per working slab
     int32_t recon_rows;        // full-resolution rows per reconstruction tile
+    int32_t recon_tiles_x;     // such tiles per full-resolution slab
     int32_t wtile_rows;        // working rows per tile of the step kernels
     int32_t wtiles_x;          // such tiles per working slab (spart has W0*wtiles_x entries)
     int32_t hist_copies;       // tile t adds its histogram into copy t % hist_copies

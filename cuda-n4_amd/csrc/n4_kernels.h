@@ -85,11 +85,12 @@ int launch_persist(const VolDesc* vols, const Slab* slabs, const PWork* work, in
 // Resident path (n4_resident.h): every volume's level/iteration loop in one
 // launch of nwg workgroups (one per compute unit); slots[k] names the volume
 // whose team the k-th workgroup to ask joins (a volume's nchunk slots are
-// consecutive), *ticket (zero) counts the slots taken.
+// consecutive); run (two words, zero): slots taken, volumes ready.  Some of
+// the reconstruction may be done by it; launch_recon does the rest.
 size_t lds_resident(const VolDesc& v, int nbins, int P, int prec);
 int resident_limits(int* cus, size_t* lds);
-int launch_resident(const VolDesc* vols, const int32_t* slots, int nslots, int nwg, uint32_t* ticket, RunParams rp,
-                    size_t lds, void* stream);
+int launch_resident(const VolDesc* vols, int nvol, const int32_t* slots, int nslots, int nwg, uint32_t* run,
+                    RunParams rp, size_t lds, void* stream);
 
 // Flat (1-D) stage helpers used by the stage entry points.  A flat array of
 // n voxels is cut into slabs of kChunkVox voxels; each slab writes

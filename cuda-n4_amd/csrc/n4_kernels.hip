@@ -44,11 +44,13 @@
 
 #ifdef N4_DEVICE_PASS
 #define BLOCK_FOR(t) { const int t = (int)threadIdx.x; (void)t;
+#define BLOCK_FOR_N(t, n) BLOCK_FOR(t)
 #define BLOCK_END }
 #define BLOCK_SYNC() __syncthreads()
 #define UNROLL _Pragma("unroll")
 #else
 #define BLOCK_FOR(t) for (int t = 0; t < kBlock; ++t) {
+#define BLOCK_FOR_N(t, n) for (int t = 0; t < n; ++t) {
 #define BLOCK_END }
 #define BLOCK_SYNC() do { } while (0)
 #define UNROLL
@@ -1979,10 +1981,10 @@ HD void recon_rows(const VolDesc& V, const N4_LDS float* B, int Cz, size_t v0, i
     }
 }
 
-HD void body_recon(const VolDesc* vols, const Slab* slabs, int level, RunParams rp, int bid,
-                   N4_LDS unsigned char* smem) {
-    const Slab sl = slabs[bid];
-    const VolDesc& V = vols[sl.vol];
+// One tile, rows [yt, yt + nyt) of slab x, by a workgroup of NT threads.
+// AGENT: the lattice was written in the same launch.
+template <int NT, bool AGENT>
+HD void recon_tile(const VolDesc& V, int level, float low, int x, int yt, int nyt, N4_LDS unsigned char* smem) {
     const LevelDesc& LD = V.lev[level];
     const int Y = V.F[1], Z = V.F[2];
     const int Cy = LD.C[1], Cz = LD.C[2];
@@ -1990,54 +1992,67 @@ HD void body_recon(const VolDesc* vols, const Slab* slabs, int level, RunParams 
     const int R = recon_chunk_rows(V.recon_rows, Cz);
     ReconLds S;
     carve_recon(smem, R, V.recon_rows, Cy, Cz, &S);
-    const int x = sl.x;
     const F4 ex = V.fw[0][x];
     const int xb = V.fb[0][x];
     // set-up: x-contracted planes, the (tile) y factor table and the threads'
     // own columns and first image quads, from one round of global loads
-    const size_t vt = ((size_t)x * Y + sl.y0) * Z;
+    const size_t vt = ((size_t)x * Y + yt) * Z;
 #ifdef N4_DEVICE_PASS
     ReconThread T;
-    recon_thread<kBlock>(V, (int)threadIdx.x, vt, sl.ny < R ? sl.ny : R, T);
+    recon_thread<NT>(V, (int)threadIdx.x, vt, nyt < R ? nyt : R, T);
 #endif
-    BLOCK_FOR(t)
-    for (int pr = t; pr < CyCz; pr += kBlock) {
+    BLOCK_FOR_N(t, NT)
+    for (int pr = t; pr < CyCz; pr += NT) {
         float a = 0.0f;
-        for (int k = 0; k < 4; ++k) a += ex.v[k] * V.latf[(size_t)(xb + k) * CyCz + pr];
+        for (int k = 0; k < 4; ++k) {
+            const float* l = V.latf + (size_t)(xb + k) * CyCz + pr;
+            a += ex.v[k] * (AGENT ? ld_agent(l) : *l);
+        }
         S.A[pr] = a;
     }
-    for (int r = t; r < sl.ny; r += kBlock) {
-        const F4 e = V.fw[1][sl.y0 + r];
+    for (int r = t; r < nyt; r += NT) {
+        const F4 e = V.fw[1][yt + r];
         for (int k = 0; k < 4; ++k) S.yw[4 * r + k] = e.v[k];
-        S.yb[r] = V.fb[1][sl.y0 + r];
+        S.yb[r] = V.fb[1][yt + r];
     }
-    for (int r = t; r < R; r += kBlock) S.B[r * (Cz + 1) + Cz] = 0.0f;
+    for (int r = t; r < R; r += NT) S.B[r * (Cz + 1) + Cz] = 0.0f;
     BLOCK_END
     BLOCK_SYNC();
-    const int yend = sl.y0 + sl.ny;
-    for (int y0 = sl.y0; y0 < yend; y0 += R) {
-        const int ny = (yend - y0 < R) ? yend - y0 : R;
-        BLOCK_FOR(t)
-        for (int pr = t; pr < ny * Cz; pr += kBlock) {
+    for (int y0 = 0; y0 < nyt; y0 += R) {
+        const int ny = (nyt - y0 < R) ? nyt - y0 : R;
+        BLOCK_FOR_N(t, NT)
+        for (int pr = t; pr < ny * Cz; pr += NT) {
             const int r = (int)fdiv((uint32_t)pr, LD.mCz), c = pr - r * Cz;
-            const int tr = y0 - sl.y0 + r;  // tile row
-            const N4_LDS float* yw = S.yw + 4 * tr;
-            const int b0 = S.yb[tr];
+            const N4_LDS float* yw = S.yw + 4 * (y0 + r);
+            const int b0 = S.yb[y0 + r];
             float b = 0.0f;
             for (int k = 0; k < 4; ++k) b += yw[k] * S.A[(b0 + k) * Cz + c];
             S.B[r * (Cz + 1) + c] = b;
         }
         BLOCK_END
         BLOCK_SYNC();
-        BLOCK_FOR(t)
+        BLOCK_FOR_N(t, NT)
 #ifndef N4_DEVICE_PASS
         ReconThread T;
-        recon_thread<kBlock>(V, t, vt, sl.ny < R ? sl.ny : R, T);
+        recon_thread<NT>(V, t, vt, nyt < R ? nyt : R, T);
 #endif
-        recon_rows(V, S.B, Cz, ((size_t)x * Y + y0) * Z, ny, rp.low_f, T, y0 == sl.y0);
+        recon_rows(V, S.B, Cz, vt + (size_t)y0 * Z, ny, low, T, y0 == 0);
         BLOCK_END
-        if (y0 + R < yend) BLOCK_SYNC();
+        if (y0 + R < nyt) BLOCK_SYNC();
     }
+}
+
+HD void body_recon(const VolDesc* vols, const Slab* slabs, int level, RunParams rp, int bid,
+                   N4_LDS unsigned char* smem) {
+    const Slab sl = slabs[bid];
+    const VolDesc& V = vols[sl.vol];
+    // (tiles that the resident kernel has reconstructed while other volumes
+    // were still iterating)
+    if (V.res.nchunk > 0 && V.res.team) {
+        const uint32_t done = V.res.team[kRwTiles];
+        if ((uint32_t)(sl.x * V.recon_tiles_x + sl.y0 / V.recon_rows) < done) return;
+    }
+    recon_tile<kBlock, false>(V, level, rp.low_f, sl.x, sl.y0, sl.ny, smem);
 }
 
 // ------------------------------------------------------------------ flat --
@@ -2875,25 +2890,38 @@ int launch_persist(const VolDesc* vols, const Slab* slabs, const PWork* work, in
 }
 
 // Resident path: workgroups take the slots in order, each with the volume
-// whose team it joins, until none is left.
+// whose team it joins, until none is left.  A workgroup without a slot then
+// reconstructs tiles of the volumes that are ready (its own first) while
+// others still iterate -- their chains leave the memory idle -- but waits
+// for none: what is left when the last volume is ready belongs to the
+// reconstruction launch, which spreads it over the whole device (64-volume
+// BF16 batch 7.18 -> 6.62 ms, 12 mixed volumes 3.39 -> 3.24 ms).
+// run: [0] slots taken, [1] volumes whose lattice is final.
 template <int PREC>
-__global__ __launch_bounds__(kResThreads) void k_resident(const VolDesc* __restrict__ vols,
+__global__ __launch_bounds__(kResThreads) void k_resident(const VolDesc* __restrict__ vols, int nvol,
                                                           const int32_t* __restrict__ slots, int nslots,
-                                                          uint32_t* ticket, RunParams rp) {
+                                                          uint32_t* run, RunParams rp) {
     HIP_DYNAMIC_SHARED(double, smem_);
     const LdsP smem = SMEM();
     N4_LDS int* bc = reinterpret_cast<N4_LDS int*>(smem);
+    int last = 0;
     for (;;) {
         __syncthreads();
         if (threadIdx.x == 0)
-            bc[3] = (int)__hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            bc[3] = (int)__hip_atomic_fetch_add(run, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __syncthreads();
         const int k = uni(bc[3]);
-        if (k >= nslots) return;
-        const VolDesc& V = vols[slots[k]];
+        if (k >= nslots) break;
+        last = slots[k];
+        const VolDesc& V = vols[last];
         const int rank = uni(res_join(V.res.team, V.res.nchunk, smem));
         if (rank == -1) continue;  // its team runs without this workgroup
-        if (rank < 0 || !res_volume<PREC>(V, rp, rank, uni(bc[2]), smem)) return;
+        if (rank < 0 || !res_volume<PREC>(V, rp, rank, uni(bc[2]), nvol > 1 ? run + 1 : nullptr, smem)) return;
+    }
+    if (nvol == 1) return;
+    for (int i = 0; i < nvol; ++i) {
+        const int v = last + i < nvol ? last + i : last + i - nvol;
+        res_recon(vols + v, nvol, run, rp.nlevels - 1, rp.low_f, smem);
     }
 }
 
@@ -2910,17 +2938,17 @@ int resident_limits(int* cus, size_t* lds) {
     return (int)e;
 }
 
-int launch_resident(const VolDesc* vols, const int32_t* slots, int nslots, int nwg, uint32_t* ticket, RunParams rp,
-                    size_t lds, void* stream) {
+int launch_resident(const VolDesc* vols, int nvol, const int32_t* slots, int nslots, int nwg, uint32_t* run,
+                    RunParams rp, size_t lds, void* stream) {
     if (nwg <= 0) return 0;
     const dim3 g(nwg), b(kResThreads);
     const hipStream_t s = (hipStream_t)stream;
     if (rp.prec == 1)
-        hipLaunchKernelGGL(k_resident<1>, g, b, lds, s, vols, slots, nslots, ticket, rp);
+        hipLaunchKernelGGL(k_resident<1>, g, b, lds, s, vols, nvol, slots, nslots, run, rp);
     else if (rp.prec == 2)
-        hipLaunchKernelGGL(k_resident<2>, g, b, lds, s, vols, slots, nslots, ticket, rp);
+        hipLaunchKernelGGL(k_resident<2>, g, b, lds, s, vols, nvol, slots, nslots, run, rp);
     else
-        hipLaunchKernelGGL(k_resident<0>, g, b, lds, s, vols, slots, nslots, ticket, rp);
+        hipLaunchKernelGGL(k_resident<0>, g, b, lds, s, vols, nvol, slots, nslots, run, rp);
     return last_launch_status();
 }
 

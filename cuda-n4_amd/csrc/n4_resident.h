@@ -58,9 +58,6 @@ constexpr uint64_t kResJoinTicks = 20000;  // 100 MHz clock: 200 us
 
 #define N4_PHASE __device__ __attribute__((noinline))
 
-// Words of a volume's team area (64 bytes, zeroed before the launch).
-enum ResWord : int { kRwJoin = 0, kRwSize = 1, kRwBarrier = 2, kRwAbort = 3, kRwMaskWork = 4, kRwMaskFull = 6 };
-
 // One unit of the current batch in LDS, with its slab's x factors.
 struct alignas(16) ResLUnit {
     int32_t x, y0, zlo, tile;
@@ -141,7 +138,6 @@ __device__ inline T* uni(T* p) {
 // LDS base and context of a phase function (its arguments arrive in vector
 // registers).
 __device__ inline LdsP res_base(LdsP smem) { return (LdsP)(uintptr_t)uni((uint32_t)(uintptr_t)smem); }
-constexpr uint32_t kResBcBytes = 64;  // broadcast words, then the context
 __device__ inline CtxP res_ctx(LdsP base) { return reinterpret_cast<CtxP>(base + kResBcBytes); }
 template <class T>
 __device__ inline N4_LDS T* lds_at(LdsP base, uint32_t off) {
@@ -1212,10 +1208,38 @@ N4_PHASE bool res_enter_level(const VolDesc* Vp, LdsP smem, int level_, uint32_t
     return true;
 }
 
+// Reconstruction tiles of one volume, if its lattice is ready, while other
+// volumes still iterate (run[1] < nvol).
+N4_PHASE void res_recon(const VolDesc* Vp, int nvol_, uint32_t* run_, int level, float low, LdsP smem) {
+    const VolDesc& V = *uni(Vp);
+    const LdsP base = res_base(smem);
+    const int nvol = uni(nvol_);
+    uint32_t* run = uni(run_);
+    uint32_t* team = V.res.team;
+    N4_LDS int* bc = reinterpret_cast<N4_LDS int*>(base);
+    const int tx = V.recon_tiles_x, rows = V.recon_rows, Y = V.F[1], total = V.F[0] * tx;
+    for (;;) {
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            int tile = -1;
+            if (ld_agent(run + 1) < (uint32_t)nvol && ld_agent(team + kRwReady) != 0 &&
+                ld_agent(team + kRwTiles) < (uint32_t)total)
+                tile = (int)__hip_atomic_fetch_add(team + kRwTiles, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            bc[4] = tile;
+        }
+        __syncthreads();
+        const int tile = uni(bc[4]);
+        if (tile < 0 || tile >= total) return;
+        const int x = tile / tx, y0 = (tile - x * tx) * rows;
+        recon_tile<kResThreads, true>(V, uni(level), low, x, y0, Y - y0 < rows ? Y - y0 : rows, base + kResBcBytes);
+    }
+}
+
 // One volume, from its set-up to its final lattice, as member `rank` of a
-// team of m; false if the team gave up.
+// team of m; false if the team gave up.  ready: count of finished volumes,
+// null where no other volume is there to wait for.
 template <int PREC>
-__device__ bool res_volume(const VolDesc& V, const RunParams& rp, int rank, int m, LdsP smem) {
+__device__ bool res_volume(const VolDesc& V, const RunParams& rp, int rank, int m, uint32_t* ready, LdsP smem) {
     const int t = (int)threadIdx.x, wv = uni(t >> 6), lane = t & 63;
     uint32_t* team = V.res.team;
     const int nb = rp.nbins, nch = V.res.nchunk;
@@ -1341,7 +1365,7 @@ __device__ bool res_volume(const VolDesc& V, const RunParams& rp, int rank, int 
             const int o0 = uni(C->o0), o1 = uni(C->o1);
             for (int l = o0 + t; l < o1; l += kResThreads) {
                 const float f = (float)ld_agent(fin + l);
-                V.latf[l] = f;
+                st_agent(V.latf + l, f);
                 if (rec) rec[l] = f;
                 if (V.out_lattice) V.out_lattice[l] = f;
             }
@@ -1357,6 +1381,11 @@ __device__ bool res_volume(const VolDesc& V, const RunParams& rp, int rank, int 
             }
             if (pt.on && t == 0)
                 for (int k = 0; k < kPhases; ++k) V.tphase[k] = tick[k];
+            if (ready && !res_barrier(team, m, gen, smem)) return false;
+            if (ready && leader && t == 0) {  // the lattice is complete: its reconstruction may start
+                st_agent(team + kRwReady, 1u);
+                __hip_atomic_fetch_add(ready, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
             return true;
         }
         pt.mark(kPhReduce);
