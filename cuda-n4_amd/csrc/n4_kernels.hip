@@ -1005,6 +1005,19 @@ HD void dft_small(D2 (&v)[R], double sg) {
     UNROLL for (int i = 0; i < R; ++i) v[i] = u[i];
 }
 
+// Index of point i in the LDS transform buffers; PAD: one element of padding
+// per eight.  The first pass writes, and the second reads its twiddles, with
+// a stride of eight 16-byte elements, which without it all lie in the same
+// four banks.
+template <bool PAD>
+HD constexpr int fft_at(int i) {
+    return PAD ? i + (i >> 3) : i;
+}
+HD constexpr int fft_len(int P, bool pad) { return pad ? P + (P >> 3) : P; }
+// 1024 points fill a workgroup's 64 KB without it.
+HD constexpr bool fft_pad(int P) { return P <= 512; }
+HD constexpr size_t wiener_lds(int P) { return (size_t)(P + 3 * fft_len(P, fft_pad(P))) * sizeof(D2); }
+
 // One Stockham pass of radix R over P points (span Ns): butterfly j takes
 // a[j + r*P/R], twiddles them by exp(-+2 pi i r k / (Ns R)) (k = j mod Ns)
 // and writes b[(j - k) R + k + r Ns].  Thread t of the block takes
@@ -1012,7 +1025,7 @@ HD void dft_small(D2 (&v)[R], double sg) {
 // constants: with every pass unrolled and its index arithmetic folded, a
 // 512-point transform takes 1.3 us on MI355X against 2.3 us for the same
 // code with a run-time size and direction.
-template <int R, int P, bool INV, int NT>
+template <int R, int P, bool INV, int NT, bool PAD>
 HD void block_fft_pass(const N4_LDS D2* a, N4_LDS D2* b, const N4_LDS D2* tw, int Ns) {
     constexpr int nbf = P / R;
     const int tstep = P / (Ns * R);
@@ -1021,17 +1034,17 @@ HD void block_fft_pass(const N4_LDS D2* a, N4_LDS D2* b, const N4_LDS D2* tw, in
     for (int j = t; j < nbf; j += NT) {
         const int k = j & (Ns - 1);
         D2 v[R];
-        UNROLL for (int r = 0; r < R; ++r) v[r] = a[j + r * nbf];
+        UNROLL for (int r = 0; r < R; ++r) v[r] = a[fft_at<PAD>(j + r * nbf)];
         if (Ns > 1) {
             UNROLL for (int r = 1; r < R; ++r) {
-                D2 w = tw[r * k * tstep];
+                D2 w = tw[fft_at<PAD>(r * k * tstep)];
                 if (INV) w.y = -w.y;
                 v[r] = cmul(v[r], w);
             }
         }
         dft_small<R>(v, sg);
         const int o = (j - k) * R + k;
-        UNROLL for (int r = 0; r < R; ++r) b[o + r * Ns] = v[r];
+        UNROLL for (int r = 0; r < R; ++r) b[fft_at<PAD>(o + r * Ns)] = v[r];
     }
     BLOCK_END
 }
@@ -1042,17 +1055,17 @@ HD void block_fft_pass(const N4_LDS D2* a, N4_LDS D2* b, const N4_LDS D2* tw, in
 // free).  (Radix 2 and 4 over all 256 threads, and radix 8 in one
 // wavefront with wave-level ordering, measured equal or slower on MI355X.)
 constexpr int kFftRadix = 8;
-template <int P, bool INV, int NT>
+template <int P, bool INV, int NT, bool PAD>
 HD N4_LDS D2* block_fft(N4_LDS D2* a, N4_LDS D2* b, const N4_LDS D2* tw) {
     UNROLL for (int Ns = 1; Ns < P;) {
         const int rem = P / Ns;
         const int R = rem >= kFftRadix ? kFftRadix : rem;
         if (R == 8)
-            block_fft_pass<8, P, INV, NT>(a, b, tw, Ns);
+            block_fft_pass<8, P, INV, NT, PAD>(a, b, tw, Ns);
         else if (R == 4)
-            block_fft_pass<4, P, INV, NT>(a, b, tw, Ns);
+            block_fft_pass<4, P, INV, NT, PAD>(a, b, tw, Ns);
         else
-            block_fft_pass<2, P, INV, NT>(a, b, tw, Ns);
+            block_fft_pass<2, P, INV, NT, PAD>(a, b, tw, Ns);
         BLOCK_SYNC();
         N4_LDS D2* tmp = a;
         a = b;
@@ -1071,13 +1084,15 @@ HD void wiener_table_p(const VolDesc& V, double bmin, double slope, const RunPar
                        N4_LDS float* Ef) {
     constexpr bool TEAM = WM == kWienerTeam;
     constexpr bool AGENT = WM != kWienerLocal;
+    // (the persistent kernel's LDS is sized without the padding)
+    constexpr bool PAD = fft_pad(P) && !(TEAM && NT == kBlock);
     constexpr int half = P / 2;
     const int off = rp.offset, nb = rp.nbins;
     Carve cv{smem, 0};
-    N4_LDS D2* z = cv.take<D2>(P);
-    N4_LDS D2* y = cv.take<D2>(P);
+    N4_LDS D2* z = cv.take<D2>(fft_len(P, PAD));
+    N4_LDS D2* y = cv.take<D2>(fft_len(P, PAD));
     N4_LDS D2* ff = cv.take<D2>(P);
-    N4_LDS D2* tw = cv.take<D2>(P);
+    N4_LDS D2* tw = cv.take<D2>(fft_len(P, PAD));
     const double scaledFWHM = rp.fwhm / slope;
     const double expF = 4.0 * log(2.0) / (scaledFWHM * scaledFWHM);
     const double scale = 2.0 * sqrt(log(2.0) / M_PI) / scaledFWHM;
@@ -1105,49 +1120,49 @@ HD void wiener_table_p(const VolDesc& V, double bmin, double slope, const RunPar
 
             Vj = (double)s * 0x1p-32;
         }
-        z[j] = D2{Vj, Fj};
-        tw[j] = rp.twiddle[j];
+        z[fft_at<PAD>(j)] = D2{Vj, Fj};
+        tw[fft_at<PAD>(j)] = rp.twiddle[j];
     }
     BLOCK_END
     BLOCK_SYNC();
     // the chain of transforms and pointwise steps, block-wide
-    N4_LDS D2* Z = block_fft<P, false, NT>(z, y, tw);
+    N4_LDS D2* Z = block_fft<P, false, NT, PAD>(z, y, tw);
     N4_LDS D2* U = (Z == z) ? y : z;
     // Split Vf and Ff, Gf = conj(Ff)/(conj(Ff)Ff + noise), Uf = Vf*Re(Gf)
     BLOCK_FOR(t)
     for (int k = t; k < P; k += NT) {
-        const D2 a = Z[k];
-        const D2 m = Z[(P - k) & (P - 1)];
+        const D2 a = Z[fft_at<PAD>(k)];
+        const D2 m = Z[fft_at<PAD>((P - k) & (P - 1))];
         const D2 Vf{0.5 * (a.x + m.x), 0.5 * (a.y - m.y)};
         const D2 Ff{0.5 * (a.y + m.y), -0.5 * (a.x - m.x)};
         ff[k] = Ff;
         const double g = Ff.x / ((Ff.x * Ff.x + Ff.y * Ff.y) + rp.noise);
-        U[k] = D2{Vf.x * g, Vf.y * g};
+        U[fft_at<PAD>(k)] = D2{Vf.x * g, Vf.y * g};
     }
     BLOCK_END
     BLOCK_SYNC();
-    N4_LDS D2* Ur = block_fft<P, true, NT>(U, Z, tw);
+    N4_LDS D2* Ur = block_fft<P, true, NT, PAD>(U, Z, tw);
     N4_LDS D2* Wb = (Ur == U) ? Z : U;
     const double invP = 1.0 / (double)P;
     BLOCK_FOR(t)
     for (int j = t; j < P; j += NT) {
-        double u = Ur[j].x * invP;
+        double u = Ur[fft_at<PAD>(j)].x * invP;
         if (u < 0.0) u = 0.0;
-        Wb[j] = D2{(bmin + (double)(j - off) * slope) * u, u};
+        Wb[fft_at<PAD>(j)] = D2{(bmin + (double)(j - off) * slope) * u, u};
     }
     BLOCK_END
     BLOCK_SYNC();
-    N4_LDS D2* Wf = block_fft<P, false, NT>(Wb, Ur, tw);
+    N4_LDS D2* Wf = block_fft<P, false, NT, PAD>(Wb, Ur, tw);
     N4_LDS D2* Wo = (Wf == Wb) ? Ur : Wb;
     BLOCK_FOR(t)
-    for (int k = t; k < P; k += NT) Wf[k] = cmul(Wf[k], ff[k]);
+    for (int k = t; k < P; k += NT) Wf[fft_at<PAD>(k)] = cmul(Wf[fft_at<PAD>(k)], ff[k]);
     BLOCK_END
     BLOCK_SYNC();
-    N4_LDS D2* R = block_fft<P, true, NT>(Wf, Wo, tw);
+    N4_LDS D2* R = block_fft<P, true, NT, PAD>(Wf, Wo, tw);
     BLOCK_FOR(t)
     for (int i = t; i < nb; i += NT) {
-        const double nu = R[off + i].x * invP;
-        const double de = R[off + i].y * invP;
+        const double nu = R[fft_at<PAD>(off + i)].x * invP;
+        const double de = R[fft_at<PAD>(off + i)].y * invP;
         const double e = (de != 0.0) ? nu / de : 0.0;
         if (TEAM)
             Ef[i] = (float)e;
@@ -2694,7 +2709,7 @@ size_t lds_level() { return align16(4 * kBlock * sizeof(double)); }
 size_t lds_hist(int nbins) {
     return std::max(align16(4 * kBlock * sizeof(double)), align16((size_t)kHistLanes * hist_stride(nbins) * sizeof(uint64_t)));
 }
-size_t lds_wiener(int P) { return align16(4 * (size_t)P * sizeof(D2)); }
+size_t lds_wiener(int P) { return align16(wiener_lds(P)); }
 size_t lds_lattice() { return align16(kBlock * sizeof(double)); }
 size_t lds_flat(int nbins) { return align16(4 * kBlock * sizeof(double)) + align16(nbins * sizeof(double)); }
 

@@ -183,7 +183,7 @@ HD size_t carve_res(const VolDesc& V, int nbins, int P, int prec, ResCtx* o) {
     c.lu = take(sizeof(ResLUnit) * V.res.nbatch);
     c.sf = take(sizeof(int) * (V.res.nbatch + 2));
     size_t um = (size_t)V.res.nbatch * 1024;
-    const size_t fft = 4 * (size_t)P * sizeof(D2);
+    const size_t fft = wiener_lds(P);
     const size_t setup = (size_t)2 * (V.W[0] + 1) * sizeof(int) + (size_t)2 * Y * sizeof(int) + 64;
     const size_t br = (size_t)kResWaves * 16 * kResBr * sizeof(float);
     um = um > fft ? um : fft;
