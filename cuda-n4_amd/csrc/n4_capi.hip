@@ -362,7 +362,6 @@ struct Plan {
     std::vector<int> max_iter;  // per level (max over volumes)
     std::vector<int> recon_tiles;  // recon tiles per volume
     size_t lds_fit_max[kMaxLevels] = {0}, lds_eval_max[kMaxLevels] = {0}, lds_eval32_max[kMaxLevels] = {0};
-    int cx_max[kMaxLevels] = {0};
     int mt[kMaxLevels] = {0}, nt[kMaxLevels] = {0};  // MFMA tiles along y, z per level
     size_t lds_hist = 0, lds_wiener = 0, lds_recon = 0, lds_recon_limit = 0;
     // persistent path
@@ -391,6 +390,18 @@ static void step_tiles(const int W[3], bool tiled, int tile_vox, int* rows, int*
     *tiles_x = (W[1] + r - 1) / r;
 }
 
+// Fit stage: rows per tile -- about a thousand tiles or more, of 512 to 5120
+// voxels -- and the floats of one tile's T2 (the control points that its
+// rows reach along y, all of them along z).
+static int field_rows(const int W[3]) {
+    const double vox = (double)W[0] * W[1] * W[2];
+    const double tile = std::min(5120.0, std::max(512.0, vox / 1024.0));
+    return std::min(W[1], std::max(1, std::min(64, (int)(tile / W[2]))));
+}
+static size_t field_tile(const int W[3], const int C[3]) {
+    const int spans = (int)(((int64_t)(field_rows(W) - 1) * (C[1] - 3) + W[1] - 1) / W[1]) + 1;
+    return (size_t)std::min(C[1], spans + 4) * C[2];
+}
 
 // Magic multiplier for floor(v / d) (see fdiv in the kernels).
 static uint64_t magic_div(uint32_t d) { return ((uint64_t)1 << kDivShift) / d + 1; }
@@ -566,10 +577,11 @@ struct ResPlan {
 // words (pinned host memory).
 // res (nullable, resident path): the plan holds the packed foreground in
 // place of logU, the unit lists and the slot list; no step tiles.
+// field_fit: the fit stage's tiles.
 static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4_params* p, Plan* P,
                             bool need_tables_full = true, bool tiled = false, int tile_vox = kStepTileVox,
                             const std::vector<int>* teams = nullptr, bool noalloc = false,
-                            const ResPlan* res = nullptr) {
+                            const ResPlan* res = nullptr, bool field_fit = false) {
     const int nv = (int)in.size();
     const int L = (int)p->number_of_fitting_levels;
     h->last.valid = false;  // the plan reuses the memory of the last run's records
@@ -584,7 +596,7 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
     struct VInfo {
         int W[3];
         int C[kMaxLevels][3];
-        size_t Lmax, part_stride;
+        size_t Lmax;
         int prep_rows, prep_tiles_x, recon_rows, recon_tiles_x, wtile_rows, wtiles_x;
     };
     std::vector<VInfo> vi(nv);
@@ -599,7 +611,6 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
             for (int d = 0; d < 3; ++d) I.C[l][d] = level_ncpt((int)p->ncpt[d], l);
         const int* Cf = I.C[L - 1];
         I.Lmax = (size_t)Cf[0] * Cf[1] * Cf[2];
-        I.part_stride = (size_t)Cf[1] * Cf[2];
         I.prep_rows = rows_for(I.W[1], I.W[2], kPrepTileVox);
         I.prep_tiles_x = (I.W[1] + I.prep_rows - 1) / I.prep_rows;
         I.recon_rows = rows_for(in[v].F[1], in[v].F[2], recon_tile);
@@ -708,7 +719,8 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
         o.den = lay.take(sizeof(double) * I.Lmax);
         o.latf = lay.take(sizeof(float) * I.Lmax);
         o.lresf = lay.take(sizeof(float) * I.Lmax);
-        o.part = res ? 0 : lay.take(sizeof(float) * I.W[0] * I.part_stride);
+        o.part = field_fit ? lay.take(sizeof(float) * 2 * field_tile(in[v].F, I.C[0]) * ((size_t)I.W[0] *
+                                      ((I.W[1] + field_rows(in[v].F) - 1) / field_rows(in[v].F)))) : 0;
         o.numfx = lay.take(sizeof(uint64_t) * I.Lmax * ncopies(v));
         o.hist = lay.take(sizeof(uint64_t) * nb * hcopies(v));
         o.spart = res ? 0 : lay.take(sizeof(double) * 4 * I.W[0] * I.wtiles_x);
@@ -828,7 +840,12 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
         D.den = (double*)(base + o.den);
         D.latf = (float*)(base + o.latf);
         D.lresf = (float*)(base + o.lresf);
-        D.part = res ? nullptr : (float*)(base + o.part);
+        if (field_fit) {
+            D.part = (float*)(base + o.part);
+            D.field_rows = field_rows(in[v].F);
+            D.field_tiles_x = (I.W[1] + D.field_rows - 1) / D.field_rows;
+            D.part_stride = (int32_t)field_tile(in[v].F, I.C[0]);
+        }
         D.numfx = (uint64_t*)(base + o.numfx);
         D.num_copies = ncopies(v);
         D.lmax = (int32_t)I.Lmax;
@@ -866,7 +883,6 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
         D.trace_cap = tiled ? trace_cap : 0;
         D.lvlat = tiled ? (float*)(base + o.lvlat) : nullptr;
         D.nlevels = L;
-        D.part_stride = (int32_t)I.part_stride;
         for (int l = 0; l < L; ++l) {
             D.max_iter[l] = (int)p->max_iterations[l];
             LevelDesc& LD = D.lev[l];
@@ -910,7 +926,6 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
             P->lds_fit_max[l] = std::max(P->lds_fit_max[l], lds_fit(nb, D, l, prec));
             P->lds_eval_max[l] = std::max(P->lds_eval_max[l], lds_eval(D, l, prec));
             P->lds_eval32_max[l] = std::max(P->lds_eval32_max[l], lds_eval(D, l, 0));
-            P->cx_max[l] = std::max(P->cx_max[l], D.lev[l].C[0]);
             P->mt[l] = mfma_tiles(D.lev[l].C[1]);
             P->nt[l] = mfma_tiles(D.lev[l].C[2]);
         }
@@ -2300,26 +2315,18 @@ n4_status n4_fit_bspline3d(n4_handle* h, const float* d_field, const uint8_t* d_
     for (int d = 0; d < 3; ++d)
         if (v.F[d] < 1) return fail(N4_ERR_INVALID_ARG, "empty dimension");
     Plan P;
-    s = build_plan(h, std::vector<VolIn>{v}, &p, &P, false);
+    s = build_plan(h, std::vector<VolIn>{v}, &p, &P, false, false, kStepTileVox, nullptr, false, nullptr, true);
     if (s != N4_OK) return s;
     s = check_lds(P, true, false);
     if (s != N4_OK) return s;
     VolDesc& D = P.desc[0];
+    D.logU = const_cast<float*>(d_field);
+    D.wmask = const_cast<uint8_t*>(d_mask);
+    D.lresf = d_lattice;
+    memcpy(h->stage + P.off_desc, &D, sizeof D);
     s = stage_upload(h, P.base, 0, P.upload_bytes, nullptr);
     if (s != N4_OK) return s;
-    // the fit kernel takes 16-byte loads of aligned voxel quads: it reads
-    // the plan's own padded copies of the field and the mask
-    const size_t nvox = (size_t)dims[0] * dims[1] * dims[2];
-    D2D(D.logU, d_field, sizeof(float) * nvox, nullptr);
-    D2D(D.wmask, d_mask, nvox, nullptr);
-    VolDesc* dd = dev_desc(h, P);
-    Slab* sl = dev_wslab(h, P);
-    LAUNCH(launch_level(dd, 1, 0, P.rp, nullptr));
-    LAUNCH(launch_fit(dd, sl, P.n_wslab, 0, 0, kFitDen, P.rp, P.lds_fit_max[0], P.mt[0], P.nt[0], nullptr));
-    LAUNCH(launch_lattice(dd, 1, P.cx_max[0], 0, kFitDen, P.rp, nullptr));
-    LAUNCH(launch_fit(dd, sl, P.n_wslab, 0, 0, kFitField, P.rp, P.lds_fit_max[0], P.mt[0], P.nt[0], nullptr));
-    LAUNCH(launch_lattice(dd, 1, P.cx_max[0], 0, kFitField, P.rp, nullptr));
-    D2D(d_lattice, D.lresf, sizeof(float) * D.lev[0].L, nullptr);
+    LAUNCH(launch_field_fit(dev_desc(h, P), D.W[0] * D.field_tiles_x, D.lev[0].C[0] * D.lev[0].C[1], P.rp.eps, nullptr));
     SYNC(nullptr);
     return N4_OK;
 }

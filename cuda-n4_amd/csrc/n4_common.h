@@ -7,7 +7,7 @@
 //   lattice: lat[2] f64 (ping-pong across levels), den f64, latf f32,
 //            lresf f32 (largest level size)
 //   per-slab partials (one slab = one working x index):
-//     part  f32 [W0][Cy*Cz]   fit contraction over (y, z) of the slab
+//     part  f32 [tile][2][..] fit contraction over (y, z) of a tile (fit stage)
 //     spart f64 [W0][4]       CV sums / counts and logU min / max
 //   hist  u64 [nbins]         fixed-point (2^-32) fractional histogram
 //   etab f64 [nbins], state (VolState)
@@ -138,7 +138,7 @@ struct VolDesc {
     float* latf;
     float* lresf;
     // partials
-    float* part;               // per-slab fit contraction (DEN and FIELD modes)
+    float* part;               // fit stage: numerator and denominator T2 of each tile
     uint64_t* numfx;           // num_copies x lmax fixed-point lattice numerator copies
     uint64_t* hist;            // hist_copies x nbins fixed-point bins (summed by the Wiener step)
     double* spart;
@@ -155,7 +155,9 @@ struct VolDesc {
     const int32_t* fb[3];
     int32_t nlevels;
     int32_t max_iter[kMaxLevels];
-    int32_t part_stride;       // floats per slab in part (max Cy*Cz)
+    int32_t part_stride;       // fit stage: floats of one T2 in part
+    int32_t field_rows;        // fit stage: rows per tile
+    int32_t field_tiles_x;     // such tiles per slab
     int32_t prep_rows;         // working rows per prep tile
     int32_t prep_tiles_x;      // prep tiles per working slab
     int32_t recon_rows;        // full-resolution rows per reconstruction tile
@@ -250,7 +252,7 @@ constexpr int kDivShift = 40;
 // loop); DEN and FIELD write per-slab partials reduced by the lattice
 // kernel (stage calls).  STEP takes the mode, level and iteration from the
 // volume's current step (ITER -> NUM, TRANS -> DEN_SCATTER, else nothing).
-enum FitMode : int32_t { kFitNum = 0, kFitDen = 1, kFitField = 2, kFitDenScatter = 3, kFitStep = 4 };
+enum FitMode : int32_t { kFitNum = 0, kFitDen = 1, kFitStep = 2 };
 
 // Fixed-point scale of the lattice numerator accumulated by the fit's
 // integer atomics (order-independent, so bitwise reproducible): 2^-30

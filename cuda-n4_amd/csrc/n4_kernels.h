@@ -27,7 +27,6 @@ size_t lds_hist(int nbins);
 size_t lds_wiener(int P);
 // prec (RunParams::prec) selects the FP32 or the MFMA kernels.
 size_t lds_fit(int nbins, const VolDesc& v, int level, int prec);
-size_t lds_lattice();
 size_t lds_eval(const VolDesc& v, int level, int prec);
 size_t lds_recon(const VolDesc& v);
 // What the refusal of volumes too large for a workgroup goes by: z factors of
@@ -61,7 +60,9 @@ int launch_wiener(const VolDesc* vols, int nvol, RunParams rp, size_t lds, void*
 // it: iteration within the level (selects the numerator buffer by parity).
 int launch_fit(const VolDesc* vols, const Slab* slabs, int nslab, int level, int it, int mode, RunParams rp,
                size_t lds, int mt, int nt, void* stream);
-int launch_lattice(const VolDesc* vols, int nvol, int cx_max, int level, int mode, RunParams rp, void* stream);
+// Fit stage of one volume's field V.logU under V.wmask: ntile tiles (all
+// slabs), then the lattice V.lresf of ncol = Cx * Cy control point columns.
+int launch_field_fit(const VolDesc* vols, int ntile, int ncol, double eps, void* stream);
 // Lattice update of a step (numerator copies -> lattice increment or level
 // denominator); chunks = ceil(largest level size / kBlock).
 int launch_update(const VolDesc* vols, int nvol, int chunks, RunParams rp, void* stream);

@@ -48,12 +48,14 @@
 #define BLOCK_END }
 #define BLOCK_SYNC() __syncthreads()
 #define UNROLL _Pragma("unroll")
+#define UNROLL_4 _Pragma("unroll 4")
 #else
 #define BLOCK_FOR(t) for (int t = 0; t < kBlock; ++t) {
 #define BLOCK_FOR_N(t, n) for (int t = 0; t < n; ++t) {
 #define BLOCK_END }
 #define BLOCK_SYNC() do { } while (0)
 #define UNROLL
+#define UNROLL_4
 #endif
 
 #define HD __host__ __device__ inline
@@ -1340,9 +1342,9 @@ HD void body_update(const VolDesc* vols, RunParams rp, int chunk, int vol) {
 // because the normaliser sum(w^2) factorises per axis):
 //   T1[y,cz] = sum_z g[y,z] Pz[z,cz]      (LDS, per row chunk)
 //   T2[cy,cz] += sum_y Py[y,cy] T1[y,cz]  (LDS, accumulated over the slab)
-//   part[x] = T2                          (global, per slab)
+//   the lattice numerator += T2 x the slab's x factors (fixed-point atomics)
 // Modes: NUM (g = residual, P = w^3/S), DEN (g = mask, Q = w^2; once per
-// level), FIELD (g = the logU buffer itself; stage API).
+// level).
 struct FitLds {
     N4_LDS float* E;
     N4_LDS float* zwc;  // [Cz][zmax]  factor of control point cz at z = lo(cz) + i
@@ -1373,7 +1375,7 @@ HD bool fit_step_mode(const VolState* st, int* mode, int* level, int* it) {
         return true;
     }
     if (st->s_kind == kStepTrans) {
-        *mode = kFitDenScatter;
+        *mode = kFitDen;
         *level = st->s_lvl;
         *it = 0;
         return true;
@@ -1398,14 +1400,13 @@ HD Remap make_remap(const N4_LDS float* E, double bmin, double slope, int nb) {
 
 // Contracted quantity g of one working voxel: the residual logU - E[u|v]
 // (N4.py:103-115 remap with the cudaN4.cu:242 clamp, then N4.py:313) for
-// NUM, the mask for DEN, logU itself for FIELD; 0 outside the mask.  With
+// NUM, the mask for DEN; 0 outside the mask.  With
 // confidence weights (V.wconf), the fit kernels scale g of a foreground
 // voxel by its weight (conf_scale), which scales both its numerator and its
 // denominator contribution.
 HD float fit_input(int mode, uint8_t m, float xv, bool degenerate, const Remap& R) {
     if (!m) return 0.0f;
     if (mode == kFitDen) return 1.0f;
-    if (mode == kFitField) return xv;
     if (degenerate) return 0.0f;
     float c = (xv - R.bmin) * R.islope;
     c = fminf(fmaxf(c, 0.0f), (float)R.nb);
@@ -1542,18 +1543,13 @@ HD void fit_chunks(const VolDesc& V, const LevelDesc& LD, const Slab sl, const F
 }
 
 // Adds a tile's T2, weighted by the slab's x factors, to the numerator
-// (scatter: fixed-point atomics into copy tile % num_copies) or writes it
-// as the slab's partial (stage calls).
-HD void fit_scatter(const VolDesc& V, const LevelDesc& LD, const Slab sl, const FitLds& S, bool scatter, bool den) {
+// (fixed-point atomics into copy tile % num_copies).
+HD void fit_scatter(const VolDesc& V, const LevelDesc& LD, const Slab sl, const FitLds& S, bool den) {
     const int CyCz = LD.C[1] * LD.C[2];
     BLOCK_FOR(t)
     const AxisEntry ex = *S.ex;
-    for (int pr = t; pr < CyCz; pr += kBlock) {
-        if (scatter)
-            scatter_numerator(V, LD, ex, tile_id(V, sl) % V.num_copies, den, pr, S.T2[pr]);
-        else
-            V.part[(size_t)sl.x * V.part_stride + pr] = S.T2[pr];
-    }
+    for (int pr = t; pr < CyCz; pr += kBlock)
+        scatter_numerator(V, LD, ex, tile_id(V, sl) % V.num_copies, den, pr, S.T2[pr]);
     BLOCK_END
 }
 
@@ -1570,9 +1566,7 @@ HD void body_fit(const VolDesc* vols, const Slab* slabs, int level, int it, int 
     FitLds S;
     carve_fit(smem, nb, Y, Z, rows_per_chunk(Y, Z), Cy, Cz, &S);
     const bool num = (mode == kFitNum);
-    const bool den = (mode == kFitDen || mode == kFitDenScatter);
-    const bool scatter = (mode == kFitNum || mode == kFitDenScatter);
-    const int gmode = den ? (int)kFitDen : mode;
+    const bool den = (mode == kFitDen);
     const bool degenerate = num && st->degenerate;
     const double bmin = st->bin_min, slope = st->slope;
     const Remap rm = make_remap(S.E, bmin, slope, nb);
@@ -1587,64 +1581,214 @@ HD void body_fit(const VolDesc* vols, const Slab* slabs, int level, int it, int 
         reinterpret_cast<N4_LDS int32_t*>(S.ex)[t] = reinterpret_cast<const int32_t*>(&LD.ax[0][x])[t];
     BLOCK_END
     BLOCK_SYNC();
-    fit_chunks(V, LD, sl, S, gmode, den, degenerate, rm);
-    fit_scatter(V, LD, sl, S, scatter, den);
+    fit_chunks(V, LD, sl, S, mode, den, degenerate, rm);
+    fit_scatter(V, LD, sl, S, den);
 }
 
-// --------------------------------------------------------------- lattice --
-// Mode-x contraction of the slab partials and the lattice update; one block
-// per (control-point plane cx, volume):
-//   num[cx,p] = sum_x Px[x,cx] part[x][p]   (FP64, fixed summation order)
-//   NUM  : lres = num/(den+eps); lat += lres  (N4.py:236, 317)
-//   DEN  : den = num
-//   FIELD: lres = num/(den+eps)
-// Each column p is summed by G = kBlock/CyCz threads over interleaved slabs,
-// then combined in a fixed order.
-HD void body_lattice(const VolDesc* vols, int level, int mode, RunParams rp, int cx, int vol,
-                     N4_LDS unsigned char* smem) {
-    const VolDesc& V = vols[vol];
-    const LevelDesc& LD = V.lev[level];
-    if (cx >= LD.C[0]) return;
-    if (mode == kFitNum && V.st->done) return;
-    Carve cv{smem, 0};
-    N4_LDS double* red = cv.take<double>(kBlock);
-    const int CyCz = LD.C[1] * LD.C[2];
-    const int lo = LD.sup[0][2 * cx], hi = LD.sup[0][2 * cx + 1];
-    const AxisEntry* axx = LD.ax[0];
-    const int cols = (CyCz <= kBlock) ? CyCz : kBlock;
-    const int G = kBlock / cols;
-    double* lat = V.lat[level & 1];
-    for (int p0 = 0; p0 < CyCz; p0 += cols) {
+// ----------------------------------------------------- fit of a field --
+// The fit stage (N4.py:186-237) of a given field under a mask: numerator and
+// denominator in one pass over the voxels, which it is bound by.  A workgroup
+// takes field_rows rows of one slab; a thread owns a column of voxels (one z)
+// and walks it in y, eight rows' loads at a time, with the four control
+// points of its span in registers:
+//   Q[cy,z]   = sum_y Py[y,cy] g[y,z]       (LDS, by column)
+//   T2[cy,cz] = sum_z Pz[z,cz] Q[cy,z]      (FP64)
+//   part[tile][numerator, denominator] = T2 (the tile's own rows of T2)
+// Every voxel is read as it lies (no alignment or padding asked for).  Two
+// passes of the step's slab kernel over padded copies, one workgroup of 256
+// threads per slab, took 2 x 116 us at 256 x 256 x 160 besides the copies.
+constexpr int kFieldCols = kBlock;  // columns of one z chunk
+constexpr int kFieldSpans = 12;     // rows of Q (control points) of one row batch
+constexpr int kFieldRowsMax = 64;   // rows of a tile
+struct FieldLds {
+    N4_LDS float* yp;  // [rows][4] factors of the tile's rows
+    N4_LDS float* yq;
+    N4_LDS int* yb;
+    N4_LDS float* zp;  // [columns][4]
+    N4_LDS float* zq;
+    N4_LDS int* zb;
+    N4_LDS int* cz;    // support [lo, hi) of the chunk's control points
+    N4_LDS float* Q;   // [part][numerator, denominator][cy][column]
+};
+HD size_t carve_field(N4_LDS unsigned char* base, FieldLds* o) {
+    Carve c{base, 0};
+    FieldLds L;
+    L.yp = c.take<float>(4 * kFieldRowsMax);
+    L.yq = c.take<float>(4 * kFieldRowsMax);
+    L.yb = c.take<int>(kFieldRowsMax);
+    L.zp = c.take<float>(4 * kFieldCols);
+    L.zq = c.take<float>(4 * kFieldCols);
+    L.zb = c.take<int>(kFieldCols);
+    L.cz = c.take<int>(2 * (kFieldCols + 3));
+    L.Q = c.take<float>(2 * kFieldSpans * kFieldCols);
+    if (o) *o = L;
+    return align16(c.off);
+}
+
+HD void body_field_fit(const VolDesc* vols, int bid, N4_LDS unsigned char* smem) {
+    const VolDesc& V = vols[0];
+    const LevelDesc& LD = V.lev[0];
+    const int Y = V.W[1], Z = V.W[2], Cz = LD.C[2], rows = V.field_rows;
+    const int x = bid / V.field_tiles_x, yt = (bid - x * V.field_tiles_x) * rows;
+    const int ny = Y - yt < rows ? Y - yt : rows;
+    FieldLds S;
+    carve_field(smem, &S);
+    float* dst = V.part + (size_t)bid * 2 * V.part_stride;
+    const float* im = V.logU + ((size_t)x * Y + yt) * Z;
+    const uint8_t* mask = V.wmask + ((size_t)x * Y + yt) * Z;
+    BLOCK_FOR(t)
+    for (int r = t; r < ny; r += kBlock) {
+        const AxisEntry& a = LD.ax[1][yt + r];
+        for (int k = 0; k < 4; ++k) {
+            S.yp[4 * r + k] = a.p[k];
+            S.yq[4 * r + k] = a.q[k];
+        }
+        S.yb[r] = a.b;
+    }
+    BLOCK_END
+    BLOCK_SYNC();
+    const int bt = S.yb[0], ncy = S.yb[ny - 1] - bt + 4;  // control points of the tile along y
+    for (int z0 = 0; z0 < Z; z0 += kFieldCols) {
+        const int nz = Z - z0 < kFieldCols ? Z - z0 : kFieldCols;
+        const int parts = kBlock / nz;  // runs of rows walked side by side
+        for (int y0 = 0, y1; y0 < ny; y0 = y1) {
+            // a batch of rows whose control points fit Q
+            const int b0 = S.yb[y0];
+            y1 = ny;
+            while (S.yb[y1 - 1] - b0 > kFieldSpans - 4) --y1;
+            const int cyl = S.yb[y1 - 1] - b0 + 4;
+            BLOCK_FOR(t)
+            if (y0 == 0) {
+                if (t < nz) {
+                    const AxisEntry& a = LD.ax[2][z0 + t];
+                    for (int k = 0; k < 4; ++k) {
+                        S.zp[4 * t + k] = a.p[k];
+                        S.zq[4 * t + k] = a.q[k];
+                    }
+                    S.zb[t] = a.b;
+                }
+                const int c0 = LD.ax[2][z0].b, nc = LD.ax[2][z0 + nz - 1].b + 4 - c0;
+                for (int i = t; i < 2 * nc && i < 2 * (kFieldCols + 3); i += kBlock) S.cz[i] = LD.sup[2][2 * c0 + i];
+            }
+            for (int i = t; i < 2 * parts * cyl * nz; i += kBlock) S.Q[i] = 0.0f;
+            BLOCK_END
+            BLOCK_SYNC();
+            BLOCK_FOR(t)
+            const int part = t / nz, z = t - part * nz;
+            const int r0 = y0 + (y1 - y0) * part / parts, r1 = y0 + (y1 - y0) * (part + 1) / parts;
+            if (part < parts && r0 < r1) {
+                N4_LDS float* qn = S.Q + 2 * part * cyl * nz + z;
+                N4_LDS float* qd = qn + cyl * nz;
+                float an[4] = {0, 0, 0, 0}, ad[4] = {0, 0, 0, 0};
+                int b = S.yb[r0];
+                for (int r = r0; r < r1; r += 8) {
+                    float xs[8];
+                    uint8_t ms[8];
+                    UNROLL for (int u = 0; u < 8; ++u) {
+                        const size_t w = (size_t)(r + u < r1 ? r + u : r) * Z + z0 + z;
+                        xs[u] = gp(im)[w];
+                        ms[u] = gp(mask)[w];
+                    }
+                    UNROLL for (int u = 0; u < 8; ++u) {
+                        if (r + u >= r1) break;
+                        const int br = S.yb[r + u];
+                        if (br != b) {
+                            for (int k = 0; k < 4; ++k) {
+                                qn[(b - b0 + k) * nz] += an[k];
+                                qd[(b - b0 + k) * nz] += ad[k];
+                                an[k] = ad[k] = 0.0f;
+                            }
+                            b = br;
+                        }
+                        const float g = ms[u] ? xs[u] : 0.0f, h = ms[u] ? 1.0f : 0.0f;
+                        for (int k = 0; k < 4; ++k) {
+                            an[k] += g * S.yp[4 * (r + u) + k];
+                            ad[k] += h * S.yq[4 * (r + u) + k];
+                        }
+                    }
+                }
+                for (int k = 0; k < 4; ++k) {
+                    qn[(b - b0 + k) * nz] += an[k];
+                    qd[(b - b0 + k) * nz] += ad[k];
+                }
+            }
+            BLOCK_END
+            BLOCK_SYNC();
+            // every output keeps its thread over the batches and z chunks
+            // (the first one writes it)
+            const bool first = z0 == 0 && y0 == 0;
+            const int c0 = S.zb[0], nc = S.zb[nz - 1] + 4 - c0;
+            BLOCK_FOR(t)
+            for (int e = t; e < 2 * ncy * Cz; e += kBlock) {
+                const int den = e >= ncy * Cz, pr = e - den * ncy * Cz, cy = pr / Cz + bt - b0, c = pr % Cz - c0;
+                double acc = 0.0;
+                if (cy >= 0 && cy < cyl && c >= 0 && c < nc) {
+                    const int zl = S.cz[2 * c] - z0, zh = S.cz[2 * c + 1] - z0;
+                    const int za = zl > 0 ? zl : 0, ze = zh < nz ? zh : nz;
+                    const N4_LDS float* w = den ? S.zq : S.zp;
+                    for (int part = 0; part < parts; ++part) {
+                        const N4_LDS float* q = S.Q + ((2 * part + den) * cyl + cy) * nz;
+                        for (int i = za; i < ze; ++i) acc += (double)w[4 * i + c + c0 - S.zb[i]] * (double)q[i];
+                    }
+                }
+                float* o = dst + (den ? V.part_stride : 0) + pr;
+                *o = (float)(first ? acc : (double)*o + acc);
+            }
+            BLOCK_END
+            BLOCK_SYNC();
+        }
+    }
+}
+
+// The tiles' T2 contracted along x, one block per (cx, cy): num and den in
+// FP64 over the tiles that reach the control point, in a fixed order, and
+//   lattice = num / (den + eps)  (N4.py:236)
+HD size_t carve_field_lattice(N4_LDS unsigned char* base, N4_LDS double** num, N4_LDS double** den) {
+    Carve c{base, 0};
+    N4_LDS double* a = c.take<double>(kBlock);
+    N4_LDS double* b = c.take<double>(kBlock);
+    if (num) *num = a;
+    if (den) *den = b;
+    return align16(c.off);
+}
+
+HD void body_field_lattice(const VolDesc* vols, double eps, int bid, N4_LDS unsigned char* smem) {
+    const VolDesc& V = vols[0];
+    const LevelDesc& LD = V.lev[0];
+    const int Cy = LD.C[1], Cz = LD.C[2];
+    const int cx = bid / Cy, cy = bid - cx * Cy;
+    N4_LDS double *rn, *rd;
+    carve_field_lattice(smem, &rn, &rd);
+    const int xlo = LD.sup[0][2 * cx], nx = LD.sup[0][2 * cx + 1] - xlo;
+    const int ylo = LD.sup[1][2 * cy], yhi = LD.sup[1][2 * cy + 1];
+    const int t0 = ylo / V.field_rows, nt = yhi > ylo ? (yhi - 1) / V.field_rows + 1 - t0 : 0;
+    const int cols = Cz < 64 ? Cz : 64, G = kBlock / cols, n = nx * nt;
+    for (int z0 = 0; z0 < Cz; z0 += cols) {
         BLOCK_FOR(t)
-        double acc = 0.0;
-        const int g = t / cols, p = p0 + (t - (t / cols) * cols);
-        if (g < G && p < CyCz) {
-            for (int xx = lo + g; xx < hi; xx += G) {
-                const AxisEntry& e = axx[xx];
-                const float wx = (mode == kFitDen) ? e.q[cx - e.b] : e.p[cx - e.b];
-                acc += (double)wx * (double)V.part[(size_t)xx * V.part_stride + p];
+        const int g = t / cols, c = z0 + (t - g * cols);
+        double an = 0.0, ad = 0.0;
+        if (g < G && c < Cz) {
+            UNROLL_4 for (int i = g; i < n; i += G) {
+                const int xi = i / nt, tile = t0 + (i - xi * nt), x = xlo + xi;
+                const AxisEntry& e = LD.ax[0][x];
+                const int cyl = cy - LD.ax[1][tile * V.field_rows].b;
+                const float* p = V.part + ((size_t)x * V.field_tiles_x + tile) * 2 * V.part_stride + cyl * Cz + c;
+                an += (double)e.p[cx - e.b] * (double)p[0];
+                ad += (double)e.q[cx - e.b] * (double)p[V.part_stride];
             }
         }
-        red[t] = acc;
+        rn[t] = an;
+        rd[t] = ad;
         BLOCK_END
         BLOCK_SYNC();
         BLOCK_FOR(t)
-        const int p = p0 + t;
-        if (t < cols && p < CyCz) {
-            double numv = 0.0;
-            for (int g = 0; g < G; ++g) numv += red[g * cols + t];
-            const size_t l = (size_t)cx * CyCz + p;
-            if (mode == kFitDen) {
-                V.den[l] = numv;
-            } else {
-                const double lres = numv / (V.den[l] + rp.eps);
-                if (mode == kFitNum) {
-                    const double nl = lat[l] + lres;
-                    lat[l] = nl;
-                    V.latf[l] = (float)nl;
-                }
-                V.lresf[l] = (float)lres;
+        if (t < cols && z0 + t < Cz) {
+            double num = 0.0, den = 0.0;
+            for (int g = 0; g < G; ++g) {
+                num += rn[g * cols + t];
+                den += rd[g * cols + t];
             }
+            V.lresf[(size_t)bid * Cz + z0 + t] = (float)(num / (den + eps));
         }
         BLOCK_END
         BLOCK_SYNC();
@@ -2476,7 +2620,7 @@ HD void persist_fit(const VolDesc& V, const LevelDesc& LD, const Slab* my, int n
             if (t < (int)(sizeof(AxisEntry) / 4))
                 reinterpret_cast<N4_LDS int32_t*>(S.M.ex)[t] = reinterpret_cast<const int32_t*>(&LD.ax[0][sl.x])[t];
             __syncthreads();
-            fit_mfma_tile<PREC, 1, 1>(V, LD, sl, S.M, gmode, den, true, degenerate, rm, ms, xs);
+            fit_mfma_tile<PREC, 1, 1>(V, LD, sl, S.M, gmode, den, degenerate, rm, ms, xs);
             __syncthreads();
         }
         return;
@@ -2491,7 +2635,7 @@ HD void persist_fit(const VolDesc& V, const LevelDesc& LD, const Slab* my, int n
         BLOCK_END
         BLOCK_SYNC();
         fit_chunks(V, LD, sl, S.F, gmode, den, degenerate, rm);
-        fit_scatter(V, LD, sl, S.F, true, den);
+        fit_scatter(V, LD, sl, S.F, den);
         BLOCK_SYNC();
     }
 }
@@ -2710,7 +2854,8 @@ size_t lds_hist(int nbins) {
     return std::max(align16(4 * kBlock * sizeof(double)), align16((size_t)kHistLanes * hist_stride(nbins) * sizeof(uint64_t)));
 }
 size_t lds_wiener(int P) { return align16(wiener_lds(P)); }
-size_t lds_lattice() { return align16(kBlock * sizeof(double)); }
+size_t lds_field_fit() { return carve_field(nullptr, nullptr); }
+size_t lds_field_lattice() { return carve_field_lattice(nullptr, nullptr, nullptr); }
 size_t lds_flat(int nbins) { return align16(4 * kBlock * sizeof(double)) + align16(nbins * sizeof(double)); }
 
 size_t lds_fit(int nbins, const VolDesc& v, int level, int prec) {
@@ -2790,9 +2935,14 @@ __global__ __launch_bounds__(kBlock) void k_fit(const VolDesc* __restrict__ vols
     body_fit(vols, slabs, level, it, mode, rp, blockIdx.x, SMEM());
 }
 
-__global__ __launch_bounds__(kBlock) void k_lattice(const VolDesc* __restrict__ vols, int level, int mode, RunParams rp) {
+__global__ __launch_bounds__(kBlock) void k_field_fit(const VolDesc* __restrict__ vols) {
     HIP_DYNAMIC_SHARED(double, smem_);
-    body_lattice(vols, level, mode, rp, blockIdx.x, blockIdx.y, SMEM());
+    body_field_fit(vols, (int)blockIdx.x, SMEM());
+}
+
+__global__ __launch_bounds__(kBlock) void k_field_lattice(const VolDesc* __restrict__ vols, double eps) {
+    HIP_DYNAMIC_SHARED(double, smem_);
+    body_field_lattice(vols, eps, (int)blockIdx.x, SMEM());
 }
 
 __global__ __launch_bounds__(kBlock) void k_update(const VolDesc* __restrict__ vols, RunParams rp) {
@@ -3013,10 +3163,11 @@ int launch_fit(const VolDesc* vols, const Slab* slabs, int nslab, int level, int
     return last_launch_status();
 }
 
-int launch_lattice(const VolDesc* vols, int nvol, int cx_max, int level, int mode, RunParams rp, void* stream) {
-    if (nvol <= 0 || cx_max <= 0) return 0;
-    hipLaunchKernelGGL(k_lattice, dim3(cx_max, nvol), dim3(kBlock), lds_lattice(), (hipStream_t)stream, vols, level,
-                       mode, rp);
+int launch_field_fit(const VolDesc* vols, int ntile, int ncol, double eps, void* stream) {
+    hipLaunchKernelGGL(k_field_fit, dim3(ntile), dim3(kBlock), lds_field_fit(), (hipStream_t)stream, vols);
+    const int s = last_launch_status();
+    if (s) return s;
+    hipLaunchKernelGGL(k_field_lattice, dim3(ncol), dim3(kBlock), lds_field_lattice(), (hipStream_t)stream, vols, eps);
     return last_launch_status();
 }
 
@@ -3130,10 +3281,11 @@ int launch_fit(const VolDesc* vols, const Slab* slabs, int nslab, int level, int
     return 0;
 }
 
-int launch_lattice(const VolDesc* vols, int nvol, int cx_max, int level, int mode, RunParams rp, void*) {
-    unsigned char* b = emu_lds(lds_lattice());
-    for (int v = 0; v < nvol; ++v)
-        for (int cx = 0; cx < cx_max; ++cx) body_lattice(vols, level, mode, rp, cx, v, b);
+int launch_field_fit(const VolDesc* vols, int ntile, int ncol, double eps, void*) {
+    unsigned char* b = emu_lds(lds_field_fit());
+    for (int i = 0; i < ntile; ++i) body_field_fit(vols, i, b);
+    b = emu_lds(lds_field_lattice());
+    for (int i = 0; i < ncol; ++i) body_field_lattice(vols, eps, i, b);
     return 0;
 }
 

@@ -259,15 +259,13 @@ __device__ inline void fit_mfma_load(const VolDesc& V, const Slab sl, int y0, in
 
 // The (y, z) contraction of one tile on MFMA (tables, E for NUM, and the
 // slab's x factors in S.ex ready; ms/xs hold this wave's first block,
-// fit_mfma_load(16 * wave, 0)), then the scatter (or the slab partial for
-// stage calls).
+// fit_mfma_load(16 * wave, 0)), then the scatter.
 template <int PREC, int MT, int NT>
 __device__ void fit_mfma_tile(const VolDesc& V, const LevelDesc& LD, const Slab sl, const FitMfmaLds& S, int gmode,
-                              bool den, bool scatter, bool degenerate, const Remap& rm,
+                              bool den, bool degenerate, const Remap& rm,
                               uint8_t (&ms)[4 * kFitRuns], float (&xs)[4 * kFitRuns]) {
     const int Z = V.W[2];
     const int Cy = LD.C[1], Cz = LD.C[2];
-    const int x = sl.x;
     const int t = (int)threadIdx.x, lane = t & 63, wv = t >> 6, r16 = lane & 15, g4 = lane >> 4;
     const int Yt = sl.ny;  // the tile's rows sl.y0 .. sl.y0 + Yt (Py columns are tile-local)
     f32x4 acc[MT][NT];
@@ -369,7 +367,6 @@ __device__ void fit_mfma_tile(const VolDesc& V, const LevelDesc& LD, const Slab 
             __syncthreads();
         }
     }
-    float* out = V.part + (size_t)x * V.part_stride;
     const AxisEntry ex = *S.ex;
     for (int e = t; e < kE; e += kBlock) {
         const int ln = e & 63, i = (e >> 6) & 3, tile = e >> 8;
@@ -377,10 +374,7 @@ __device__ void fit_mfma_tile(const VolDesc& V, const LevelDesc& LD, const Slab 
         const int cy = m * 16 + 4 * (ln >> 4) + i, cz = n * 16 + (ln & 15);
         if (cy < Cy && cz < Cz) {
             const float r = kSlots ? ((S.red[e] + S.red[kE + e]) + S.red[2 * kE + e]) + S.red[3 * kE + e] : S.red[e];
-            if (scatter)
-                scatter_numerator(V, LD, ex, tile_id(V, sl) % V.num_copies, den, cy * Cz + cz, r);
-            else
-                out[cy * Cz + cz] = r;
+            scatter_numerator(V, LD, ex, tile_id(V, sl) % V.num_copies, den, cy * Cz + cz, r);
         }
     }
 }
@@ -398,9 +392,7 @@ __device__ void body_fit_mfma(const VolDesc* vols, const Slab* slabs, int level,
     FitMfmaLds S;
     carve_fit_mfma(smem, nb, V.wtile_rows, Z, MT, NT, PREC, &S);
     const bool num = (mode == kFitNum);
-    const bool den = (mode == kFitDen || mode == kFitDenScatter);
-    const bool scatter = (mode == kFitNum || mode == kFitDenScatter);
-    const int gmode = den ? (int)kFitDen : mode;
+    const bool den = (mode == kFitDen);
     const bool degenerate = num && st->degenerate;
     const double bmin = st->bin_min, slope = st->slope;
     const int kf = den ? 2 : 1;  // q = w^2 for the denominator, p = w^3/S otherwise
@@ -418,7 +410,7 @@ __device__ void body_fit_mfma(const VolDesc* vols, const Slab* slabs, int level,
     if (t < (int)(sizeof(AxisEntry) / 4))
         reinterpret_cast<N4_LDS int32_t*>(S.ex)[t] = reinterpret_cast<const int32_t*>(&LD.ax[0][sl.x])[t];
     __syncthreads();
-    fit_mfma_tile<PREC, MT, NT>(V, LD, sl, S, gmode, den, scatter, degenerate, rm, ms, xs);
+    fit_mfma_tile<PREC, MT, NT>(V, LD, sl, S, mode, den, degenerate, rm, ms, xs);
 }
 
 // ------------------------------------------------------------------ eval --
