@@ -577,11 +577,24 @@ struct ResPlan {
 // words (pinned host memory).
 // res (nullable, resident path): the plan holds the packed foreground in
 // place of logU, the unit lists and the slot list; no step tiles.
-// field_fit: the fit stage's tiles.
+// use: the parts of the upload that the call's kernels read.  A stage call
+// takes what its one or two kernels need: the other tables and slab lists of
+// a correction cost it more than those kernels (512 sines and cosines and
+// 22528 preparation tiles for the evaluation of 256 x 256 x 176, say).
+enum PlanUse : unsigned {
+    kUseFull = 1,       // full-resolution axis tables and reconstruction tiles
+    kUseWork = 2,       // working-grid axis tables of every level
+    kUsePrep = 4,       // preparation tiles
+    kUseSteps = 8,      // working slabs (step tiles)
+    kUseTwiddle = 16,   // Wiener transforms
+    kUseFieldFit = 32,  // the fit stage's tiles
+    kUseCorrection = kUseFull | kUseWork | kUsePrep | kUseSteps | kUseTwiddle
+};
 static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4_params* p, Plan* P,
-                            bool need_tables_full = true, bool tiled = false, int tile_vox = kStepTileVox,
+                            unsigned use = kUseCorrection, bool tiled = false, int tile_vox = kStepTileVox,
                             const std::vector<int>* teams = nullptr, bool noalloc = false,
-                            const ResPlan* res = nullptr, bool field_fit = false) {
+                            const ResPlan* res = nullptr) {
+    const bool need_tables_full = use & kUseFull, field_fit = use & kUseFieldFit;
     const int nv = (int)in.size();
     const int L = (int)p->number_of_fitting_levels;
     h->last.valid = false;  // the plan reuses the memory of the last run's records
@@ -620,7 +633,8 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
         nps += I.W[0] * I.prep_tiles_x;
         nfs += in[v].F[0] * I.recon_tiles_x;
     }
-    if (res) nws = 0;  // no step tiles
+    if (res || !(use & kUseSteps)) nws = 0;  // no step tiles
+    if (!(use & kUsePrep)) nps = 0;
     P->n_wslab = nws;
     P->n_pslab = nps;
     P->recon_tiles.assign(nv, 0);
@@ -638,7 +652,7 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
     if (res)
         for (int v = 0; v < nv; ++v) P->n_slots += res->nchunk[v];
     P->off_slots = lay.take(sizeof(int32_t) * P->n_slots);
-    P->off_tw = lay.take(sizeof(D2) * P->rp.P);
+    P->off_tw = lay.take(use & kUseTwiddle ? sizeof(D2) * P->rp.P : 0);
     P->n_work = 0;
     if (teams)
         for (int v = 0; v < nv; ++v) P->n_work += (*teams)[v];
@@ -669,7 +683,7 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
         return ax_jobs[it->second];
     };
     std::vector<size_t> off_ax(nv * kMaxLevels * 3), off_sup(nv * kMaxLevels * 3), off_fw(nv * 3), off_fb(nv * 3);
-    for (int v = 0; v < nv; ++v)
+    for (int v = 0; v < nv && (use & kUseWork); ++v)
         for (int l = 0; l < L; ++l)
             for (int d = 0; d < 3; ++d) {
                 const AxisJob& j = axis_slot(false, vi[v].W[d], (double)vi[v].W[d], vi[v].C[l][d]);
@@ -772,7 +786,7 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
     Slab* fs = (Slab*)(hb + P->off_fslab);
     Slab* ps = (Slab*)(hb + P->off_pslab);
     int iws = 0, ifs = 0, ips = 0, iwk = 0;
-    {
+    if (use & kUseTwiddle) {
         D2* tw = (D2*)(hb + P->off_tw);
         for (int m = 0; m < P->rp.P; ++m) {
             const double ang = 2.0 * (double)m / (double)P->rp.P;  // in units of pi
@@ -888,6 +902,7 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
             LevelDesc& LD = D.lev[l];
             for (int d = 0; d < 3; ++d) {
                 LD.C[d] = I.C[l][d];
+                if (!(use & kUseWork)) continue;
                 LD.ax[d] = (const AxisEntry*)(base + off_ax[(v * kMaxLevels + l) * 3 + d]);
                 LD.sup[d] = (const int32_t*)(base + off_sup[(v * kMaxLevels + l) * 3 + d]);
             }
@@ -909,9 +924,9 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
             P->lds_persist = std::max(P->lds_persist, lds_persist(D, nb, P->rp.P, P->rp.prec));
         }
         for (int x = 0; x < I.W[0]; ++x) {
-            for (int y0 = 0; y0 < I.W[1] && !res; y0 += I.wtile_rows)
+            for (int y0 = 0; y0 < I.W[1] && nws; y0 += I.wtile_rows)
                 ws[iws++] = Slab{v, x, y0, std::min(I.wtile_rows, I.W[1] - y0)};
-            for (int y0 = 0; y0 < I.W[1]; y0 += I.prep_rows)
+            for (int y0 = 0; y0 < I.W[1] && nps; y0 += I.prep_rows)
                 ps[ips++] = Slab{v, x, y0, std::min(I.prep_rows, I.W[1] - y0)};
         }
         if (need_tables_full)
@@ -1519,14 +1534,14 @@ static n4_status run_batch(n4_handle* h, const std::vector<VolIn>& in_user, cons
         stage_wait(h);
         memcpy(h->stage + P.off_desc, P.desc.data(), sizeof(VolDesc) * nv);
     } else {
-        s = build_plan(h, in, p, &P, true, true, sch.tile_vox, teams_path ? &teams : nullptr, noalloc,
+        s = build_plan(h, in, p, &P, kUseCorrection, true, sch.tile_vox, teams_path ? &teams : nullptr, noalloc,
                        resident ? &res : nullptr);
         if (s == N4_ERR_NO_MEMORY && noalloc && resident) {
             // (the step path needs a little less of the scratch array)
             resident = false;
             g_err.clear();
             P = Plan();
-            s = build_plan(h, in, p, &P, true, true, sch.tile_vox, nullptr, true);
+            s = build_plan(h, in, p, &P, kUseCorrection, true, sch.tile_vox, nullptr, true);
         }
         if (s != N4_OK) return s;
         if (!noalloc) {
@@ -2208,7 +2223,7 @@ static n4_status flat_plan(n4_handle* h, uint64_t n, int nbins, Plan* P, const f
     p.number_of_fitting_levels = 1;
     const int nslab = (int)((n + kChunkVox - 1) / kChunkVox);
     VolIn v{x, m, N4_MASK_U8, {nslab, 1, kChunkVox}, 1, nullptr, nullptr, nullptr, nullptr};
-    n4_status s = build_plan(h, std::vector<VolIn>{v}, &p, P, false);
+    n4_status s = build_plan(h, std::vector<VolIn>{v}, &p, P, kUseSteps | (hist ? kUseTwiddle : 0u));
     if (s != N4_OK) return s;
     VolDesc& D = P->desc[0];
     D.nvox_w = (int64_t)n;
@@ -2315,7 +2330,7 @@ n4_status n4_fit_bspline3d(n4_handle* h, const float* d_field, const uint8_t* d_
     for (int d = 0; d < 3; ++d)
         if (v.F[d] < 1) return fail(N4_ERR_INVALID_ARG, "empty dimension");
     Plan P;
-    s = build_plan(h, std::vector<VolIn>{v}, &p, &P, false, false, kStepTileVox, nullptr, false, nullptr, true);
+    s = build_plan(h, std::vector<VolIn>{v}, &p, &P, kUseWork | kUseFieldFit);
     if (s != N4_OK) return s;
     s = check_lds(P, true, false);
     if (s != N4_OK) return s;
@@ -2345,7 +2360,7 @@ n4_status n4_evaluate_bspline3d(n4_handle* h, const float* d_lattice, const uint
     for (int d = 0; d < 3; ++d)
         if (v.F[d] < 1) return fail(N4_ERR_INVALID_ARG, "empty dimension");
     Plan P;
-    s = build_plan(h, std::vector<VolIn>{v}, &p, &P, true);
+    s = build_plan(h, std::vector<VolIn>{v}, &p, &P, kUseFull);
     if (s != N4_OK) return s;
     s = check_lds(P, false, true);
     if (s != N4_OK) return s;
@@ -2410,7 +2425,7 @@ n4_status n4_upsample_lattice3d(n4_handle* h, const float* d_lattice, const uint
     // A 1x1x1 dummy grid: only the lattice buffers of the plan are used.
     VolIn v{nullptr, nullptr, N4_MASK_NONE, {1, 1, 1}, 1, nullptr, nullptr, nullptr, nullptr};
     Plan P;
-    s = build_plan(h, std::vector<VolIn>{v}, &p, &P, false);
+    s = build_plan(h, std::vector<VolIn>{v}, &p, &P, kUseWork);
     if (s != N4_OK) return s;
     s = stage_upload(h, P.base, 0, P.upload_bytes, nullptr);
     if (s != N4_OK) return s;
