@@ -1589,21 +1589,24 @@ HD void body_fit(const VolDesc* vols, const Slab* slabs, int level, int it, int 
 // The fit stage (N4.py:186-237) of a given field under a mask: numerator and
 // denominator in one pass over the voxels, which it is bound by.  A workgroup
 // takes field_rows rows of one slab; a thread owns a column of voxels (one z)
-// and walks it in y, eight rows' loads at a time, with the four control
-// points of its span in registers:
+// and walks it in y, span by span, eight rows' loads at a time, with the
+// span's four control points in registers:
 //   Q[cy,z]   = sum_y Py[y,cy] g[y,z]       (LDS, by column)
 //   T2[cy,cz] = sum_z Pz[z,cz] Q[cy,z]      (FP64)
 //   part[tile][numerator, denominator] = T2 (the tile's own rows of T2)
 // Every voxel is read as it lies (no alignment or padding asked for).  Two
 // passes of the step's slab kernel over padded copies, one workgroup of 256
-// threads per slab, took 2 x 116 us at 256 x 256 x 160 besides the copies.
+// threads per slab, took 2 x 116 us at 256 x 256 x 160 besides the copies;
+// this takes 25.3 us, the read alone about 13.
 constexpr int kFieldCols = kBlock;  // columns of one z chunk
-constexpr int kFieldSpans = 12;     // rows of Q (control points) of one row batch
+constexpr int kFieldSpans = 6;      // rows of Q (control points) of one row batch
 constexpr int kFieldRowsMax = 64;   // rows of a tile
+constexpr int kFieldAhead = 8;      // rows in flight per thread (16: 27.3 against 26.0 us)
 struct FieldLds {
     N4_LDS float* yp;  // [rows][4] factors of the tile's rows
     N4_LDS float* yq;
     N4_LDS int* yb;
+    N4_LDS int* ye;    // end of the row's span, in rows of the tile
     N4_LDS float* zp;  // [columns][4]
     N4_LDS float* zq;
     N4_LDS int* zb;
@@ -1613,9 +1616,10 @@ struct FieldLds {
 HD size_t carve_field(N4_LDS unsigned char* base, FieldLds* o) {
     Carve c{base, 0};
     FieldLds L;
-    L.yp = c.take<float>(4 * kFieldRowsMax);
-    L.yq = c.take<float>(4 * kFieldRowsMax);
+    L.yp = c.take<float>(4 * (kFieldRowsMax + kFieldAhead));
+    L.yq = c.take<float>(4 * (kFieldRowsMax + kFieldAhead));
     L.yb = c.take<int>(kFieldRowsMax);
+    L.ye = c.take<int>(kFieldRowsMax);
     L.zp = c.take<float>(4 * kFieldCols);
     L.zq = c.take<float>(4 * kFieldCols);
     L.zb = c.take<int>(kFieldCols);
@@ -1644,7 +1648,9 @@ HD void body_field_fit(const VolDesc* vols, int bid, N4_LDS unsigned char* smem)
             S.yq[4 * r + k] = a.q[k];
         }
         S.yb[r] = a.b;
+        S.ye[r] = LD.sup[1][2 * a.b + 1] - yt;
     }
+    for (int r = 4 * ny + t; r < 4 * (ny + kFieldAhead); r += kBlock) S.yp[r] = S.yq[r] = 0.0f;
     BLOCK_END
     BLOCK_SYNC();
     const int bt = S.yb[0], ncy = S.yb[ny - 1] - bt + 4;  // control points of the tile along y
@@ -1679,41 +1685,45 @@ HD void body_field_fit(const VolDesc* vols, int bid, N4_LDS unsigned char* smem)
             if (part < parts && r0 < r1) {
                 N4_LDS float* qn = S.Q + 2 * part * cyl * nz + z;
                 N4_LDS float* qd = qn + cyl * nz;
-                float an[4] = {0, 0, 0, 0}, ad[4] = {0, 0, 0, 0};
-                int b = S.yb[r0];
-                for (int r = r0; r < r1; r += 8) {
-                    float xs[8];
-                    uint8_t ms[8];
-                    UNROLL for (int u = 0; u < 8; ++u) {
-                        const size_t w = (size_t)(r + u < r1 ? r + u : r) * Z + z0 + z;
-                        xs[u] = gp(im)[w];
-                        ms[u] = gp(mask)[w];
-                    }
-                    UNROLL for (int u = 0; u < 8; ++u) {
-                        if (r + u >= r1) break;
-                        const int br = S.yb[r + u];
-                        if (br != b) {
+                for (int r = r0; r < r1;) {  // the rows of one span
+                    const int b = S.yb[r], re = S.ye[r] < r1 ? S.ye[r] : r1;
+                    float an[4] = {0, 0, 0, 0}, ad[4] = {0, 0, 0, 0};
+                    for (; r < re; r += kFieldAhead) {
+                        float xs[kFieldAhead];
+                        uint8_t ms[kFieldAhead];
+                        UNROLL for (int u = 0; u < kFieldAhead; ++u) {
+                            const uint32_t w = (uint32_t)((r + u < re ? r + u : r) * Z + z0 + z);
+                            xs[u] = gp(im)[w];
+                            ms[u] = gp(mask)[w];
+                        }
+                        UNROLL for (int u = 0; u < kFieldAhead; ++u) {
+                            const bool m = r + u < re && ms[u];
+                            const float g = m ? xs[u] : 0.0f, h = m ? 1.0f : 0.0f;
                             for (int k = 0; k < 4; ++k) {
-                                qn[(b - b0 + k) * nz] += an[k];
-                                qd[(b - b0 + k) * nz] += ad[k];
-                                an[k] = ad[k] = 0.0f;
+                                an[k] += g * S.yp[4 * (r + u) + k];
+                                ad[k] += h * S.yq[4 * (r + u) + k];
                             }
-                            b = br;
-                        }
-                        const float g = ms[u] ? xs[u] : 0.0f, h = ms[u] ? 1.0f : 0.0f;
-                        for (int k = 0; k < 4; ++k) {
-                            an[k] += g * S.yp[4 * (r + u) + k];
-                            ad[k] += h * S.yq[4 * (r + u) + k];
                         }
                     }
-                }
-                for (int k = 0; k < 4; ++k) {
-                    qn[(b - b0 + k) * nz] += an[k];
-                    qd[(b - b0 + k) * nz] += ad[k];
+                    r = re;
+                    for (int k = 0; k < 4; ++k) {
+                        qn[(b - b0 + k) * nz] += an[k];
+                        qd[(b - b0 + k) * nz] += ad[k];
+                    }
                 }
             }
             BLOCK_END
             BLOCK_SYNC();
+            if (parts > 1) {
+                BLOCK_FOR(t)
+                for (int e = t; e < 2 * cyl * nz; e += kBlock) {
+                    float a = S.Q[e];
+                    for (int i = 1; i < parts; ++i) a += S.Q[2 * i * cyl * nz + e];
+                    S.Q[e] = a;
+                }
+                BLOCK_END
+                BLOCK_SYNC();
+            }
             // every output keeps its thread over the batches and z chunks
             // (the first one writes it)
             const bool first = z0 == 0 && y0 == 0;
@@ -1723,12 +1733,14 @@ HD void body_field_fit(const VolDesc* vols, int bid, N4_LDS unsigned char* smem)
                 const int den = e >= ncy * Cz, pr = e - den * ncy * Cz, cy = pr / Cz + bt - b0, c = pr % Cz - c0;
                 double acc = 0.0;
                 if (cy >= 0 && cy < cyl && c >= 0 && c < nc) {
-                    const int zl = S.cz[2 * c] - z0, zh = S.cz[2 * c + 1] - z0;
-                    const int za = zl > 0 ? zl : 0, ze = zh < nz ? zh : nz;
-                    const N4_LDS float* w = den ? S.zq : S.zp;
-                    for (int part = 0; part < parts; ++part) {
-                        const N4_LDS float* q = S.Q + ((2 * part + den) * cyl + cy) * nz;
-                        for (int i = za; i < ze; ++i) acc += (double)w[4 * i + c + c0 - S.zb[i]] * (double)q[i];
+                    const N4_LDS float* q = S.Q + (den * cyl + cy) * nz;
+                    for (int k = 3; k >= 0; --k) {  // the spans that c reaches: c - k
+                        const int sp = c - k;
+                        if (sp < 0 || sp > nc - 4) continue;
+                        const int zl = S.cz[2 * sp + 6] - z0, zh = S.cz[2 * sp + 1] - z0;
+                        const int za = zl > 0 ? zl : 0, ze = zh < nz ? zh : nz;
+                        const N4_LDS float* w = (den ? S.zq : S.zp) + k;
+                        UNROLL_4 for (int i = za; i < ze; ++i) acc += (double)w[4 * i] * (double)q[i];
                     }
                 }
                 float* o = dst + (den ? V.part_stride : 0) + pr;
@@ -1743,10 +1755,12 @@ HD void body_field_fit(const VolDesc* vols, int bid, N4_LDS unsigned char* smem)
 // The tiles' T2 contracted along x, one block per (cx, cy): num and den in
 // FP64 over the tiles that reach the control point, in a fixed order, and
 //   lattice = num / (den + eps)  (N4.py:236)
+// (11^3 control points of 256 x 256 x 160: 6.9 us; 256 threads 10.4, 1024 7.6)
+constexpr int kFieldLatticeBlock = 512;
 HD size_t carve_field_lattice(N4_LDS unsigned char* base, N4_LDS double** num, N4_LDS double** den) {
     Carve c{base, 0};
-    N4_LDS double* a = c.take<double>(kBlock);
-    N4_LDS double* b = c.take<double>(kBlock);
+    N4_LDS double* a = c.take<double>(kFieldLatticeBlock);
+    N4_LDS double* b = c.take<double>(kFieldLatticeBlock);
     if (num) *num = a;
     if (den) *den = b;
     return align16(c.off);
@@ -1762,9 +1776,9 @@ HD void body_field_lattice(const VolDesc* vols, double eps, int bid, N4_LDS unsi
     const int xlo = LD.sup[0][2 * cx], nx = LD.sup[0][2 * cx + 1] - xlo;
     const int ylo = LD.sup[1][2 * cy], yhi = LD.sup[1][2 * cy + 1];
     const int t0 = ylo / V.field_rows, nt = yhi > ylo ? (yhi - 1) / V.field_rows + 1 - t0 : 0;
-    const int cols = Cz < 64 ? Cz : 64, G = kBlock / cols, n = nx * nt;
+    const int cols = Cz < 64 ? Cz : 64, G = kFieldLatticeBlock / cols, n = nx * nt;
     for (int z0 = 0; z0 < Cz; z0 += cols) {
-        BLOCK_FOR(t)
+        BLOCK_FOR_N(t, kFieldLatticeBlock)
         const int g = t / cols, c = z0 + (t - g * cols);
         double an = 0.0, ad = 0.0;
         if (g < G && c < Cz) {
@@ -1781,7 +1795,7 @@ HD void body_field_lattice(const VolDesc* vols, double eps, int bid, N4_LDS unsi
         rd[t] = ad;
         BLOCK_END
         BLOCK_SYNC();
-        BLOCK_FOR(t)
+        BLOCK_FOR_N(t, kFieldLatticeBlock)
         if (t < cols && z0 + t < Cz) {
             double num = 0.0, den = 0.0;
             for (int g = 0; g < G; ++g) {
@@ -2940,7 +2954,7 @@ __global__ __launch_bounds__(kBlock) void k_field_fit(const VolDesc* __restrict_
     body_field_fit(vols, (int)blockIdx.x, SMEM());
 }
 
-__global__ __launch_bounds__(kBlock) void k_field_lattice(const VolDesc* __restrict__ vols, double eps) {
+__global__ __launch_bounds__(kFieldLatticeBlock) void k_field_lattice(const VolDesc* __restrict__ vols, double eps) {
     HIP_DYNAMIC_SHARED(double, smem_);
     body_field_lattice(vols, eps, (int)blockIdx.x, SMEM());
 }
@@ -3167,7 +3181,7 @@ int launch_field_fit(const VolDesc* vols, int ntile, int ncol, double eps, void*
     hipLaunchKernelGGL(k_field_fit, dim3(ntile), dim3(kBlock), lds_field_fit(), (hipStream_t)stream, vols);
     const int s = last_launch_status();
     if (s) return s;
-    hipLaunchKernelGGL(k_field_lattice, dim3(ncol), dim3(kBlock), lds_field_lattice(), (hipStream_t)stream, vols, eps);
+    hipLaunchKernelGGL(k_field_lattice, dim3(ncol), dim3(kFieldLatticeBlock), lds_field_lattice(), (hipStream_t)stream, vols, eps);
     return last_launch_status();
 }
 
