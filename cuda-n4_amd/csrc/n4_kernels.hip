@@ -2234,6 +2234,9 @@ HD void body_recon(const VolDesc* vols, const Slab* slabs, int level, RunParams 
 // reductions write spart[x] (reduced on the host):
 //   minmax (count, count, min, max); sum (sum, count, min, max);
 //   cv (count, sum u, sum u^2, -) with u = exp(a-b) - 1; remap writes out.
+// kFlatAhead voxels per thread in flight: the loads (the mask's first) of one
+// voxel at a time took 11.4 us of a 64 x 64 x 44 image's 45 workgroups.
+constexpr int kFlatAhead = 8;
 HD void body_flat(const VolDesc* vols, const Slab* slabs, int op, const float* a, const float* b,
                   float* out, RunParams rp, int bid, N4_LDS unsigned char* smem) {
     const Slab sl = slabs[bid];
@@ -2250,51 +2253,67 @@ HD void body_flat(const VolDesc* vols, const Slab* slabs, int op, const float* a
         for (int i = t; i < nb; i += kBlock) E[i] = V.etab[i];
         BLOCK_END
         BLOCK_SYNC();
+        const bool degenerate = V.st->degenerate;
         BLOCK_FOR(t)
-        for (int k = t; k < kChunkVox; k += kBlock) {
-            const int64_t v = v0 + k;
-            if (v >= n) break;
-            const bool m = V.wmask ? (V.wmask[v] != 0) : true;
-            float o = 0.0f;
-            if (m) {
-                if (V.st->degenerate) {
-                    o = a[v];
-                } else {
-                    double c = ((double)a[v] - bmin) / slope;
-                    c = fmin(fmax(c, 0.0), (double)nb);
-                    const double fl = floor(c);
-                    const int idx = (int)fl;
-                    o = (float)((idx < nb - 1) ? E[idx] + (E[idx + 1] - E[idx]) * (c - fl) : E[nb - 1]);
-                }
+        for (int k = t; k < kChunkVox && v0 + k < n; k += kFlatAhead * kBlock) {
+            float as[kFlatAhead];
+            bool ms[kFlatAhead];
+            UNROLL for (int u = 0; u < kFlatAhead; ++u) {
+                const int64_t v = v0 + k + u * kBlock, w = v < n ? v : v0 + k;
+                as[u] = gp(a)[w];
+                ms[u] = V.wmask ? gp(V.wmask)[w] != 0 : true;
             }
-            out[v] = o;
+            UNROLL for (int u = 0; u < kFlatAhead; ++u) {
+                const int64_t v = v0 + k + u * kBlock;
+                if (v >= n) break;
+                float o = 0.0f;
+                if (ms[u]) {
+                    if (degenerate) {
+                        o = as[u];
+                    } else {
+                        double c = ((double)as[u] - bmin) / slope;
+                        c = fmin(fmax(c, 0.0), (double)nb);
+                        const double fl = floor(c);
+                        const int idx = (int)fl;
+                        o = (float)((idx < nb - 1) ? E[idx] + (E[idx + 1] - E[idx]) * (c - fl) : E[nb - 1]);
+                    }
+                }
+                gp(out)[v] = o;
+            }
         }
         BLOCK_END
         return;
     }
     BLOCK_FOR(t)
     double r0 = 0.0, r1 = 0.0, r2 = (op == kFlatCV) ? 0.0 : INFINITY, r3 = -INFINITY;
-    for (int k = t; k < kChunkVox; k += kBlock) {
-        const int64_t v = v0 + k;
-        if (v >= n) break;
-        const bool m = V.wmask ? (V.wmask[v] != 0) : true;
-        if (!m) continue;
-        if (op == kFlatCV) {
-            const double u = (double)expm1f(a[v] - b[v]);
-            r0 += 1.0;
-            r1 += u;
-            r2 += u * u;
-        } else {
-            const double xv = (double)a[v];
-            if (op == kFlatSum) {
-                r0 += xv;
-                r1 += 1.0;
-            } else {
+    for (int k = t; k < kChunkVox && v0 + k < n; k += kFlatAhead * kBlock) {
+        float as[kFlatAhead], bs[kFlatAhead];
+        bool ms[kFlatAhead];
+        UNROLL for (int i = 0; i < kFlatAhead; ++i) {
+            const int64_t v = v0 + k + i * kBlock, w = v < n ? v : v0 + k;
+            as[i] = gp(a)[w];
+            bs[i] = op == kFlatCV ? gp(b)[w] : 0.0f;
+            ms[i] = (V.wmask ? gp(V.wmask)[w] != 0 : true) && v < n;
+        }
+        UNROLL for (int i = 0; i < kFlatAhead; ++i) {
+            if (!ms[i]) continue;
+            if (op == kFlatCV) {
+                const double u = (double)expm1f(as[i] - bs[i]);
                 r0 += 1.0;
-                r1 += 1.0;
+                r1 += u;
+                r2 += u * u;
+            } else {
+                const double xv = (double)as[i];
+                if (op == kFlatSum) {
+                    r0 += xv;
+                    r1 += 1.0;
+                } else {
+                    r0 += 1.0;
+                    r1 += 1.0;
+                }
+                r2 = fmin(r2, xv);
+                r3 = fmax(r3, xv);
             }
-            r2 = fmin(r2, xv);
-            r3 = fmax(r3, xv);
         }
     }
     red[t] = r0;
