@@ -63,7 +63,6 @@ static void dev_free(void* p) {
 #define H2D(dst, src, n, st) N4_CHECK_HIP(hipMemcpyAsync((dst), (src), (n), hipMemcpyHostToDevice, (hipStream_t)(st)))
 #define D2H(dst, src, n, st) N4_CHECK_HIP(hipMemcpyAsync((dst), (src), (n), hipMemcpyDeviceToHost, (hipStream_t)(st)))
 #define D2D(dst, src, n, st) N4_CHECK_HIP(hipMemcpyAsync((dst), (src), (n), hipMemcpyDeviceToDevice, (hipStream_t)(st)))
-#define DSET(dst, v, n, st) N4_CHECK_HIP(hipMemsetAsync((dst), (v), (n), (hipStream_t)(st)))
 #define SYNC(st) N4_CHECK_HIP(hipStreamSynchronize((hipStream_t)(st)))
 #define LAUNCH(expr)                                                                         \
     do {                                                                                     \
@@ -81,7 +80,6 @@ static void dev_free(void* p) { free(p); }
 #define H2D(dst, src, n, st) memcpy((dst), (src), (n))
 #define D2H(dst, src, n, st) memcpy((dst), (src), (n))
 #define D2D(dst, src, n, st) memcpy((dst), (src), (n))
-#define DSET(dst, v, n, st) memset((dst), (v), (n))
 #define SYNC(st) \
     do {         \
     } while (0)
@@ -2214,7 +2212,8 @@ done:
 // Flat stage plans reuse the engine's kernels on a 1-D array cut into
 // kChunkVox-voxel slabs.
 // hist: the histogram kernel will read x and m; it takes 16-byte loads of
-// aligned voxel quads, so the plan's own padded buffers get copies of them.
+// aligned voxel quads, so the min/max kernel copies them to the plan's own
+// padded buffers.
 // The flat kernels read x, m directly (m may be NULL: no mask).
 static n4_status flat_plan(n4_handle* h, uint64_t n, int nbins, Plan* P, const float* x, const uint8_t* m,
                            bool hist = false) {
@@ -2234,14 +2233,7 @@ static n4_status flat_plan(n4_handle* h, uint64_t n, int nbins, Plan* P, const f
     }
     memcpy(h->stage + P->off_desc, &D, sizeof D);
     s = stage_upload(h, P->base, 0, P->upload_bytes, nullptr);
-    if (s != N4_OK) return s;
-    if (hist) {
-        const size_t nw = (size_t)nslab * kChunkVox;
-        D2D(D.logU, x, sizeof(float) * n, nullptr);
-        D2D(D.wmask, m, n, nullptr);
-        DSET(D.wmask + n, 0, nw + kQuadPad - n, nullptr);
-    }
-    return N4_OK;
+    return s;
 }
 
 // Host-side reduction of the flat kernels' slab partials.
@@ -2256,10 +2248,12 @@ static n4_status read_partials(n4_handle* h, const Plan& P, std::vector<double>*
 // Min/max + histogram (+ Wiener E table) of a flat array: flat min/max
 // partials -> level 0 setup (mask count, cleared accumulators) -> hist ->
 // wiener.
-static n4_status flat_hist(n4_handle* h, const Plan& P, const float* d_x, RunParams rp, int32_t* d_bin_index) {
+static n4_status flat_hist(n4_handle* h, const Plan& P, const float* d_x, const uint8_t* d_mask, RunParams rp,
+                           int32_t* d_bin_index) {
     VolDesc* dd = dev_desc(h, P);
     Slab* sl = dev_wslab(h, P);
-    LAUNCH(launch_flat(dd, sl, P.n_wslab, kFlatMinMax, d_x, nullptr, nullptr, rp, nullptr));
+    LAUNCH(launch_flat(dd, sl, P.n_wslab, kFlatMinMax, d_x, reinterpret_cast<const float*>(d_mask), nullptr, rp,
+                       nullptr));
     LAUNCH(launch_level(dd, 1, 0, rp, nullptr));
     LAUNCH(launch_hist(dd, sl, P.n_wslab, -1, rp, d_bin_index, P.lds_hist, nullptr));
     return N4_OK;
@@ -2273,7 +2267,7 @@ n4_status n4_histogram(n4_handle* h, const float* d_x, const uint8_t* d_mask, ui
     Plan P;
     n4_status s = flat_plan(h, n, (int)nbins, &P, d_x, d_mask, true);
     if (s != N4_OK) return s;
-    s = flat_hist(h, P, d_x, P.rp, d_bin_index);
+    s = flat_hist(h, P, d_x, d_mask, P.rp, d_bin_index);
     if (s != N4_OK) return s;
     VolState st;
     D2H(&st, dev_state(h, P), sizeof st, nullptr);
@@ -2305,7 +2299,7 @@ n4_status n4_sharpen_image(n4_handle* h, const float* d_before, const uint8_t* d
     RunParams rp = P.rp;
     rp.noise = wiener_noise;
     rp.fwhm = fwhm;
-    s = flat_hist(h, P, d_before, rp, nullptr);
+    s = flat_hist(h, P, d_before, d_mask, rp, nullptr);
     if (s != N4_OK) return s;
     VolDesc* dd = dev_desc(h, P);
     Slab* sl = dev_wslab(h, P);

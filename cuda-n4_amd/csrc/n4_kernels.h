@@ -95,7 +95,9 @@ int launch_resident(const VolDesc* vols, int nvol, const int32_t* slots, int nsl
 
 // Flat (1-D) stage helpers used by the stage entry points.  A flat array of
 // n voxels is cut into slabs of kChunkVox voxels; each slab writes
-// spart[x] = 4 doubles (reduced on the host by the stage call).
+// spart[x] = 4 doubles (reduced on the host by the stage call).  kFlatMinMax
+// reads a under the uint8 mask b and copies both to logU and wmask, from
+// which the histogram takes aligned quads.
 enum FlatOp : int32_t { kFlatMinMax = 0, kFlatSum = 1, kFlatCV = 2, kFlatRemap = 3 };
 int launch_flat(const VolDesc* vols, const Slab* slabs, int nslab, int op, const float* a, const float* b,
                 float* out, RunParams rp, void* stream);

@@ -2286,6 +2286,8 @@ HD void body_flat(const VolDesc* vols, const Slab* slabs, int op, const float* a
     }
     BLOCK_FOR(t)
     double r0 = 0.0, r1 = 0.0, r2 = (op == kFlatCV) ? 0.0 : INFINITY, r3 = -INFINITY;
+    if (op == kFlatMinMax && v0 + kChunkVox >= n)  // the last slab: no mask behind the array
+        for (int64_t v = n + t; v < v0 + kChunkVox + kQuadPad; v += kBlock) V.wmask[v] = 0;
     for (int k = t; k < kChunkVox && v0 + k < n; k += kFlatAhead * kBlock) {
         float as[kFlatAhead], bs[kFlatAhead];
         bool ms[kFlatAhead];
@@ -2293,6 +2295,15 @@ HD void body_flat(const VolDesc* vols, const Slab* slabs, int op, const float* a
             const int64_t v = v0 + k + i * kBlock, w = v < n ? v : v0 + k;
             as[i] = gp(a)[w];
             bs[i] = op == kFlatCV ? gp(b)[w] : 0.0f;
+            if (op == kFlatMinMax) {  // (the mask comes in b)
+                const uint8_t m = gp(reinterpret_cast<const uint8_t*>(b))[w];
+                ms[i] = m && v < n;
+                if (v < n) {
+                    gp(V.logU)[v] = as[i];
+                    gp(V.wmask)[v] = m;
+                }
+                continue;
+            }
             ms[i] = (V.wmask ? gp(V.wmask)[w] != 0 : true) && v < n;
         }
         UNROLL for (int i = 0; i < kFlatAhead; ++i) {
