@@ -1321,7 +1321,6 @@ static bool plan_resident(const std::vector<VolIn>& in, const n4_params* p, cons
     if (resident_limits(&R->cus, &lds_cap) != 0 || R->cus < 1) return false;
     R->nchunk.assign(nv, 1);
     R->nbatch.assign(nv, 64);
-    const int per = std::max(1, env_int("N4_RES_UNITS", kResUnitsPerChunk));
     std::vector<double> want(nv);
     std::vector<int> strips(nv);
     for (int v = 0; v < nv; ++v) {
@@ -1345,7 +1344,7 @@ static bool plan_resident(const std::vector<VolIn>& in, const n4_params* p, cons
         R->nbatch[v] = D.res.nbatch;
         strips[v] = D.W[0] * strips_x;
         // about three quarters of a head volume's 16-row units hold foreground
-        want[v] = 0.75 * D.W[0] * ((D.W[1] + 15) / 16) / per;
+        want[v] = 0.75 * D.W[0] * ((D.W[1] + 15) / 16) / kResUnitsPerChunk;
     }
     // at most 1024 chunks: their partials are reduced by one workgroup
     std::vector<int> most(nv);

@@ -94,7 +94,7 @@ struct alignas(16) ResCtx {
     uint32_t red;   // [4 * kResWaves] doubles
     // union: set-up arrays | histogram copies | FFT | T1 slots (1 KB per unit
     // of a batch) | evaluation: a block of 16 x kResBr floats per wave
-    uint32_t u;
+    uint32_t u, ubytes;
     int32_t hc;     // histogram copies
     int32_t pzs, pys;
     // global buffers
@@ -194,6 +194,7 @@ HD size_t carve_res(const VolDesc& V, int nbins, int P, int prec, ResCtx* o) {
     um = um > 8 * hone ? um : 8 * hone;
     c.hc = um >= 32 * hone ? 32 : (um >= 16 * hone ? 16 : 8);
     c.u = take(um);
+    c.ubytes = (uint32_t)um;
     if (o) *o = c;
     return align16(off);
 }
@@ -861,6 +862,110 @@ N4_PHASE void res_hist(LdsP smem, double mn, double slope) {
     }
 }
 
+// Cuts of the chunks at strip boundaries that keep the largest chunk small,
+// where chunks hold few strips: cutting at equal tile counts leaves a chunk
+// up to a strip too large, and every phase waits for it (256 x 256 x 160
+// working voxels, 256 chunks of 3.6 strips: 119 tiles at most where 85 is
+// the mean, 100 the least possible).  Each wave fills chunks up to a limit
+// of its own, the smallest limit that suffices wins; the same in every
+// member.  Chunks of many strips are even as they are, and small ones gain
+// less than this costs (30 us), so they keep the equal counts (false).
+// After the scan of the slabs (pt, pu in the union).
+N4_PHASE bool res_even_cuts(const VolDesc* Vp, LdsP smem) {
+    const VolDesc& V = *uni(Vp);
+    const LdsP base = res_base(smem);
+    const CtxP C = res_ctx(base);
+    const int t = (int)threadIdx.x, wv = uni(t >> 6), lane = t & 63;
+    const int W0 = V.W[0], nch = V.res.nchunk, c0 = uni(C->c0), c1 = uni(C->c1), rows = V.wtile_rows;
+    N4_LDS int* pt = lds_at<int>(base, C->u);
+    N4_LDS int* pu = pt + W0 + 1;
+    const int T = uni(pt[W0]);
+    if (T < 32 * nch || sizeof(int) * (3 * (size_t)W0 + 4) > uni(C->ubytes)) return false;
+    N4_LDS int* ps = pu + W0 + 1;  // [W0 + 1] first strip of every slab, [1] the largest strip
+    N4_LDS int* st = ps + W0 + 2;
+    // strips of every slab
+    for (int x = t; x < W0; x += kResThreads) {
+        const int nu = pu[x + 1] - pu[x];
+        int n = 0, last = -1;
+        UNROLL_4 for (int k = 0; k < nu; ++k) {
+            const int strip = (int)(ld_agent(V.res.uent + (size_t)x * V.res.umax + k) & 0xffff) / rows;
+            n += strip != last;
+            last = strip;
+        }
+        ps[x] = n;
+    }
+    if (t == 0) ps[W0 + 1] = 0;
+    __syncthreads();
+    if (wv == 0) {
+        int sum = 0;
+        for (int x0 = 0; x0 < W0; x0 += 64) {
+            const int n = x0 + lane < W0 ? ps[x0 + lane] : 0;
+            int inc = n;
+            UNROLL for (int sh = 1; sh < 64; sh <<= 1) {
+                const int a = __shfl_up(inc, sh);
+                if (lane >= sh) inc += a;
+            }
+            if (x0 + lane < W0) ps[x0 + lane] = sum + inc - n;
+            sum += __shfl(inc, 63);
+        }
+        if (lane == 0) ps[W0] = sum;
+    }
+    __syncthreads();
+    const int ns = uni(ps[W0]);
+    // first tile and first unit of every strip, the waves' cuts and verdicts
+    N4_LDS int* su = st + ns + 1;
+    N4_LDS int* ok = su + ns + 1;
+    N4_LDS uint16_t* cut = reinterpret_cast<N4_LDS uint16_t*>(ok + kResWaves);
+    const size_t need = sizeof(int) * (size_t)(3 * W0 + 2 * ns + 6 + kResWaves) + sizeof(uint16_t) * kResWaves * (nch + 1);
+    if (ns >= 6 * nch || ns > 0xffff || need > uni(C->ubytes)) return false;
+    for (int x = t; x < W0; x += kResThreads) {
+        const int nu = pu[x + 1] - pu[x];
+        int s = ps[x], last = -1;
+        UNROLL_4 for (int k = 0; k < nu; ++k) {
+            const uint64_t e = ld_agent(V.res.uent + (size_t)x * V.res.umax + k);
+            const int strip = (int)(e & 0xffff) / rows;
+            if (strip != last) {
+                st[s] = pt[x] + (int)(e >> 48);
+                su[s] = pu[x] + k;
+                ++s;
+            }
+            last = strip;
+        }
+    }
+    if (t == 0) {
+        st[ns] = T;
+        su[ns] = pu[W0];
+    }
+    __syncthreads();
+    for (int i = t; i < ns; i += kResThreads)
+        __hip_atomic_fetch_max(ps + W0 + 1, st[i + 1] - st[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __syncthreads();
+    const int limit = (T + nch - 1) / nch + uni(ps[W0 + 1]) * (wv + 1) / kResWaves;
+    N4_LDS uint16_t* my = cut + wv * (nch + 1);
+    int s = 0, k = 0;
+    for (; k < nch && s < ns; ++k) {
+        if (lane == 0) my[k] = (uint16_t)s;
+        const int i = s + lane;
+        const unsigned long long fit = __ballot(i < ns && st[i < ns ? i + 1 : ns] - st[s] <= limit);
+        const int n = __popcll(fit);
+        if (n == 0) break;
+        s += n;
+    }
+    if (lane == 0) ok[wv] = s >= ns;
+    for (int i = k + lane; i <= nch; i += 64) my[i] = (uint16_t)ns;
+    __syncthreads();
+    int w = 0;
+    while (w < kResWaves && !uni(ok[w])) ++w;
+    if (w == kResWaves) return false;
+    N4_LDS int* cb = lds_at<int>(base, C->cb);
+    for (int b = c0 + t; b <= c1; b += kResThreads) {
+        const int i = cut[w * (nch + 1) + b];
+        cb[2 * (b - c0)] = su[i];
+        cb[2 * (b - c0) + 1] = st[i];
+    }
+    return true;
+}
+
 // Set-up of a volume: every slab's units (rows of foreground, z ranges) by
 // the team's members in turn, the split of the units over the chunks, and
 // the packed copy of the own chunks' voxels.  Returns false if the team gave
@@ -976,8 +1081,9 @@ N4_PHASE bool res_setup(const VolDesc* Vp, LdsP smem) {
     }
     __syncthreads();
     const int T = pt[W0], nch = V.res.nchunk;
-    // chunk c starts at the first strip whose first tile is >= T c / nchunk
-    for (int b = c0 + wv; b <= c1; b += kResWaves) {
+    const bool even = res_even_cuts(Vp, smem);
+    // else chunk c starts at the first strip whose first tile is >= T c / nchunk
+    for (int b = c0 + wv; b <= c1 && !even; b += kResWaves) {
         const int target = (int)((int64_t)T * b / nch);
         int fu = uni(pu[W0]), ft = T;
         if (target < T) {
