@@ -1305,14 +1305,14 @@ static bool plan_teams(const std::vector<VolIn>& in, const n4_params* p, const S
 // factor tables, lattice increment and one batch of units share a compute
 // unit's LDS, and the unit entries hold 16-bit positions.
 // Chunks: a workgroup per kResUnitsPerChunk units (below that a workgroup's
-// share of the per-iteration chain outweighs its work), scaled down in
-// proportion to the volumes' sizes when the batch asks for more workgroups
-// than the device has compute units.
+// share of the per-iteration chain outweighs its work; 2, 3, 5, 6 and 8 units
+// measured 0 to 4% slower on 64 x 64 x 44 and 256 x 256 x 160 FP32), fewer
+// when the batch asks for more workgroups than the device has compute units.
 // The resident kernel runs wherever it covers the call.  Measured against the
-// step kernels (five launches a step), whole calls: 64^3 FP32 2.30 -> 1.62
-// ms, 256x256x176 at shrink 4 FP32 2.63 -> 2.03, 512x512x320 at shrink 2 BF16
-// 4.91 -> 3.65, 12 mixed volumes split BF16 5.40 -> 3.52, 64 volumes at
-// shrink 4 BF16 7.70 -> 7.62.
+// step kernels (five launches a step), whole calls: 64 x 64 x 44
+// FP32 2.70 -> 1.83 ms, 256 x 256 x 176 at shrink 4 FP32 2.89 -> 2.12, 512 x
+// 512 x 320 at shrink 2 BF16 4.72 -> 3.44, 12 mixed volumes split BF16 5.54
+// -> 3.25, 64 volumes at shrink 4 BF16 8.06 -> 5.78.
 #ifndef N4_EMULATE
 static bool plan_resident(const std::vector<VolIn>& in, const n4_params* p, const Schedule& sch, ResPlan* R) {
     const int nv = (int)in.size(), L = (int)p->number_of_fitting_levels;

@@ -50,7 +50,7 @@
 
 namespace n4 {
 
-constexpr int kResThreads = 1024;
+constexpr int kResThreads = kResBlock;
 constexpr int kResWaves = kResThreads / 64;
 constexpr int kResBr = 20;  // row stride of a wave's y-contracted block (16-byte rows, distinct banks)
 constexpr uint32_t kResClosed = 0x80000000u;
@@ -216,35 +216,73 @@ struct ResTimer {
     }
 };
 
+// What the Wiener step needs besides the histogram -- the Gaussian and the
+// twiddles -- laid into its buffers by the waves that have nothing to do
+// while the first polls the barrier of the complete histogram.
+template <int P>
+__device__ inline void res_wiener_ready_p(LdsP u, const RunParams& rp, double slope) {
+    constexpr bool PAD = fft_pad(P);
+    const WienerLds L = carve_wiener<P, PAD>(u);
+    const WienerGauss G = wiener_gauss(rp, slope);
+    for (int j = (int)threadIdx.x - 64; j < P; j += kResThreads - 64) {
+        L.tw[fft_at<PAD>(j)] = rp.twiddle[j];
+        L.z[fft_at<PAD>(j)].y = wiener_gauss_at<P>(G, j);
+    }
+}
+__device__ inline void res_wiener_ready(LdsP base, double slope) {
+    const CtxP C = res_ctx(base);
+    RunParams rp;
+    rp.fwhm = C->fwhm;
+    rp.twiddle = uni(C->twiddle);
+    const LdsP u = lds_at<unsigned char>(base, C->u);
+    switch (uni(C->P)) {
+        case 4: res_wiener_ready_p<4>(u, rp, slope); break;
+        case 8: res_wiener_ready_p<8>(u, rp, slope); break;
+        case 16: res_wiener_ready_p<16>(u, rp, slope); break;
+        case 32: res_wiener_ready_p<32>(u, rp, slope); break;
+        case 64: res_wiener_ready_p<64>(u, rp, slope); break;
+        case 128: res_wiener_ready_p<128>(u, rp, slope); break;
+        case 256: res_wiener_ready_p<256>(u, rp, slope); break;
+        case 512: res_wiener_ready_p<512>(u, rp, slope); break;
+        default: res_wiener_ready_p<1024>(u, rp, slope); break;
+    }
+}
+
+
 // Team barrier number gen + 1 (see team_barrier): bounded, false once the
 // team has given up.
-N4_PHASE bool res_barrier(uint32_t* team_, int m_, uint32_t gen, LdsP smem) {
+template <bool WIENER>
+N4_PHASE bool res_barrier_t(uint32_t* team_, int m_, uint32_t gen, LdsP smem, double slope) {
     uint32_t* team = uni(team_);
     const int m = uni(m_);
-    N4_LDS int* bc = reinterpret_cast<N4_LDS int*>(res_base(smem));
+    const LdsP base = res_base(smem);
+    N4_LDS int* bc = reinterpret_cast<N4_LDS int*>(base);
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __builtin_amdgcn_s_waitcnt(0);
     __atomic_signal_fence(__ATOMIC_SEQ_CST);
     __syncthreads();
-    if (m > 1) {
-        if (threadIdx.x == 0) {
-            int ok = 1;
-            __hip_atomic_fetch_add(team + kRwBarrier, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            const uint32_t target = (gen + 1u) * (uint32_t)m;
-            for (uint32_t spins = 1; ld_agent(team + kRwBarrier) < target; ++spins) {
-                __builtin_amdgcn_s_sleep(1);
-                if ((spins & 63u) == 0 && (spins > kSpinLimit || ld_agent(team + kRwAbort) != 0)) {
-                    ok = 0;
-                    break;
-                }
+    int ok = 1;
+    if (m > 1 && threadIdx.x == 0)
+        __hip_atomic_fetch_add(team + kRwBarrier, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (WIENER && threadIdx.x >= 64) res_wiener_ready(base, slope);
+    if (m > 1 && threadIdx.x == 0) {
+        const uint32_t target = (gen + 1u) * (uint32_t)m;
+        for (uint32_t spins = 1; ld_agent(team + kRwBarrier) < target; ++spins) {
+            __builtin_amdgcn_s_sleep(1);
+            if ((spins & 63u) == 0 && (spins > kSpinLimit || ld_agent(team + kRwAbort) != 0)) {
+                ok = 0;
+                break;
             }
-            if (!ok) st_agent(team + kRwAbort, 1u);
-            bc[0] = ok;
         }
-        __syncthreads();
-        return uni(bc[0]) != 0;
+        if (!ok) st_agent(team + kRwAbort, 1u);
+        bc[0] = ok;
     }
-    return true;
+    if (m == 1 && !WIENER) return true;
+    __syncthreads();
+    return m == 1 || uni(bc[0]) != 0;
+}
+__device__ inline bool res_barrier(uint32_t* team, int m, uint32_t gen, LdsP smem) {
+    return res_barrier_t<false>(team, m, gen, smem, 0.0);
 }
 
 // Joins the team of a volume with n chunks: rank (>= 0; the team's
@@ -1509,7 +1547,8 @@ __device__ bool res_volume(const VolDesc& V, const RunParams& rp, int rank, int 
         res_clear_numerator(smem, false);
         if (!degenerate) res_hist(smem, mn, slope);
         pt.mark(kPhHist);
-        if (!res_barrier(team, m, gen++, smem)) return false;
+        if (!(degenerate ? res_barrier(team, m, gen, smem) : res_barrier_t<true>(team, m, gen, smem, slope))) return false;
+        ++gen;
         pt.mark(kPhWait);
         if (!degenerate) res_wiener(&V, smem, mn, slope);
         pt.mark(kPhWiener);
