@@ -1306,10 +1306,10 @@ static bool plan_teams(const std::vector<VolIn>& in, const n4_params* p, const S
 // unit's LDS, and the unit entries hold 16-bit positions.
 // Chunks: a workgroup per kResUnitsPerChunk units (below that a workgroup's
 // share of the per-iteration chain outweighs its work; 2, 3, 5, 6 and 8 units
-// measured 0 to 4% slower on 64 x 64 x 44 and 256 x 256 x 160 FP32), fewer
+// measured 0 to 4% slower on 64 x 64 x 64 and, at shrink 4, 256 x 256 x 176 FP32), fewer
 // when the batch asks for more workgroups than the device has compute units.
 // The resident kernel runs wherever it covers the call.  Measured against the
-// step kernels (five launches a step), whole calls: 64 x 64 x 44
+// step kernels (five launches a step), whole calls: 64 x 64 x 64
 // FP32 2.70 -> 1.83 ms, 256 x 256 x 176 at shrink 4 FP32 2.89 -> 2.12, 512 x
 // 512 x 320 at shrink 2 BF16 4.72 -> 3.44, 12 mixed volumes split BF16 5.54
 // -> 3.25, 64 volumes at shrink 4 BF16 8.06 -> 5.78.

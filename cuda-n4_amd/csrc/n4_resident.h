@@ -6,8 +6,8 @@
 // and meet at three team barriers per iteration (range of logU known;
 // histogram complete; fit numerator complete), in place of five launches.
 //
-// What bounds it: the chain of one iteration -- three barriers, the FP64
-// Wiener step, and per phase one round trip to L2 -- and, for large volumes,
+// What bounds it: the chain of one iteration -- three barriers (2.2 us each),
+// the FP64 Wiener step (7.6 us), and per phase one round trip to L2 -- and, for large volumes,
 // the vector work per foreground voxel.  So
 //  * only the foreground is worked on: a strip (the row tile of a slab that
 //    the step kernels give one workgroup) is cut into units of 16 rows, each
@@ -218,7 +218,8 @@ struct ResTimer {
 
 // What the Wiener step needs besides the histogram -- the Gaussian and the
 // twiddles -- laid into its buffers by the waves that have nothing to do
-// while the first polls the barrier of the complete histogram.
+// while the first polls the barrier of the complete histogram (Wiener step
+// 8.25 -> 7.6 us).
 template <int P>
 __device__ inline void res_wiener_ready_p(LdsP u, const RunParams& rp, double slope) {
     constexpr bool PAD = fft_pad(P);
@@ -444,7 +445,7 @@ __device__ inline int res_batch_len(CtxP C, int ub, int u1) {
 // last bin on the entry itself comes back as fma(0, ., E)).  on: all ones
 // where the voxel counts, else 0; as a bit mask it keeps the table reads of
 // all voxels in flight (a select becomes a branch around each read, with a
-// wait of its own; FP32, 256 x 256 x 160: 2.17 against 2.19 ms).
+// wait of its own; FP32, 256 x 256 x 176 at shrink 4: 2.17 against 2.19 ms).
 template <bool DEN>
 __device__ inline float res_input(int on, float xv, const Remap& R, const N4_LDS float* Ed) {
     if constexpr (DEN) return __int_as_float(on & __float_as_int(1.0f));

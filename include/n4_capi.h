@@ -136,10 +136,11 @@ n4_status n4_correct(n4_handle *h, const float *d_im, const void *d_mask,
  * buffers live in a file-scope device array of 64 MiB per device (held
  * until the process ends) instead of the handle's arena, so the working
  * grid is limited (about 6.5 M working voxels at the default parameters);
- * larger requests fail with N4_ERR_NO_MEMORY.  It runs the step kernels on
- * `stream` with every step enqueued up front (no progress words in pinned
- * memory, no events, no graph instantiation; kernel timing is ignored) and
- * returns after the work completes.  Calls that overlap on one device race
+ * larger requests fail with N4_ERR_NO_MEMORY.  It runs on
+ * `stream` (the resident kernel, or where that is not used or does not fit,
+ * the step kernels with every step enqueued up front; no progress words in
+ * pinned memory, no events, no graph instantiation; kernel timing is ignored)
+ * and returns after the work completes.  Calls that overlap on one device race
  * on the shared array.  Call on the handle's device. */
 n4_status n4_correct_noalloc(n4_handle *h, const float *d_im, const void *d_mask,
                              uint32_t mask_kind, uint32_t fx, uint32_t fy, uint32_t fz,
