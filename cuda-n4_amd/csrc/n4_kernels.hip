@@ -2090,7 +2090,11 @@ HD void store_run4(float* p, const F4& x) {
 // the column's factors and the image quads of its first rows.  On the
 // device they are loaded in the set-up round of the tile, before the
 // barriers.
-constexpr int kReconRows = 4;  // rows in flight
+// Rows in flight: with more, the resident kernel's instance (128 registers)
+// spills and its idle workgroups reconstruct the slower -- 64-volume batch
+// with 4 / 2 / 1 rows 5.55 / 5.24 / 5.06 ms, 512 x 512 x 320 and the
+// reconstruction launch alone unchanged from 2 to 1.
+constexpr int kReconRows = 1;
 struct ReconThread {
     int cols, nr, r0, q0;
     ReconCol c;
