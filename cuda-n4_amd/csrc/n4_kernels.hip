@@ -2020,8 +2020,8 @@ HD void body_eval(const VolDesc* vols, const Slab* slabs, RunParams rp, int bid,
 // reads and 20 FMAs.  (With voxels dealt to the lanes one by one -- a
 // division by the row length, 4 z factors and 4 row values from LDS each --
 // the kernel was bound by vector instructions: 64 volumes of 652 M voxels
-// 2010 us, 3.9 TB/s, now 1497 us, 5.2 TB/s; 512x512x320 260 -> 196 us;
-// 256x256x176, field only, 23.8 -> 21.4 us.)
+// 2010 us, 3.9 TB/s, so 1497 us, 5.2 TB/s; 512x512x320 260 -> 196 us;
+// 256x256x176, field only, 23.8 -> 21.4 us, with four rows in flight.)
 struct ReconLds {
     N4_LDS float* A;
     N4_LDS float* B;
