@@ -98,6 +98,26 @@ HD void sincospi_d(double x, double* s, double* c) {
 #endif
 }
 
+// float -> BF16 bits, round to nearest even (finite inputs).
+HD unsigned short bf16_rn(float f) {
+    uint32_t u;
+    memcpy(&u, &f, sizeof u);
+    u += 0x7fffu + ((u >> 16) & 1u);
+    return (unsigned short)(u >> 16);
+}
+HD float bf16_to_f32(unsigned short h) {
+    const uint32_t u = (uint32_t)h << 16;
+    float f;
+    memcpy(&f, &u, sizeof f);
+    return f;
+}
+
+// f ~= hi + lo with both halves BF16.
+HD void bf16_split(float f, unsigned short& hi, unsigned short& lo) {
+    hi = bf16_rn(f);
+    lo = bf16_rn(f - bf16_to_f32(hi));
+}
+
 HD size_t align16(size_t v) { return (v + 15) & ~size_t(15); }
 
 // Global-memory view of a descriptor pointer.  A pointer loaded from a
@@ -2913,9 +2933,7 @@ HD void body_persist(const VolDesc* vols, const Slab* slabs, const PWork* work, 
 
 }  // namespace n4
 
-#ifndef N4_EMULATE
 #include "n4_resident.h"
-#endif
 
 namespace n4 {
 
@@ -3432,6 +3450,41 @@ extern "C" int n4emu_remap_residual(const float* x, const uint8_t* m, int64_t n,
     const n4::Remap rm = n4::make_remap(Ef, bmin, slope, nb);
     for (int64_t i = 0; i < n; ++i) out[i] = n4::fit_input(n4::kFitNum, m[i], x[i], degenerate != 0, rm);
     return 0;
+}
+
+// Test hook of the emulation build only: the LDS of the resident kernel for
+// one level of an 8 x Y x Z working grid, with its factor tables filled
+// (kf as res_tables) over whatever lds (cap bytes) holds.  off: byte offsets
+// of zw, zb, wy, pz, pzl, py, pyl, then the row lengths pzs, pys.  Returns
+// the LDS size; the CPU tests check every entry that the kernel reads.
+extern "C" int64_t n4emu_resident_tables(const n4::AxisEntry* axy, int Y, const n4::AxisEntry* axz, int Z, int ncp,
+                                         int prec, int kf, unsigned char* lds, int64_t cap, uint32_t* off) {
+    using namespace n4;
+    VolDesc V;
+    memset(&V, 0, sizeof V);
+    V.W[0] = 8;
+    V.W[1] = Y;
+    V.W[2] = Z;
+    V.nlevels = 1;
+    V.lev[0].L = 4 * ncp * ncp;
+    V.res.nchunk = 1;
+    V.res.nbatch = 64;
+    ResCtx c;
+    memset(&c, 0, sizeof c);
+    const size_t n = carve_res(V, 200, 512, prec, &c);
+    if ((int64_t)n > cap) return -1;
+    c.Y = Y;
+    c.Z = Z;
+    c.ax[1] = axy;
+    c.ax[2] = axz;
+    memcpy(lds + kResBcBytes, &c, sizeof c);
+    if (prec == 0)
+        res_tables<0>(lds, kf);
+    else
+        res_tables<1>(lds, kf);
+    const uint32_t o[9] = {c.zw, c.zb, c.wy, c.pz, c.pzl, c.py, c.pyl, (uint32_t)c.pzs, (uint32_t)c.pys};
+    memcpy(off, o, sizeof o);
+    return (int64_t)n;
 }
 
 namespace n4 {

@@ -32,20 +32,6 @@ typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-// float -> BF16 bits, round to nearest even (finite inputs).
-__device__ inline unsigned short bf16_rn(float f) {
-    uint32_t u = __float_as_uint(f);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (unsigned short)(u >> 16);
-}
-__device__ inline float bf16_to_f32(unsigned short h) { return __uint_as_float((uint32_t)h << 16); }
-
-// f ~= hi + lo with both halves BF16.
-__device__ inline void bf16_split(float f, unsigned short& hi, unsigned short& lo) {
-    hi = bf16_rn(f);
-    lo = bf16_rn(f - bf16_to_f32(hi));
-}
-
 __device__ inline f32x4 mma_k32(u16x8 a, u16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c,
                                                    0, 0, 0);

@@ -1,5 +1,6 @@
 // n4_resident.h -- the whole level/iteration loop of a correction in one
-// launch (device build only; included by n4_kernels.hip).
+// launch (included by n4_kernels.hip; the host emulation build takes the LDS
+// layout and the factor tables only).
 //
 // One workgroup of 1024 threads per compute unit.  A volume is worked on by
 // a team of workgroups that stay on it from its first iteration to its last
@@ -57,6 +58,7 @@ constexpr uint32_t kResClosed = 0x80000000u;
 constexpr uint64_t kResJoinTicks = 20000;  // 100 MHz clock: 200 us
 
 #define N4_PHASE __device__ __attribute__((noinline))
+#define N4_PHASE_HD __host__ __device__ __attribute__((noinline))
 
 // One unit of the current batch in LDS, with its slab's x factors.
 struct alignas(16) ResLUnit {
@@ -128,19 +130,31 @@ struct alignas(16) ResCtx {
 typedef const N4_LDS ResCtx* CtxP;
 typedef N4_LDS unsigned char* LdsP;
 
-__device__ inline int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-__device__ inline uint32_t uni(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+HD uint32_t uni(uint32_t v) {
+#ifdef N4_DEVICE_PASS
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+#else
+    return v;
+#endif
+}
+HD int uni(int v) { return (int)uni((uint32_t)v); }
 template <class T>
-__device__ inline T* uni(T* p) {
+HD T* uni(T* p) {
     const uint64_t v = (uint64_t)p;
     return (T*)((uint64_t)uni((uint32_t)v) | ((uint64_t)uni((uint32_t)(v >> 32)) << 32));
 }
 // LDS base and context of a phase function (its arguments arrive in vector
 // registers).
-__device__ inline LdsP res_base(LdsP smem) { return (LdsP)(uintptr_t)uni((uint32_t)(uintptr_t)smem); }
-__device__ inline CtxP res_ctx(LdsP base) { return reinterpret_cast<CtxP>(base + kResBcBytes); }
+HD LdsP res_base(LdsP smem) {
+#ifdef N4_DEVICE_PASS
+    return (LdsP)(uintptr_t)uni((uint32_t)(uintptr_t)smem);
+#else
+    return smem;
+#endif
+}
+HD CtxP res_ctx(LdsP base) { return reinterpret_cast<CtxP>(base + kResBcBytes); }
 template <class T>
-__device__ inline N4_LDS T* lds_at(LdsP base, uint32_t off) {
+HD N4_LDS T* lds_at(LdsP base, uint32_t off) {
     return reinterpret_cast<N4_LDS T*>(base + uni(off));
 }
 
@@ -198,6 +212,77 @@ HD size_t carve_res(const VolDesc& V, int nbins, int P, int prec, ResCtx* o) {
     if (o) *o = c;
     return align16(off);
 }
+
+// Factor tables of a level (kf 2: w^2 for the denominator, 1: w^3/sum w^2
+// and the evaluation factors): one position per thread, zeros outside the
+// position's 4-point support and past the grid.
+template <int PREC>
+N4_PHASE_HD void res_tables(LdsP smem, int kf) {
+    const LdsP base = res_base(smem);
+    const CtxP C = res_ctx(base);
+    const int Y = uni(C->Y), Z = uni(C->Z), pzs = uni(C->pzs), pys = uni(C->pys);
+    const AxisEntry* axz = uni(C->ax[2]);
+    const AxisEntry* axy = uni(C->ax[1]);
+    N4_LDS float* zw = lds_at<float>(base, C->zw);
+    N4_LDS int* zb = lds_at<int>(base, C->zb);
+    N4_LDS float* wy = lds_at<float>(base, C->wy);
+    // positions the tables hold (past the grid: zeros): the evaluation's go 16
+    // past the grid, where a unit's last tile or block of rows may reach, the
+    // fit's to the end of their rows
+    const int fz = PREC == 0 ? 4 * pzs : pzs, fy = PREC == 0 ? 4 * pys : pys;
+    const int npz = fz > Z + 16 ? fz : Z + 16, npy = fy > Y + 16 ? fy : Y + 16;
+    BLOCK_FOR_N(t, kResThreads)
+    for (int e = t; e < npz + npy; e += kResThreads) {
+        const bool isz = e < npz;
+        const int pos = isz ? e : e - npz;
+        const int n = isz ? Z : Y;
+        const int st = isz ? pzs : pys;
+        const uint32_t tab = isz ? C->pz : C->py, tabl = isz ? C->pzl : C->pyl;
+        const AxisEntry* ax = isz ? axz : axy;
+        float f[4] = {0.0f, 0.0f, 0.0f, 0.0f}, w[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        int b = 0;
+        if (pos < n) {
+            const AxisEntry& a = ax[pos];
+            b = a.b;
+            UNROLL for (int k = 0; k < 4; ++k) {
+                f[k] = kf == 2 ? a.q[k] : a.p[k];
+                w[k] = a.w[k];
+            }
+        }
+        const bool ev = kf != 2 && pos < n + 16, fit = pos < (isz ? fz : fy);
+        if (ev && isz) {
+            // the factors of row z in the association of eval_chunks (see res_eval);
+            // past the grid zeros, in the last span
+            UNROLL for (int k = 0; k < 4; ++k) zw[4 * pos + k] = w[k < 2 ? 1 - k : k];
+            zb[pos] = pos < n ? b : axz[n - 1].b;
+        }
+        for (int c = 0; c < 16; ++c) {
+            const int k = c - b;
+            float fv = 0.0f, wv = 0.0f;
+            UNROLL for (int a = 0; a < 4; ++a)
+                if (k == a) {
+                    fv = f[a];
+                    wv = w[a];
+                }
+            if (!fit) {
+            } else if constexpr (PREC == 0) {
+                lds_at<float>(base, 0)[tab / 4 + (4 * c + (pos & 3)) * st + (pos >> 2)] = fv;
+            } else {
+                unsigned short h, l;
+                bf16_split(fv, h, l);
+                lds_at<unsigned short>(base, 0)[tab / 2 + c * st + pos] = h;
+                lds_at<unsigned short>(base, 0)[tabl / 2 + c * st + pos] = l;
+            }
+            if (ev && !isz) wy[pos * 16 + 4 * (c & 3) + (c >> 2)] = wv;
+        }
+    }
+    BLOCK_END
+}
+
+}  // namespace n4
+
+#ifndef N4_EMULATE
+namespace n4 {
 
 __device__ inline f32x4 mma_f32(float a, float b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
@@ -323,66 +408,6 @@ N4_PHASE int res_join(uint32_t* team, int n, LdsP smem) {
     }
     __syncthreads();
     return uni(bc[1]);
-}
-
-// Factor tables of a level (kf 2: w^2 for the denominator, 1: w^3/sum w^2
-// and the evaluation factors): one position per thread, zeros outside the
-// position's 4-point support and past the grid.
-template <int PREC>
-N4_PHASE void res_tables(LdsP smem, int kf) {
-    const LdsP base = res_base(smem);
-    const CtxP C = res_ctx(base);
-    const int Y = uni(C->Y), Z = uni(C->Z), pzs = uni(C->pzs), pys = uni(C->pys);
-    const AxisEntry* axz = uni(C->ax[2]);
-    const AxisEntry* axy = uni(C->ax[1]);
-    N4_LDS float* zw = lds_at<float>(base, C->zw);
-    N4_LDS int* zb = lds_at<int>(base, C->zb);
-    N4_LDS float* wy = lds_at<float>(base, C->wy);
-    // positions the tables hold (past the grid: zeros)
-    const int npz = PREC == 0 ? 4 * pzs : pzs, npy = PREC == 0 ? 4 * pys : pys;
-    for (int e = (int)threadIdx.x; e < npz + npy; e += kResThreads) {
-        const bool isz = e < npz;
-        const int pos = isz ? e : e - npz;
-        const int n = isz ? Z : Y;
-        const int st = isz ? pzs : pys;
-        const uint32_t tab = isz ? C->pz : C->py, tabl = isz ? C->pzl : C->pyl;
-        const AxisEntry* ax = isz ? axz : axy;
-        float f[4] = {0.0f, 0.0f, 0.0f, 0.0f}, w[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        int b = 0;
-        if (pos < n) {
-            const AxisEntry& a = ax[pos];
-            b = a.b;
-            UNROLL for (int k = 0; k < 4; ++k) {
-                f[k] = kf == 2 ? a.q[k] : a.p[k];
-                w[k] = a.w[k];
-            }
-        }
-        const bool ev = kf != 2 && pos < n + 16;
-        if (ev && isz) {
-            // the factors of row z in the association of eval_chunks (see res_eval);
-            // past the grid zeros, in the last span
-            UNROLL for (int k = 0; k < 4; ++k) zw[4 * pos + k] = w[k < 2 ? 1 - k : k];
-            zb[pos] = pos < n ? b : axz[n - 1].b;
-        }
-        for (int c = 0; c < 16; ++c) {
-            const int k = c - b;
-            float fv = 0.0f, wv = 0.0f;
-            UNROLL for (int a = 0; a < 4; ++a)
-                if (k == a) {
-                    fv = f[a];
-                    wv = w[a];
-                }
-            if constexpr (PREC == 0) {
-                lds_at<float>(base, 0)[tab / 4 + (4 * c + (pos & 3)) * st + (pos >> 2)] = fv;
-            } else {
-                unsigned short h, l;
-                bf16_split(fv, h, l);
-                lds_at<unsigned short>(base, 0)[tab / 2 + c * st + pos] = h;
-                lds_at<unsigned short>(base, 0)[tabl / 2 + c * st + pos] = l;
-            }
-            if (ev && !isz) wy[pos * 16 + 4 * (c & 3) + (c >> 2)] = wv;
-        }
-    }
 }
 
 // Units [ub, ub + n) of the volume's list (whole strips, n <= 64) into LDS,
@@ -1568,3 +1593,4 @@ __device__ bool res_volume(const VolDesc& V, const RunParams& rp, int rank, int 
 }
 
 }  // namespace n4
+#endif

@@ -103,3 +103,21 @@ def test_covered_up_to_16_control_points_then_steps(gpu):
     finally:
         gpu.set_tuning(reset=True)
     assert np.array_equal(a[0]["log_bias"], b[0]["log_bias"])
+
+
+def _box(dims, z0, seed):
+    """Tissue that the end of the field of view cuts off: foreground from z0
+    to the last z, rows of several lengths."""
+    rng = np.random.default_rng(seed)
+    x, y, z = np.meshgrid(*(np.linspace(-1, 1, n) for n in dims), indexing="ij")
+    im = np.where(x * x + y * y < 0.5, 200.0, 100.0) * np.exp(0.2 * (z + x * y)) + rng.normal(0, 4, dims)
+    m = np.zeros(dims, np.uint8)
+    m[1:-1, :, z0:] = 1
+    m[:, dims[1] // 2:, :z0 + 4] = 0
+    return im.astype(np.float32), m
+
+
+@pytest.mark.parametrize("precision", ["fp32", "bf16", "split_bf16"])
+@pytest.mark.parametrize("nz,z0", [(29, 12), (31, 12), (32, 12), (32, 28), (64, 12), (64, 28), (61, 44), (96, 76)])
+def test_foreground_to_the_last_z(gpu, precision, nz, z0):
+    _both(gpu, [_box((9, 37, nz), z0, nz)], levels=3, max_iter=[3, 3, 2], fixed_iterations=True, precision=precision)
