@@ -1646,7 +1646,7 @@ HD void body_fit(const VolDesc* vols, const Slab* slabs, int level, int it, int 
 // passes of the step's slab kernel over padded copies, one workgroup of 256
 // threads per slab, took 2 x 116 us at 256 x 256 x 160 besides the copies;
 // this takes 25.3 us, the read alone about 13.
-constexpr int kFieldCols = kBlock;  // columns of one z chunk
+constexpr int kFieldCols = kBlock;  // columns of one z chunk, at most
 constexpr int kFieldSpans = 6;      // rows of Q (control points) of one row batch
 constexpr int kFieldRowsMax = 64;   // rows of a tile
 constexpr int kFieldAhead = 8;      // rows in flight per thread (16: 27.3 against 26.0 us)
@@ -1661,6 +1661,13 @@ struct FieldLds {
     N4_LDS int* cz;    // support [lo, hi) of the chunk's control points
     N4_LDS float* Q;   // [part][numerator, denominator][cy][column]
 };
+// Columns of one z chunk: as many as reach at most kFieldCols + 3 control
+// points (n columns reach less than (n - 1) (Cz - 3) / Z + 5), so that the
+// chunk's table of them fits; 256 unless spans are shorter than a voxel.
+HD int field_cols(int Z, int Cz) {
+    const int64_t n = 1 + (int64_t)(kFieldCols - 2) * Z / (Cz - 3);
+    return n < kFieldCols ? (int)n : kFieldCols;
+}
 HD size_t carve_field(N4_LDS unsigned char* base, FieldLds* o) {
     Carve c{base, 0};
     FieldLds L;
@@ -1702,8 +1709,9 @@ HD void body_field_fit(const VolDesc* vols, int bid, N4_LDS unsigned char* smem)
     BLOCK_END
     BLOCK_SYNC();
     const int bt = S.yb[0], ncy = S.yb[ny - 1] - bt + 4;  // control points of the tile along y
-    for (int z0 = 0; z0 < Z; z0 += kFieldCols) {
-        const int nz = Z - z0 < kFieldCols ? Z - z0 : kFieldCols;
+    const int cols = field_cols(Z, Cz);
+    for (int z0 = 0; z0 < Z; z0 += cols) {
+        const int nz = Z - z0 < cols ? Z - z0 : cols;
         const int parts = kBlock / nz;  // runs of rows walked side by side
         for (int y0 = 0, y1; y0 < ny; y0 = y1) {
             // a batch of rows whose control points fit Q
