@@ -44,7 +44,7 @@ def test_gpu(gpu, dims, ncpt, fill):
 # More control points between a chunk's first and last column than it has
 # columns.
 MANY = [((2, 3, 100), (4, 4, 300)), ((2, 2, 256), (4, 4, 400)), ((3, 2, 300), (4, 4, 303)), ((2, 5, 259), (4, 6, 520)),
-        ((2, 2, 513), (4, 4, 517)), ((2, 70, 300), (4, 5, 310))]
+        ((2, 2, 513), (4, 4, 517)), ((2, 7, 300), (4, 5, 310))]
 
 
 @pytest.mark.parametrize("dims,ncpt", MANY)
