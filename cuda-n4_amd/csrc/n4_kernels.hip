@@ -1658,7 +1658,7 @@ struct FieldLds {
     N4_LDS float* zp;  // [columns][4]
     N4_LDS float* zq;
     N4_LDS int* zb;
-    N4_LDS int* cz;    // support [lo, hi) of the chunk's control points
+    N4_LDS int* cz;    // first column of each of the chunk's spans (empty ones among them), and the end
     N4_LDS float* Q;   // [part][numerator, denominator][cy][column]
 };
 // Columns of one z chunk: as many as reach at most kFieldCols + 3 control
@@ -1678,7 +1678,7 @@ HD size_t carve_field(N4_LDS unsigned char* base, FieldLds* o) {
     L.zp = c.take<float>(4 * kFieldCols);
     L.zq = c.take<float>(4 * kFieldCols);
     L.zb = c.take<int>(kFieldCols);
-    L.cz = c.take<int>(2 * (kFieldCols + 3));
+    L.cz = c.take<int>(kFieldCols + 3);
     L.Q = c.take<float>(2 * kFieldSpans * kFieldCols);
     if (o) *o = L;
     return align16(c.off);
@@ -1728,9 +1728,11 @@ HD void body_field_fit(const VolDesc* vols, int bid, N4_LDS unsigned char* smem)
                         S.zq[4 * t + k] = a.q[k];
                     }
                     S.zb[t] = a.b;
+                    // the column starts its span and the empty ones before it
+                    const int c0 = LD.ax[2][z0].b;
+                    for (int sp = t > 0 ? LD.ax[2][z0 + t - 1].b - c0 + 1 : 0; sp <= a.b - c0; ++sp) S.cz[sp] = t;
+                    if (t == nz - 1) S.cz[a.b - c0 + 1] = nz;
                 }
-                const int c0 = LD.ax[2][z0].b, nc = LD.ax[2][z0 + nz - 1].b + 4 - c0;
-                for (int i = t; i < 2 * nc && i < 2 * (kFieldCols + 3); i += kBlock) S.cz[i] = LD.sup[2][2 * c0 + i];
             }
             for (int i = t; i < 2 * parts * cyl * nz; i += kBlock) S.Q[i] = 0.0f;
             BLOCK_END
@@ -1793,8 +1795,7 @@ HD void body_field_fit(const VolDesc* vols, int bid, N4_LDS unsigned char* smem)
                     for (int k = 3; k >= 0; --k) {  // the spans that c reaches: c - k
                         const int sp = c - k;
                         if (sp < 0 || sp > nc - 4) continue;
-                        const int zl = S.cz[2 * sp + 6] - z0, zh = S.cz[2 * sp + 1] - z0;
-                        const int za = zl > 0 ? zl : 0, ze = zh < nz ? zh : nz;
+                        const int za = S.cz[sp], ze = S.cz[sp + 1];
                         const N4_LDS float* w = (den ? S.zq : S.zp) + k;
                         UNROLL_4 for (int i = za; i < ze; ++i) acc += (double)w[4 * i] * (double)q[i];
                     }

@@ -56,3 +56,20 @@ def test_many_control_points_emulated(emu, dims, ncpt):
 @pytest.mark.parametrize("dims,ncpt", MANY)
 def test_many_control_points_gpu(gpu, dims, ncpt):
     _check(gpu, dims, ncpt, 0.7)
+
+
+# Spans of a quarter voxel and less: four spans in a row without a voxel leave
+# a control point without support.
+EMPTY = [((8, 8, 3), (11, 11, 19)), ((32, 32, 5), (11, 11, 35)), ((64, 64, 12), (67, 67, 67)), ((4, 4, 2), (4, 4, 15)),
+         ((4, 4, 4), (4, 4, 35)), ((3, 4, 1), (4, 5, 300)), ((2, 5, 59), (4, 9, 300)), ((4, 3, 5), (4, 40, 5))]
+
+
+@pytest.mark.parametrize("dims,ncpt", EMPTY)
+def test_empty_spans_emulated(emu, dims, ncpt):
+    _check(emu, dims, ncpt, 0.7)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dims,ncpt", EMPTY)
+def test_empty_spans_gpu(gpu, dims, ncpt):
+    _check(gpu, dims, ncpt, 0.7)
