@@ -500,6 +500,18 @@ static int rows_for(int rows, int cols, int target) {
     return r < rows ? r : rows;
 }
 
+// Dynamic LDS of a workgroup of the step, stage and reconstruction kernels.
+static const size_t kLdsCap = 64 * 1024;
+// Rows of a reconstruction tile of about tile_vox voxels of a volume F under
+// a final lattice C: fewer where the tile's row factors (20 bytes each) would
+// not fit the LDS, so that what is refused (lds_recon_limit) depends neither
+// on the size of the volume nor on its neighbours in the call.
+static int recon_tile_rows(const int F[3], const int C[3], int tile_vox) {
+    int r = rows_for(F[1], F[2], tile_vox);
+    while (r > 1 && lds_recon(r, C[1], C[2]) > kLdsCap) r = (r + 1) / 2;
+    return r;
+}
+
 // The last upload from the stage has completed.
 static void stage_wait(n4_handle* h) {
 #ifndef N4_EMULATE
@@ -626,7 +638,7 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
         I.Lmax = (size_t)Cf[0] * Cf[1] * Cf[2];
         I.prep_rows = rows_for(I.W[1], I.W[2], kPrepTileVox);
         I.prep_tiles_x = (I.W[1] + I.prep_rows - 1) / I.prep_rows;
-        I.recon_rows = rows_for(in[v].F[1], in[v].F[2], recon_tile);
+        I.recon_rows = recon_tile_rows(in[v].F, Cf, recon_tile);
         I.recon_tiles_x = (in[v].F[1] + I.recon_rows - 1) / I.recon_rows;
         step_tiles(I.W, tiled, tile_vox, &I.wtile_rows, &I.wtiles_x);
         nws += I.W[0] * I.wtiles_x;
@@ -936,7 +948,8 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
         const int prec = P->rp.prec;
         if (res)  // (the kernel also reconstructs tiles, in the same LDS behind the broadcast words)
             P->lds_resident =
-                std::max(P->lds_resident, std::max(lds_resident(D, nb, P->rp.P, prec), lds_recon(D) + kResBcBytes));
+                std::max(P->lds_resident, std::max(lds_resident(D, nb, P->rp.P, prec),
+                                                  lds_recon(I.recon_rows, I.C[L - 1][1], I.C[L - 1][2]) + kResBcBytes));
         for (int l = 0; l < L; ++l) {
             P->lds_fit_max[l] = std::max(P->lds_fit_max[l], lds_fit(nb, D, l, prec));
             P->lds_eval_max[l] = std::max(P->lds_eval_max[l], lds_eval(D, l, prec));
@@ -945,8 +958,11 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
             P->nt[l] = mfma_tiles(D.lev[l].C[2]);
         }
         if (need_tables_full) {
-            P->lds_recon = std::max(P->lds_recon, lds_recon(D));
-            P->lds_recon_limit = std::max(P->lds_recon_limit, lds_recon_limit(D));
+            const int Cy = I.C[L - 1][1], Cz = I.C[L - 1][2];
+            P->lds_recon = std::max(P->lds_recon, lds_recon(I.recon_rows, Cy, Cz));
+            P->lds_recon_limit =
+                std::max(P->lds_recon_limit,
+                         lds_recon_limit(rows_for(in[v].F[1], in[v].F[2], kReconTileMin), in[v].F[2], Cy, Cz));
         }
     }
     if (res) {
@@ -966,7 +982,6 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
 }
 
 // LDS of every kernel a grid plan launches must fit one workgroup.
-static const size_t kLdsCap = 64 * 1024;
 static n4_status check_lds(const Plan& P, bool grid_kernels, bool recon) {
     size_t worst = std::max(P.lds_hist, P.lds_wiener);
     if (grid_kernels)

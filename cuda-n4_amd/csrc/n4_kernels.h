@@ -28,11 +28,14 @@ size_t lds_wiener(int P);
 // prec (RunParams::prec) selects the FP32 or the MFMA kernels.
 size_t lds_fit(int nbins, const VolDesc& v, int level, int prec);
 size_t lds_eval(const VolDesc& v, int level, int prec);
-size_t lds_recon(const VolDesc& v);
-// What the refusal of volumes too large for a workgroup goes by: z factors of
-// a whole row beside the kernel's own arrays (the kernel keeps them in
-// registers; the limit on the row length stays where it was).
-size_t lds_recon_limit(const VolDesc& v);
+// Reconstruction in tiles of `rows` full-resolution rows under a lattice of
+// Cy x Cz control points along y and z.
+size_t lds_recon(int rows, int Cy, int Cz);
+// What the refusal of volumes too large for a workgroup goes by, at the
+// smallest tile: z factors of a whole row beside the kernel's own arrays (the
+// kernel keeps them in registers; the limit on the row length stays where it
+// was).
+size_t lds_recon_limit(int rows, int Z, int Cy, int Cz);
 // MFMA tiles (16 control points each) for c control points along an axis.
 int mfma_tiles(int c);
 size_t lds_flat(int nbins);

@@ -2983,16 +2983,14 @@ size_t lds_eval(const VolDesc& v, int level, int prec) {
     return carve_eval(nullptr, v.W[2], rows_per_eval_chunk(v.W[1], v.W[2]), v.wtile_rows, L.C[1], L.C[2], nullptr);
 }
 
-size_t lds_recon(const VolDesc& v) {
-    const LevelDesc& L = v.lev[v.nlevels - 1];
-    return carve_recon(nullptr, recon_chunk_rows(v.recon_rows, L.C[2]), v.recon_rows, L.C[1], L.C[2], nullptr);
+size_t lds_recon(int rows, int Cy, int Cz) {
+    return carve_recon(nullptr, recon_chunk_rows(rows, Cz), rows, Cy, Cz, nullptr);
 }
 
-size_t lds_recon_limit(const VolDesc& v) {
-    const LevelDesc& L = v.lev[v.nlevels - 1];
-    const size_t Cy = L.C[1], Cz = L.C[2], Z = v.F[2], Yt = v.recon_rows;
-    const size_t R = std::min<size_t>(Yt, std::max<size_t>(1, kReconChunkFloats / Cz));
-    return align16(4 * Cy * Cz) + align16(4 * R * Cz) + align16(16 * Z) + align16(4 * Z) + align16(16 * Yt) + align16(4 * Yt);
+size_t lds_recon_limit(int rows, int Z, int Cy, int Cz) {
+    const size_t R = std::min(rows, std::max(1, kReconChunkFloats / Cz)), Yt = rows;
+    return align16(4 * (size_t)Cy * Cz) + align16(4 * R * Cz) + align16(16 * (size_t)Z) + align16(4 * (size_t)Z) +
+           align16(16 * Yt) + align16(4 * Yt);
 }
 
 int mfma_tiles(int c) { return cp_tiles(c); }
