@@ -2178,8 +2178,11 @@ HD void recon_rows(const VolDesc& V, const N4_LDS float* B, int Cz, size_t v0, i
                 if (rr >= ny) break;
                 const N4_LDS float* br = B + rr * (Cz + 1) + T.c.b;
                 F4 f, n, e;
-                if (T.c.near) {
-                    const float b0 = br[0], b1 = br[1], b2 = br[2], b3 = br[3], b4 = br[4];
+                const float b0 = br[0], b4 = br[4];
+                // (the quad's zero factors would take an infinity or NaN of a
+                // control point to a voxel that does not touch it)
+                if (T.c.near && fabsf(b0) + fabsf(b4) < INFINITY) {
+                    const float b1 = br[1], b2 = br[2], b3 = br[3];
                     UNROLL for (int j = 0; j < 4; ++j)
                         f.v[j] = T.c.w[j][0] * b0 + T.c.w[j][1] * b1 + T.c.w[j][2] * b2 + T.c.w[j][3] * b3 + T.c.w[j][4] * b4;
                 } else {

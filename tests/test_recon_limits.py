@@ -52,3 +52,38 @@ def test_accepted_beside_a_large_neighbour(emu):
     alone = emu.correct_batch(vols[:1], **dict(kw, shrink=[8]))
     assert np.array_equal(both[0]["log_bias"], alone[0]["log_bias"])
     assert np.array_equal(both[0]["normalized"], alone[0]["normalized"])
+
+
+def _check_nonfinite(lib, dims, ncpt, bad, value):
+    """Only the voxels whose span holds a non-finite control point are
+    non-finite (at the very start of a span too, where its last factor is
+    zero).  The others may be summed in another form: two sums of at most five
+    products, each rounding within 2^-24 of the largest control point."""
+    lat = np.random.default_rng(11).standard_normal(ncpt).astype(np.float32)
+    clean = lib.evaluate_bspline3d(lat, dims)
+    lat[bad] = value
+    out = lib.evaluate_bspline3d(lat, dims)
+    hit = np.ones(dims, bool)
+    for d in range(3):
+        n, c = dims[d], ncpt[d]
+        b = np.clip(np.floor((np.arange(n) + 0.5) / (n / (c - 3))).astype(int), 0, c - 4)
+        hit &= ((b <= bad[d]) & (bad[d] <= b + 3)).reshape([-1 if k == d else 1 for k in range(3)])
+    assert not np.isfinite(out[hit]).any()
+    assert np.abs(out[~hit] - clean[~hit]).max(initial=0) <= 10 * 2.0**-24 * np.abs(lat[np.isfinite(lat)]).max()
+
+
+NONFINITE = [((5, 6, 30), (4, 4, 11), (2, 1, 9)), ((6, 5, 31), (4, 5, 11), (0, 4, 3)), ((4, 4, 64), (4, 4, 7), (1, 2, 0)),
+             ((4, 9, 9), (4, 4, 11), (3, 3, 10)), ((3, 4, 45), (4, 4, 11), (1, 1, 5))]
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+@pytest.mark.parametrize("dims,ncpt,bad", NONFINITE)
+def test_nonfinite_control_point(emu, dims, ncpt, bad, value):
+    _check_nonfinite(emu, dims, ncpt, bad, value)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+@pytest.mark.parametrize("dims,ncpt,bad", NONFINITE)
+def test_nonfinite_control_point_gpu(gpu, dims, ncpt, bad, value):
+    _check_nonfinite(gpu, dims, ncpt, bad, value)
