@@ -1333,6 +1333,10 @@ static bool plan_resident(const std::vector<VolIn>& in, const n4_params* p, cons
     const int nv = (int)in.size(), L = (int)p->number_of_fitting_levels;
     const RunParams rp = make_run_params(p);
     size_t lds_cap = 0;
+    // without it a control point that no foreground voxel touches has the
+    // increment 0 / 0, which the zeros of the matrix operands would carry to
+    // voxels that do not touch it; the step kernels leave such points out
+    if (!(p->fit_eps > 0.0)) return false;
     if (resident_limits(&R->cus, &lds_cap) != 0 || R->cus < 1) return false;
     R->nchunk.assign(nv, 1);
     R->nbatch.assign(nv, 64);

@@ -121,3 +121,22 @@ def _box(dims, z0, seed):
 @pytest.mark.parametrize("nz,z0", [(29, 12), (31, 12), (32, 12), (32, 28), (64, 12), (64, 28), (61, 44), (96, 76)])
 def test_foreground_to_the_last_z(gpu, precision, nz, z0):
     _both(gpu, [_box((9, 37, nz), z0, nz)], levels=3, max_iter=[3, 3, 2], fixed_iterations=True, precision=precision)
+
+
+@pytest.mark.parametrize("precision", ["fp32", "bf16"])
+def test_no_fit_epsilon(gpu, precision):
+    """With no term in the fit's denominator, control points without foreground
+    have no value (0 / 0); the voxels that they do not touch keep theirs."""
+    im, m = _box((40, 44, 48), 4, 2)
+    m[:] = 0
+    m[5:15, 11:22, 6:18] = 1  # whole spans of 5, 5.5 and 6 voxels
+    kw = dict(levels=1, max_iter=[4], ncpt=(11, 11, 11), fixed_iterations=True, eps=0.0, precision=precision)
+    try:
+        gpu.set_tuning(path="steps")
+        ref = gpu.correct_batch([(im, m)], **kw)[0]
+    finally:
+        gpu.set_tuning(reset=True)
+    out = gpu.correct_batch([(im, m)], **kw)[0]
+    assert np.isfinite(ref["log_bias"][m != 0]).all() and np.isnan(ref["lattice"]).any()
+    for k in ("log_bias", "normalized", "lattice"):
+        assert np.array_equal(out[k], ref[k], equal_nan=True), k
