@@ -369,8 +369,8 @@ struct Plan {
     size_t lds_persist = 0;  // dynamic LDS of the persistent kernel (largest volume)
     // resident path
     size_t off_team = 0;     // team words of every volume and the ticket (zeroed with the states)
-    size_t off_slots = 0;    // int32 per workgroup slot
-    int n_slots = 0;
+    size_t off_slots = 0;    // int32 per workgroup slot (room for a slot per chunk)
+    int n_slots = 0;         // this launch's
     size_t lds_resident = 0;
     unsigned char* base = nullptr;  // device arena the plan lives in
 };
@@ -568,12 +568,28 @@ static n4_status stage_upload(n4_handle* h, void* dst, size_t off, size_t n, voi
     return N4_OK;
 }
 
-// Resident path: chunks (workgroups of a full team) and LDS batch size per
-// volume.
+// Resident path: chunks (workgroups of the largest team), workgroups of this
+// launch's team and LDS batch size per volume.
 struct ResPlan {
-    std::vector<int> nchunk, nbatch;
+    std::vector<int> nchunk, nmember, nbatch;
     int cus = 0;
 };
+
+// This launch's team sizes into the descriptors and the slot list of the
+// image hb: the largest volumes first, each with all its slots in a row.
+static void put_teams(Plan* P, const ResPlan& R, unsigned char* hb) {
+    const int nv = (int)P->desc.size();
+    std::vector<std::pair<double, int>> by(nv);
+    for (int v = 0; v < nv; ++v) {
+        by[v] = {-(double)P->desc[v].nvox_w, v};
+        P->desc[v].res.nmember = R.nmember[v];
+    }
+    std::sort(by.begin(), by.end());
+    int32_t* sl = (int32_t*)(hb + P->off_slots);
+    P->n_slots = 0;
+    for (const auto& b : by)
+        for (int k = 0; k < R.nmember[b.second]; ++k) sl[P->n_slots++] = b.second;
+}
 
 // Builds the plan and fills h->stage with the upload region.  Pointers in
 // the descriptors are arena-relative until `rebase` adds the arena base.
@@ -660,10 +676,10 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
     P->off_pslab = lay.take(sizeof(Slab) * (nps > 0 ? nps : 1));
     P->off_state = lay.take(sizeof(VolState) * nv);
     P->off_team = lay.take(res ? 64 * (size_t)(nv + 1) : 0);
-    P->n_slots = 0;
+    int slots = 0;
     if (res)
-        for (int v = 0; v < nv; ++v) P->n_slots += res->nchunk[v];
-    P->off_slots = lay.take(sizeof(int32_t) * P->n_slots);
+        for (int v = 0; v < nv; ++v) slots += res->nchunk[v];
+    P->off_slots = lay.take(sizeof(int32_t) * slots);
     P->off_tw = lay.take(use & kUseTwiddle ? sizeof(D2) * P->rp.P : 0);
     P->n_work = 0;
     if (teams)
@@ -965,15 +981,7 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
                          lds_recon_limit(rows_for(in[v].F[1], in[v].F[2], kReconTileMin), in[v].F[2], Cy, Cz));
         }
     }
-    if (res) {
-        // the largest volumes first, each with all its slots in a row
-        std::vector<std::pair<double, int>> by(nv);
-        for (int v = 0; v < nv; ++v) by[v] = {-(double)P->desc[v].nvox_w, v};
-        std::sort(by.begin(), by.end());
-        int32_t* sl = (int32_t*)(hb + P->off_slots);
-        for (const auto& b : by)
-            for (int k = 0; k < res->nchunk[b.second]; ++k) *sl++ = b.second;
-    }
+    if (res) put_teams(P, *res, hb);
     P->lds_hist = lds_hist(nb);
     P->lds_wiener = lds_wiener(P->rp.P);
     memcpy(hb + P->off_desc, P->desc.data(), sizeof(VolDesc) * nv);
@@ -1396,6 +1404,67 @@ static bool plan_resident(const std::vector<VolIn>& in, const n4_params* p, cons
 }
 #endif
 
+// The calls of this process whose resident kernels share a device, and the
+// workgroups that these have between them.
+struct ResidentUse {
+    std::mutex mu;
+    int calls = 0, wgs = 0;
+};
+static ResidentUse g_resident_use[kMaxDevices];
+
+// A call's part of the device's compute units, for as long as the call lasts:
+// those that other calls have left or, where that is less, an equal part (the
+// others come down to theirs with their next call).  A workgroup of the
+// resident kernel needs a compute unit to itself and a team works with the
+// members that it has when it closes, so teams sized for the whole device,
+// launched side by side, took the workgroups from each other and ran short:
+// two callers of 512 x 512 x 320 at shrink 2, BF16, 345 calls/s in all and
+// four 378, the slowest call 156 ms (here 530 and 750, 10 ms; one caller 475).
+// Members take whole
+// numbers of chunks (a team of 200 for 256 chunks is as slow as one of 128),
+// so a volume has ceil(chunks / k) of them, the smallest k that fits.
+// N4_RESIDENT_WGS, if set, is the most workgroups of a call.
+class ResidentShare {
+public:
+    ~ResidentShare() { give_back(); }
+    void take(int device, ResPlan* R) {
+        const int cap = env_int("N4_RESIDENT_WGS", 0);
+        ResidentUse& u = g_resident_use[device];
+        std::lock_guard<std::mutex> lk(u.mu);
+        use_ = &u;
+        ++u.calls;
+        int room = std::max(R->cus - u.wgs, R->cus / u.calls);
+        if (cap > 0) room = std::min(room, cap);
+        room = std::max(room, 1);
+        int most = 1;
+        for (int n : R->nchunk) most = std::max(most, n);
+        for (int k = 1;; ++k) {
+            R->nmember.clear();
+            int sum = 0;
+            for (int n : R->nchunk) {
+                R->nmember.push_back((n + k - 1) / k);
+                sum += R->nmember.back();
+            }
+            if (sum > room && k < most) continue;
+            wgs_ = std::min(sum, room);
+            break;
+        }
+        u.wgs += wgs_;
+    }
+    void give_back() {
+        if (!use_) return;
+        std::lock_guard<std::mutex> lk(use_->mu);
+        --use_->calls;
+        use_->wgs -= wgs_;
+        use_ = nullptr;
+    }
+    int wgs() const { return wgs_; }
+
+private:
+    ResidentUse* use_ = nullptr;
+    int wgs_ = 0;
+};
+
 #define GLAUNCH(id, expr)                  \
     do {                                   \
         ProfScope ps_(h, (id), gs);        \
@@ -1481,6 +1550,8 @@ static n4_status run_batch(n4_handle* h, const std::vector<VolIn>& in_user, cons
         resident = plan_resident(in_user, p, sch, &res_user);
     }
 #endif
+    ResidentShare share;
+    if (resident) share.take(h->device, &res_user);
     const int G = (teams_path || noalloc || resident) ? 1 : sch.groups;
     // kernel timing creates events: off for the allocation-free path
     struct ProfMaskGuard {
@@ -1523,6 +1594,7 @@ static n4_status run_batch(n4_handle* h, const std::vector<VolIn>& in_user, cons
         if (teams_path) teams[k] = teams_user[order[k]];
         if (resident) {
             res.nchunk.push_back(res_user.nchunk[order[k]]);
+            res.nmember.push_back(res_user.nmember[order[k]]);
             res.nbatch.push_back(res_user.nbatch[order[k]]);
         }
     }
@@ -1570,6 +1642,7 @@ static n4_status run_batch(n4_handle* h, const std::vector<VolIn>& in_user, cons
             D.out_lattice = in[v].out_lattice;
         }
         stage_wait(h);
+        if (resident) put_teams(&P, res, h->stage);
         memcpy(h->stage + P.off_desc, P.desc.data(), sizeof(VolDesc) * nv);
     } else {
         s = build_plan(h, in, p, &P, kUseCorrection, true, sch.tile_vox, teams_path ? &teams : nullptr, noalloc,
@@ -1587,9 +1660,10 @@ static n4_status run_batch(n4_handle* h, const std::vector<VolIn>& in_user, cons
             h->plan_key = pkey;
         }
     }
-    // the volume states and, on the resident path, the team words behind them
+    // the volume states and, on the resident path, the team words and the slot
+    // list behind them
     const size_t state_bytes =
-        resident ? P.off_team + 64 * (size_t)(nv + 1) - P.off_state : sizeof(VolState) * (size_t)nv;
+        resident ? P.off_slots + sizeof(int32_t) * P.n_slots - P.off_state : sizeof(VolState) * (size_t)nv;
     // (a call that the step kernels' LDS refuses is refused on the resident path too)
     s = check_lds(P, !teams_path, true);
     if (s != N4_OK) return s;
@@ -1598,7 +1672,7 @@ static n4_status run_batch(n4_handle* h, const std::vector<VolIn>& in_user, cons
         // twiddles, axis tables; no kernel writes them): descriptors, and the
         // volume states back to their initial (zero) image
         s = stage_upload(h, P.base + P.off_desc, P.off_desc, sizeof(VolDesc) * nv, stream);
-        if (s == N4_OK)  // (and, on the resident path, the team words behind them)
+        if (s == N4_OK)
             s = stage_upload(h, P.base + P.off_state, P.off_state, state_bytes, stream);
     } else {
         s = stage_upload(h, P.base, 0, P.upload_bytes, stream);
@@ -1689,8 +1763,7 @@ static n4_status run_batch(n4_handle* h, const std::vector<VolIn>& in_user, cons
     if (resident) {
         // one launch runs every volume's level/iteration loop
         void* gs = stream;
-        GLAUNCH(N4_K_TEAMS, launch_resident(dd, nv, (const int32_t*)(P.base + P.off_slots), P.n_slots,
-                                            std::min(P.n_slots, res.cus),
+        GLAUNCH(N4_K_TEAMS, launch_resident(dd, nv, (const int32_t*)(P.base + P.off_slots), P.n_slots, share.wgs(),
                                             (uint32_t*)(P.base + P.off_team + 64 * (size_t)nv), rp, P.lds_resident, gs));
         GLAUNCH(N4_K_RECON, launch_recon(dd, fsl, P.n_fslab, P.nlevels - 1, rp, P.lds_recon, gs));
         for (GroupRun& R : gr) R.finished = true;
@@ -1800,9 +1873,8 @@ static n4_status run_batch(n4_handle* h, const std::vector<VolIn>& in_user, cons
 #endif
         }
     }
-    std::vector<unsigned char> st_bytes(state_bytes);
-    const VolState* st = reinterpret_cast<const VolState*>(st_bytes.data());
-    D2H(st_bytes.data(), dev_state(h, P), state_bytes, stream);
+    std::vector<VolState> st(nv);
+    D2H(st.data(), dev_state(h, P), sizeof(VolState) * nv, stream);
     std::vector<uint32_t> tctr(teams_path ? 2 * nv : 0);
     std::vector<uint64_t> tph((teams_path || resident) && P.desc[0].tphase ? (size_t)kPhases * nv : 0);
     if (teams_path || resident)

@@ -100,10 +100,10 @@ enum ResWord : int {
 
 // A volume's buffers on the resident path (nchunk 0: not a resident plan).
 struct ResDesc {
-    int32_t nchunk;   // runs of strips = workgroups of a full team
+    int32_t nchunk;   // runs of strips, one per workgroup of the largest team
     int32_t umax;     // unit entries per slab
     int32_t nbatch;   // units whose list and T2 slots fit the LDS at once (at most 64)
-    int32_t pad;
+    int32_t nmember;  // workgroups of this launch's team (1 .. nchunk)
     float* xq;        // packed logU: 256 floats per tile, lane-major quads
     uint8_t* mq;      // mask bits of every quad (bits 0..3)
     float* cq;        // packed confidence weights (weighted masks; else null)

@@ -88,7 +88,7 @@ int launch_persist(const VolDesc* vols, const Slab* slabs, const PWork* work, in
 
 // Resident path (n4_resident.h): every volume's level/iteration loop in one
 // launch of nwg workgroups (one per compute unit); slots[k] names the volume
-// whose team the k-th workgroup to ask joins (a volume's nchunk slots are
+// whose team the k-th workgroup to ask joins (a volume's nmember slots are
 // consecutive); run (two words, zero): slots taken, volumes ready.  Some of
 // the reconstruction may be done by it; launch_recon does the rest.
 size_t lds_resident(const VolDesc& v, int nbins, int P, int prec);

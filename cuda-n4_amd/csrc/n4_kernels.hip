@@ -3183,7 +3183,7 @@ __global__ __launch_bounds__(kResThreads) void k_resident(const VolDesc* __restr
         if (k >= nslots) break;
         last = slots[k];
         const VolDesc& V = vols[last];
-        const int rank = uni(res_join(V.res.team, V.res.nchunk, smem));
+        const int rank = uni(res_join(V.res.team, V.res.nmember, smem));
         if (rank == -1) continue;  // its team runs without this workgroup
         if (rank < 0 || !res_volume<PREC>(V, rp, rank, uni(bc[2]), nvol > 1 ? run + 1 : nullptr, smem)) return;
     }

@@ -55,7 +55,10 @@ constexpr int kResThreads = kResBlock;
 constexpr int kResWaves = kResThreads / 64;
 constexpr int kResBr = 20;  // row stride of a wave's y-contracted block (16-byte rows, distinct banks)
 constexpr uint32_t kResClosed = 0x80000000u;
-constexpr uint64_t kResJoinTicks = 20000;  // 100 MHz clock: 200 us
+// 100 MHz clock: 1 ms, the time that other streams' kernels take to leave the
+// compute units (with 200 us the slowest call of four callers side by side,
+// batch64, two head256 and a 64^3 volume, took 30 ms in place of 12).
+constexpr uint64_t kResJoinTicks = 100000;
 
 #define N4_PHASE __device__ __attribute__((noinline))
 #define N4_PHASE_HD __host__ __device__ __attribute__((noinline))
@@ -371,8 +374,8 @@ __device__ inline bool res_barrier(uint32_t* team, int m, uint32_t gen, LdsP sme
     return res_barrier_t<false>(team, m, gen, smem, 0.0);
 }
 
-// Joins the team of a volume with n chunks: rank (>= 0; the team's
-// size in broadcast word 2); -1: the team was closed before this workgroup came; -2: gave up.
+// Joins a team of n workgroups: rank (>= 0; the team's size in broadcast
+// word 2); -1: the team was closed before this workgroup came; -2: gave up.
 N4_PHASE int res_join(uint32_t* team, int n, LdsP smem) {
     N4_LDS int* bc = reinterpret_cast<N4_LDS int*>(res_base(smem));
     __syncthreads();

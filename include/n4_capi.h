@@ -244,7 +244,10 @@ n4_status n4_reduce_min(n4_handle *h, uint64_t n, const float *d_in, float *out)
  *     workgroup of the launch is resident at once);
  *   resident: one launch in which teams, formed by the workgroups that
  *     arrive, keep a volume's foreground packed and its tables in LDS for
- *     the whole loop; up to 16 control points along y and z.
+ *     the whole loop; up to 16 control points along y and z, fit_eps above 0.
+ *     Calls that run at the same time on handles of their own share the
+ *     device's compute units (N4_RESIDENT_WGS, if set, is the most that one
+ *     call takes); the results do not depend on how many a call gets.
  * All run the same per-tile arithmetic, so they give the same bits.
  * Results do not depend on the schedule except through the summation order
  * of the FP64 convergence partials (one partial per tile).  A field left 0 takes the

@@ -140,3 +140,67 @@ def test_no_fit_epsilon(gpu, precision):
     assert np.isfinite(ref["log_bias"][m != 0]).all() and np.isnan(ref["lattice"]).any()
     for k in ("log_bias", "normalized", "lattice"):
         assert np.array_equal(out[k], ref[k], equal_nan=True), k
+
+
+@pytest.mark.parametrize("precision", ["fp32", "bf16", "split_bf16"])
+def test_any_number_of_workgroups(gpu, precision, monkeypatch):
+    """The results do not depend on how many workgroups a call gets: teams of
+    one workgroup a chunk, teams whose members have several, fewer workgroups
+    than volumes; the same plan is used again with other teams."""
+    vols = [_vol(d, 60 + k) for k, d in enumerate([(64, 60, 52), (18, 90, 47), (33, 20, 70), (5, 7, 9)])]
+    kw = dict(levels=3, max_iter=[4, 3, 3], threshold=0.0005, precision=precision)
+    ref = gpu.correct_batch(vols, **kw)
+    for wgs in (1, 2, 3, 5, 8, 13, 30, 61, 256):
+        monkeypatch.setenv("N4_RESIDENT_WGS", str(wgs))
+        for a, b in zip(ref, gpu.correct_batch(vols, **kw)):
+            assert a["iterations"] == b["iterations"] and a["last_cv"] == b["last_cv"], wgs
+            assert (a["n_mask_full"], a["n_mask_work"]) == (b["n_mask_full"], b["n_mask_work"])
+            for k in ("log_bias", "normalized", "lattice"):
+                assert np.array_equal(a[k], b[k]), (wgs, k)
+
+
+def test_handles_side_by_side(gpu):
+    """Four threads with a handle and a stream each, large and small volumes
+    and a batch: everyone gets the bits that it gets alone."""
+    import ctypes as C
+    import threading
+
+    import n4amd
+
+    jobs = [([_vol((150, 140, 130), 1)], "bf16"), ([_vol((120, 130, 140), 2)], "bf16"), ([_vol((40, 36, 33), 3)], "fp32"),
+            ([_vol((60 + 9 * k, 50, 70 - 7 * k), 10 + k) for k in range(6)], "split_bf16")]
+    state = []
+    for vols, precision in jobs:
+        lib = n4amd.Library(gpu.L, False)
+        p = n4amd.default_params(levels=2, max_iter=[6, 5], threshold=0.0005, precision=precision)
+        keep, arr = lib._batch_arrays(vols, p, True, None)
+        stream = C.c_void_p()
+        assert gpu.L.hipStreamCreateWithFlags(C.byref(stream), 1) == 0  # hipStreamNonBlocking
+        state.append((lib, p, keep, arr, (n4amd.Report * len(vols))(), stream))
+
+    def call(s):
+        lib, p, _, arr, reports, stream = s
+        return lib.L.n4_correct_batch(lib.h, arr, len(arr), C.byref(p), reports, stream)
+
+    def results(s):
+        return [k[i].download(np.float32, k[0]) for k in s[2] for i in (3, 5)]
+
+    for s in state:
+        assert call(s) == 0
+    alone = [results(s) for s in state]
+    status = [[] for _ in state]
+    threads = [threading.Thread(target=lambda s=s, r=r: r.extend(call(s) for _ in range(12)))
+               for s, r in zip(state, status)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for s, ref, st in zip(state, alone, status):
+        assert st == [0] * 12
+        assert all(np.array_equal(a, b) for a, b in zip(ref, results(s)))
+    for lib, _, keep, _, _, stream in state:
+        for k in keep:
+            for a in k[1:]:
+                if a is not None:
+                    a.free()
+        assert gpu.L.hipStreamDestroy(stream) == 0 and lib.L.n4_destroy(lib.h) == 0
