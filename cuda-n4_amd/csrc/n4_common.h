@@ -90,7 +90,7 @@ constexpr int kResNumCopies = 8;   // most numerator copies of a resident plan
 constexpr int kResMaxDim = 1024;   // most working rows / z positions it covers
 constexpr int kResMaxSlabs = 2048; // most working slabs
 
-// Words of a volume's team area (64 bytes, zero before the launch): joined
+// Words of a volume's team area (zero before the launch): joined
 // members and closed flag, team size, barrier counter, abort flag, the
 // working and full foreground counts (64-bit), lattice ready, reconstruction
 // tiles taken.
