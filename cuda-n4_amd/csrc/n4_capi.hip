@@ -1328,6 +1328,29 @@ static bool plan_teams(const std::vector<VolIn>& in, const n4_params* p, const S
     return true;
 }
 
+// Thin working grids, few voxels along z, which the step kernels correct
+// faster: a unit of the resident kernel is 16 rows by the z it holds, so a
+// slab of few z is many units of little work in every iteration, and the
+// waits of a large team outweigh the launches that they replace.  Time of the
+// steps over that of the resident kernel, 36 iterations at shrink 1, by z:
+//   volumes            4     8     16    17    20    24
+//   1 x 256^2  FP32   0.90  0.98  1.06  1.15  1.15  1.21
+//   1 x 256^2  BF16   0.80  0.86  0.88  0.98  0.95  0.98
+//   1 x 128^2  BF16   0.90  0.93  0.95  1.02  1.01  1.01
+//   1 x 64^2   BF16   1.02  1.03  1.04  1.08  1.06  1.05
+//   2 x 256^2  FP32   1.00  1.05  1.19  1.29  1.24  1.33
+//   2 x 256^2  BF16   0.89  0.92  0.97  1.08  1.03  1.09
+//   4 x 256^2  BF16   1.06  1.07  1.11  1.23  0.98  1.07
+//   4 x 512^2  BF16   0.93  0.95  1.06      (3 z: 0.86; FP32 1 z 0.84, 4 z 1.07)
+//   16 x 384^2 FP32   1.00                  (3 z: 0.91; 1 z 0.86)
+static bool thin_grid(const VolIn& in, int nv, bool mfma) {
+    int W[3];
+    for (int d = 0; d < 3; ++d) W[d] = (in.F[d] + in.s - 1) / in.s;
+    const int64_t units = (int64_t)W[0] * ((W[1] + 15) / 16);
+    if (nv <= 2) return mfma ? units > 768 && W[2] <= 16 : units > 2000 && W[2] < 6;
+    return units > 8192 && W[2] < 4;
+}
+
 // Resident path: chunks per volume, or false where a volume is not covered:
 // the matrix operands hold 16 control points along y and z, a volume's
 // factor tables, lattice increment and one batch of units share a compute
@@ -1350,6 +1373,9 @@ static bool plan_resident(const std::vector<VolIn>& in, const n4_params* p, cons
     // increment 0 / 0, which the zeros of the matrix operands would carry to
     // voxels that do not touch it; the step kernels leave such points out
     if (!(p->fit_eps > 0.0)) return false;
+    bool thin = true;
+    for (const VolIn& v : in) thin = thin && thin_grid(v, nv, p->precision != N4_PREC_FP32);
+    if (thin) return false;
     if (resident_limits(&R->cus, &lds_cap) != 0 || R->cus < 1) return false;
     R->nchunk.assign(nv, 1);
     R->nbatch.assign(nv, 64);

@@ -204,3 +204,9 @@ def test_handles_side_by_side(gpu):
                 if a is not None:
                     a.free()
         assert gpu.L.hipStreamDestroy(stream) == 0 and lib.L.n4_destroy(lib.h) == 0
+
+
+@pytest.mark.parametrize("dims,nvol,precision", [((128, 112, 16), 1, "bf16"), ((128, 112, 17), 1, "split_bf16"), ((200, 176, 5), 2, "fp32"),
+                                                 ((200, 176, 6), 2, "fp32"), ((600, 240, 3), 3, "bf16"), ((600, 240, 4), 3, "fp32")])
+def test_thin_grids_either_side_of_the_step_kernels(gpu, dims, nvol, precision):
+    _both(gpu, [_vol(dims, 70 + k) for k in range(nvol)], levels=2, max_iter=[3, 2], fixed_iterations=True, precision=precision)
