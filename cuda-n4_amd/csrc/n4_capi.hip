@@ -218,8 +218,12 @@ static n4_status ensure_arena(n4_handle* h, size_t bytes) {
     h->arena = nullptr;
     h->arena_bytes = 0;
     size_t want = bytes + bytes / 8 + (1u << 20);
-    if (dev_alloc(&h->arena, want))
+    if (dev_alloc(&h->arena, want)) {
+#ifndef N4_EMULATE
+        (void)hipGetLastError();  // (the caller may go on with a smaller plan)
+#endif
         return fail(N4_ERR_NO_MEMORY, "device allocation of %zu bytes failed", want);
+    }
     h->arena_bytes = want;
     return N4_OK;
 }
@@ -1678,12 +1682,15 @@ static n4_status run_batch(n4_handle* h, const std::vector<VolIn>& in_user, cons
     } else {
         s = build_plan(h, in, p, &P, kUseCorrection, true, sch.tile_vox, teams_path ? &teams : nullptr, noalloc,
                        resident ? &res : nullptr);
-        if (s == N4_ERR_NO_MEMORY && noalloc && resident) {
-            // (the step path needs a little less of the scratch array)
+        if (s == N4_ERR_NO_MEMORY && resident) {
+            // (the step path needs less: its logU has no padding, while the
+            // packed copy of a grid of 4 z takes up to four times the grid)
             resident = false;
+            share.give_back();
             g_err.clear();
             P = Plan();
-            s = build_plan(h, in, p, &P, kUseCorrection, true, sch.tile_vox, nullptr, true);
+            s = build_plan(h, in, p, &P, kUseCorrection, true, sch.tile_vox, nullptr, noalloc);
+            if (!noalloc) pkey = correction_plan_key(h, in, p, sch.tile_vox, nullptr, nullptr);
         }
         if (s != N4_OK) return s;
         if (!noalloc) {

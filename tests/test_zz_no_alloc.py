@@ -47,3 +47,13 @@ def test_noalloc_rejects_oversize():
     im = np.full((300, 300, 300), 100.0, np.float32)
     with pytest.raises(n4amd.N4Error, match="allocation-free"):
         gpu.correct(im, None, levels=1, max_iter=[1], noalloc=True)
+
+
+def test_noalloc_where_only_the_steps_fit():
+    """6 z of 1400 x 512: the packed copy of the resident kernel (a third of
+    every 16 z) does not fit the scratch, the step kernels' buffers do."""
+    gpu = n4amd.load()
+    rng = np.random.default_rng(4)
+    im = (100 + 50 * rng.random((1400, 512, 6))).astype(np.float32)
+    im[:40] = 0
+    _pair(gpu, im, None, levels=2, max_iter=[3, 2], fixed_iterations=True)
