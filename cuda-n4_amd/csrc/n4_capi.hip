@@ -926,7 +926,6 @@ static n4_status build_plan(n4_handle* h, const std::vector<VolIn>& in, const n4
         D.team_ctr = teams ? (uint32_t*)(base + o.team) : nullptr;
         D.tphase = ((teams || res) && (h->prof_mask >> N4_K_TEAMS & 1u)) ? (uint64_t*)(base + o.team + 64) : nullptr;
         D.mW2 = magic_div((uint32_t)I.W[2]);
-        D.mF2 = magic_div((uint32_t)in[v].F[2]);
         D.etab = (double*)(base + o.etab);
         D.st = (VolState*)(base + P->off_state) + v;
         D.progress = (!noalloc && h->dev_flags && v < h->flag_cap) ? h->dev_flags + v : nullptr;

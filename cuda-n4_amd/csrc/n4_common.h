@@ -169,7 +169,6 @@ struct VolDesc {
     int32_t lmax;              // control points of the finest level (numfx copy stride)
     double* ppart;             // prep partials [W0 * prep_tiles_x][4]
     uint64_t mW2;              // magic divisor for the working z extent
-    uint64_t mF2;              // magic divisor for the full-resolution z extent
     uint32_t* team_ctr;        // persistent path: [0] the team's barrier counter, [1] abort flag
     uint64_t* tphase;          // persistent path (nullable): leader's device-clock ticks per phase (kPhases)
     ResDesc res;               // resident path
@@ -247,11 +246,10 @@ constexpr int progress_done(uint64_t w) { return (int)(w & 1); }
 // m = floor(2^40 / d) + 1 (computed on the host).
 constexpr int kDivShift = 40;
 
-// Fit modes.  NUM and DEN_SCATTER add the slab's contraction, weighted by
-// the x factor, into the fixed-point numerator buffers (the correction
-// loop); DEN and FIELD write per-slab partials reduced by the lattice
-// kernel (stage calls).  STEP takes the mode, level and iteration from the
-// volume's current step (ITER -> NUM, TRANS -> DEN_SCATTER, else nothing).
+// Fit modes of the correction loop.  NUM and DEN add the tile's contraction
+// of the residual or of the mask, weighted by the x factor, into the
+// fixed-point numerator buffers.  STEP takes the mode, level and iteration
+// from the volume's current step (ITER -> NUM, TRANS -> DEN, else nothing).
 enum FitMode : int32_t { kFitNum = 0, kFitDen = 1, kFitStep = 2 };
 
 // Fixed-point scale of the lattice numerator accumulated by the fit's

@@ -127,7 +127,6 @@ struct alignas(16) ResCtx {
     int32_t Cy, Cz, L;
     int32_t pa, np;       // control planes of the own slabs
     int32_t o0, o1;       // control points whose update this workgroup owns
-    uint32_t mCz_lo, mCz_hi;
 };
 
 typedef const N4_LDS ResCtx* CtxP;
@@ -1345,8 +1344,6 @@ N4_PHASE bool res_enter_level(const VolDesc* Vp, LdsP smem, int level_, uint32_t
         C->Cy = LD.C[1];
         C->Cz = LD.C[2];
         C->L = LD.L;
-        C->mCz_lo = (uint32_t)LD.mCz;
-        C->mCz_hi = (uint32_t)(LD.mCz >> 32);
         C->pa = LD.ax[0][C->x0].b;
         C->np = U1 > U0 ? LD.ax[0][C->x1].b + 4 - C->pa : 0;
         int o0, o1;

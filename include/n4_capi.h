@@ -248,9 +248,13 @@ n4_status n4_reduce_min(n4_handle *h, uint64_t n, const float *d_in, float *out)
  *     Calls that run at the same time on handles of their own share the
  *     device's compute units (N4_RESIDENT_WGS, if set, is the most that one
  *     call takes); the results do not depend on how many a call gets.
- * All run the same per-tile arithmetic, so they give the same bits.
- * Results do not depend on the schedule except through the summation order
- * of the FP64 convergence partials (one partial per tile).  A field left 0 takes the
+ * All run the same per-tile arithmetic, so for equal iteration counts they
+ * give the same bits.  Results depend on the schedule only through the
+ * summation order of the FP64 convergence values (a partial per tile; on the
+ * resident path a partial per workgroup of the team planned for the volume,
+ * whose number follows the device and the other volumes of the call), which
+ * moves a recorded value by about 1e-15 of itself, and the number of
+ * iterations where that value meets the threshold.  A field left 0 takes the
  * environment override (N4_GROUPS, N4_STEP_TILE_VOX, N4_GRAPH_STEPS) if set,
  * else the built-in default. */
 #define N4_GRAPH_OFF 0xFFFFFFFFu
@@ -306,7 +310,7 @@ typedef enum n4_kernel_id {
     N4_K_EVAL = 5,    /* field + convergence partials + logU update */
     N4_K_RECON = 6,   /* full-resolution field + normalisation */
     N4_K_WIENER = 7,  /* Wiener deconvolution + E table (one block/volume) */
-    N4_K_LATTICE = 8, /* mode-x contraction + lattice update (stage calls) */
+    N4_K_LATTICE = 8, /* no launch any more (keeps the numbers after it) */
     N4_K_UPDATE = 9,  /* lattice update of a correction step */
     N4_K_TEAMS = 10,  /* persistent path: every volume's level/iteration loop */
     /* Phases of the persistent paths, timed inside the launch by each team's
