@@ -94,7 +94,23 @@ def algorithmic_bytes(kernel, vols_meta, reports, levels):
             total += 8 * nf + 9 * nw
         elif kernel == "recon":
             total += 12 * nf
+        elif kernel == "teams":
+            # the loop on the packed foreground: logU and mask bits read by the
+            # histogram, the fit and the evaluation, logU written by the last;
+            # per level the mask bits for the denominator
+            fg = int(r.n_mask_work)
+            total += (3 * 4.25 + 4) * fg * its + 0.25 * fg * levels
     return total
+
+
+def timing_schedule(schedule):
+    """The launches of the timed region, without what overlaps or replays
+    them: the resident kernel runs as it is, the step kernels in one group
+    without graphs."""
+    step_fields = any(schedule[k] for k in ("groups", "step_tile_voxels", "graph_steps", "eval_kernel"))
+    if schedule["path"] == "auto" and (schedule["team_wgs_per_cu"] or not step_fields):
+        return schedule
+    return dict(groups=1, graph_steps="off")
 
 
 def oracle_sample(vols, cfg, shrinks, cpu_seconds, nthreads):
@@ -384,19 +400,19 @@ def main():
             t1 = time.perf_counter()
             batch_step(p)
             cold_s.append(time.perf_counter() - t1)
-        # kernel durations, measured apart from the timed region with one
-        # stream group, direct launches and the default tiles (no concurrent
-        # groups sharing the CUs, no graphs; the same launches whatever the
-        # schedule of the timed region): one step with events around every launch picks
-        # the dominant kernel, then the same number of steps as timed with
-        # events around each of its launches give its average duration
-        lib.set_tuning(groups=1, graph_steps="off")  # library defaults otherwise
+        # kernel durations, measured apart from the timed region on its path
+        # (step kernels in one stream group without graphs, so that no
+        # concurrent group shares the CUs): one step with events around every
+        # launch picks the dominant kernel, then the same number of steps as
+        # timed with events around each of its launches give its average
+        # duration
+        lib.set_tuning(**timing_schedule(schedule))
         lib.profile_enable(n4amd.LAUNCH_KERNELS)
         batch_step(p)
         lib.synchronize()
         breakdown = {k: lib.profile_read(k) for k in n4amd.LAUNCH_KERNELS}
         dominant = max(breakdown, key=lambda k: breakdown[k][0])
-        log(f"[{prec}] one-group per-kernel device time (ms, launches): "
+        log(f"[{prec}] per-kernel device time (ms, launches): "
             + ", ".join(f"{k}={v[0]:.3f}/{v[1]}" for k, v in breakdown.items()))
         lib.profile_enable([dominant])
         for _ in range(args.steps):
@@ -448,9 +464,9 @@ def main():
         "iterations_per_level_mean": H["iterations_per_level_mean"],
         "precision": prec_text[args.precision] + "; FP64 histogram range, Wiener step, lattice update and CV sums",
         "roofline_note": "timed steps run without events; the dominant kernel's average duration comes from the "
-                         "same number of steps run again with one stream group, direct launches and the default "
-                         "tiles (independent of the timed region's schedule), with events around each of its "
-                         "launches",
+                         "same number of steps run again on the same path (teams: the resident kernel that runs a "
+                         "batch's whole loop, whose bytes are counted, and part of its reconstruction; step "
+                         "kernels: one stream group, direct launches), with events around each of its launches",
         "plan_note": "every timed step has the shapes and parameters of the step before, so it reuses the "
                      "handle's cached plan (device layout and upload image) and uploads only descriptors and "
                      "zeroed state; batched.*.ms_per_call_new_plan_median times calls that build their plan",
