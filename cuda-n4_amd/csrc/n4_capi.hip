@@ -19,8 +19,10 @@
 #include <array>
 #include <atomic>
 #include <chrono>
+#include <functional>
 #include <map>
 #include <queue>
+#include <tuple>
 #include <thread>
 #include <memory>
 #include <mutex>
@@ -585,19 +587,20 @@ struct ResPlan {
 };
 
 // This launch's team sizes into the descriptors and the slot list of the
-// image hb: the largest volumes first, each with all its slots in a row.
+// image hb: teams of several workgroups first, then the largest volumes, each
+// with all its slots in a row.
 static void put_teams(Plan* P, const ResPlan& R, unsigned char* hb) {
     const int nv = (int)P->desc.size();
-    std::vector<std::pair<double, int>> by(nv);
+    std::vector<std::tuple<bool, double, int>> by(nv);
     for (int v = 0; v < nv; ++v) {
-        by[v] = {-(double)P->desc[v].nvox_w, v};
+        by[v] = std::make_tuple(R.nmember[v] == 1, -(double)P->desc[v].nvox_w, v);
         P->desc[v].res.nmember = R.nmember[v];
     }
     std::sort(by.begin(), by.end());
     int32_t* sl = (int32_t*)(hb + P->off_slots);
     P->n_slots = 0;
     for (const auto& b : by)
-        for (int k = 0; k < R.nmember[b.second]; ++k) sl[P->n_slots++] = b.second;
+        for (int k = 0; k < R.nmember[std::get<2>(b)]; ++k) sl[P->n_slots++] = std::get<2>(b);
 }
 
 // Builds the plan and fills h->stage with the upload region.  Pointers in
@@ -1354,6 +1357,34 @@ static bool thin_grid(const VolIn& in, int nv, bool mfma) {
     return units > 8192 && W[2] < 4;
 }
 
+// Time that the resident kernel takes for volumes of tiles[v] tiles in
+// chunk[v] chunks, in tiles of one iteration: workgroups take the volumes in
+// the order of put_teams, and an iteration costs what kResFixedTiles tiles
+// do besides its own.
+static const double kResFixedTiles = 400.0;
+static double resident_span(const std::vector<double>& tiles, const std::vector<int>& chunk, int cus) {
+    std::vector<int> by(tiles.size());
+    for (size_t v = 0; v < by.size(); ++v) by[v] = (int)v;
+    std::sort(by.begin(), by.end(), [&](int a, int b) {
+        if ((chunk[a] == 1) != (chunk[b] == 1)) return chunk[a] > 1;
+        return tiles[a] > tiles[b];
+    });
+    std::priority_queue<double, std::vector<double>, std::greater<double>> free;
+    for (int k = 0; k < cus; ++k) free.push(0.0);
+    double span = 0.0;
+    for (int v : by) {
+        double end = 0.0;
+        for (int k = 0; k < chunk[v]; ++k) {
+            end = std::max(end, free.top());
+            free.pop();
+        }
+        end += kResFixedTiles + tiles[v] / chunk[v];
+        span = std::max(span, end);
+        for (int k = 0; k < chunk[v]; ++k) free.push(end);
+    }
+    return span;
+}
+
 // Resident path: chunks per volume, or false where a volume is not covered:
 // the matrix operands hold 16 control points along y and z, a volume's
 // factor tables, lattice increment and one batch of units share a compute
@@ -1364,9 +1395,9 @@ static bool thin_grid(const VolIn& in, int nv, bool mfma) {
 // when the batch asks for more workgroups than the device has compute units.
 // The resident kernel runs wherever it covers the call.  Measured against the
 // step kernels (five launches a step), whole calls: 64 x 64 x 64
-// FP32 2.70 -> 1.83 ms, 256 x 256 x 176 at shrink 4 FP32 2.89 -> 2.12, 512 x
-// 512 x 320 at shrink 2 BF16 4.72 -> 3.44, 12 mixed volumes split BF16 5.54
-// -> 3.25, 64 volumes at shrink 4 BF16 8.06 -> 5.78.
+// FP32 2.05 -> 1.37 ms, 256 x 256 x 176 at shrink 4 FP32 2.34 -> 1.71, 512 x
+// 512 x 320 at shrink 2 BF16 5.17 -> 3.76, 12 mixed volumes split BF16 5.04
+// -> 3.06, 64 volumes at shrink 4 BF16 7.54 -> 4.92.
 #ifndef N4_EMULATE
 static bool plan_resident(const std::vector<VolIn>& in, const n4_params* p, const Schedule& sch, ResPlan* R) {
     const int nv = (int)in.size(), L = (int)p->number_of_fitting_levels;
@@ -1382,7 +1413,7 @@ static bool plan_resident(const std::vector<VolIn>& in, const n4_params* p, cons
     if (resident_limits(&R->cus, &lds_cap) != 0 || R->cus < 1) return false;
     R->nchunk.assign(nv, 1);
     R->nbatch.assign(nv, 64);
-    std::vector<double> want(nv);
+    std::vector<double> want(nv), tiles(nv);
     std::vector<int> strips(nv);
     for (int v = 0; v < nv; ++v) {
         VolDesc D;
@@ -1406,6 +1437,7 @@ static bool plan_resident(const std::vector<VolIn>& in, const n4_params* p, cons
         strips[v] = D.W[0] * strips_x;
         // about three quarters of a head volume's 16-row units hold foreground
         want[v] = 0.75 * D.W[0] * ((D.W[1] + 15) / 16) / kResUnitsPerChunk;
+        tiles[v] = (double)D.W[0] * ((D.W[1] + 15) / 16) * ((D.W[2] + 15) / 16);
     }
     // at most 1024 chunks: their partials are reduced by one workgroup
     std::vector<int> most(nv);
@@ -1433,6 +1465,37 @@ static bool plan_resident(const std::vector<VolIn>& in, const n4_params* p, cons
         ++R->nchunk[v];
         --left;
         load.push({want[v] / R->nchunk[v], v});
+    }
+    // About as many volumes as workgroups leave none for the teams of large
+    // ones, and the call lasts as long as the largest volume on its one
+    // workgroup.  Where a chunk is that much larger than the mean, teams are
+    // sized by the mean instead, and volumes of one chunk wait their turn.
+    // Steps / one workgroup each / teams by the mean, BF16, ms: 256 volumes of
+    // 96 to 320 at shrink 2 to 4 41.3 / 69.6 / 32.7, of 96 to 224 22.1 / 36.0
+    // / 17.4, of 64 to 256 at shrink 4 13.3 / 14.9 / 9.8, 128 of 96 to 320
+    // 22.2 / 20.0 / 16.7; 200 of 96 to 256 at shrink 3 16.4 / 13.6 / 14.7.
+    double sum = 0.0, most_tiles = 0.0;
+    for (int v = 0; v < nv; ++v) {
+        sum += tiles[v];
+        most_tiles = std::max(most_tiles, tiles[v] / R->nchunk[v]);
+    }
+    const double mean = sum / R->cus;
+    if (most_tiles > 1.8 * mean) {
+        double best = 0.8 * resident_span(tiles, R->nchunk, R->cus);
+        std::vector<int> n(nv);
+        for (double f : {1.15, 1.3, 1.5, 1.75, 2.0}) {
+            int in_teams = 0;
+            for (int v = 0; v < nv; ++v) {
+                n[v] = std::max(1, std::min(most[v], (int)ceil(tiles[v] / (f * mean))));
+                if (n[v] > 1) in_teams += n[v];
+            }
+            if (in_teams > R->cus) continue;
+            const double span = resident_span(tiles, n, R->cus);
+            if (span < best) {
+                best = span;
+                R->nchunk = n;
+            }
+        }
     }
     return true;
 }
@@ -1474,12 +1537,15 @@ public:
         for (int n : R->nchunk) most = std::max(most, n);
         for (int k = 1;; ++k) {
             R->nmember.clear();
-            int sum = 0;
+            int sum = 0, in_teams = 0;
             for (int n : R->nchunk) {
-                R->nmember.push_back((n + k - 1) / k);
-                sum += R->nmember.back();
+                const int m = (n + k - 1) / k;
+                R->nmember.push_back(m);
+                sum += m;
+                if (m > 1) in_teams += m;
             }
-            if (sum > room && k < most) continue;
+            // (volumes of one member wait their turn)
+            if (in_teams > room && k < most) continue;
             wgs_ = std::min(sum, room);
             break;
         }

@@ -210,3 +210,17 @@ def test_handles_side_by_side(gpu):
                                                  ((200, 176, 6), 2, "fp32"), ((600, 240, 3), 3, "bf16"), ((600, 240, 4), 3, "fp32")])
 def test_thin_grids_either_side_of_the_step_kernels(gpu, dims, nvol, precision):
     _both(gpu, [_vol(dims, 70 + k) for k in range(nvol)], levels=2, max_iter=[3, 2], fixed_iterations=True, precision=precision)
+
+
+@pytest.mark.parametrize("precision", ["fp32", "bf16"])
+def test_large_among_many_small(gpu, precision, monkeypatch):
+    """As many volumes as compute units, a few of them large: teams for the
+    large ones, the small ones in turn; with fewer workgroups as well."""
+    small = [_vol((12 + k, 14, 13 + k), 200 + k) for k in range(5)]
+    vols = (small * 50)[:250] + [_vol((90 - 4 * k, 88, 85), 210 + k) for k in range(6)]
+    kw = dict(levels=2, max_iter=[3, 2], threshold=0.001, precision=precision)
+    ref, out = _both(gpu, vols, **kw)
+    monkeypatch.setenv("N4_RESIDENT_WGS", "40")
+    for a, b in zip(out, gpu.correct_batch(vols, **kw)):
+        assert a["iterations"] == b["iterations"]
+        assert np.array_equal(a["log_bias"], b["log_bias"]) and np.array_equal(a["lattice"], b["lattice"])
