@@ -2051,7 +2051,8 @@ HD void body_eval(const VolDesc* vols, const Slab* slabs, RunParams rp, int bid,
 // division by the row length, 4 z factors and 4 row values from LDS each --
 // the kernel was bound by vector instructions: 64 volumes of 652 M voxels
 // 2010 us, 3.9 TB/s, so 1497 us, 5.2 TB/s; 512x512x320 260 -> 196 us;
-// 256x256x176, field only, 23.8 -> 21.4 us, with four rows in flight.)
+// 256x256x176, field only, 23.8 -> 21.4 us, with four rows in flight; with
+// one, as it is (kReconRows), 1700, 208 and 21.4 us.)
 struct ReconLds {
     N4_LDS float* A;
     N4_LDS float* B;
@@ -2122,8 +2123,8 @@ HD void store_run4(float* p, const F4& x) {
 // barriers.
 // Rows in flight: with more, the resident kernel's instance (128 registers)
 // spills and its idle workgroups reconstruct the slower -- 64-volume batch
-// with 4 / 2 / 1 rows 5.55 / 5.24 / 5.06 ms, 512 x 512 x 320 and the
-// reconstruction launch alone unchanged from 2 to 1.
+// with 4 / 2 / 1 rows 5.55 / 5.24 / 5.06 ms.  The launch of its own loses: 64
+// volumes 1497 us with 4 rows, 1700 with 1, 512 x 512 x 320 196 and 208.
 constexpr int kReconRows = 1;
 struct ReconThread {
     int cols, nr, r0, q0;
